@@ -1,0 +1,656 @@
+// Device LSD radix sort for MI355X (gfx950): 8-bit digits over the unsigned
+// image of 4- and 8-byte arithmetic keys, alone or with a 4- or 8-byte
+// payload word per key.
+//
+// A pass is two or three launches.  k_radix_count counts the digit in every
+// segment (the consecutive tiles of one block), k_radix_offsets turns the
+// counts into each segment's first output positions, and k_radix_scatter
+// ranks a tile's keys in LDS and writes them out as one contiguous run per
+// digit, stably; up to kRadixDirect segments it adds up the counts by itself.
+// The first count also folds the AND and OR of all keys: digits where the two
+// agree are the same in every key, and their passes end at once.  All of that
+// is decided on the device, so a sort is a fixed sequence of launches and one
+// wait.  Up to kRadixSmall keys are sorted by one block in LDS.
+//
+// Reading the keys twice a pass costs less than learning the positions in one
+// sweep: a decoupled look-back over tiles took 0.42 ms of a 1.0 ms pass over
+// 2^28 32-bit keys (its 256 status words per 8192-key tile are walked across
+// the tiles in flight), the count takes 0.2 ms.
+//
+// Floating-point keys sort as operator< orders them: -0.0 and +0.0 compare
+// equal and keep their input order; NaNs go below -inf (sign bit set) or
+// above +inf.
+#ifndef KKMX_RADIXSORT_HPP
+#define KKMX_RADIXSORT_HPP
+
+#include <Kokkos_Core.hpp>
+
+#include <mutex>
+
+namespace Kokkos {
+namespace Impl {
+
+template <class T>
+struct RadixKey {
+  using U = std::conditional_t<sizeof(T) == 4, uint32_t, uint64_t>;
+  static constexpr U top      = U(1) << (8 * sizeof(T) - 1);
+  static constexpr int passes = int(sizeof(T));
+  KOKKOS_FORCEINLINE_FUNCTION static U encode(U u) {
+    if constexpr (std::is_floating_point<T>::value) return (u & top) ? ~u : (u | top);
+    else if constexpr (std::is_signed<T>::value) return u ^ top;
+    else return u;
+  }
+  KOKKOS_FORCEINLINE_FUNCTION static U decode_if(U u, bool yes) { return yes ? decode(u) : u; }
+  KOKKOS_FORCEINLINE_FUNCTION static U decode(U u) {
+    if constexpr (std::is_floating_point<T>::value) return (u & top) ? (u ^ top) : ~u;
+    else if constexpr (std::is_signed<T>::value) return u ^ top;
+    else return u;
+  }
+  // -0.0 (encoded ~top) takes the digits of +0.0 (encoded top), so the two
+  // compare equal and keep their input order; the key itself keeps its bits.
+  KOKKOS_FORCEINLINE_FUNCTION static U canon(U u) {
+    if constexpr (std::is_floating_point<T>::value) return u == U(~top) ? top : u;
+    else return u;
+  }
+  KOKKOS_FORCEINLINE_FUNCTION static unsigned digit(U u, int shift) { return unsigned(canon(u) >> shift) & 255u; }
+};
+
+// No payload: keys alone are sorted.
+struct NoPayload {};
+
+// AND and OR of the canonical keys of a sort.  Two of them alternate between
+// calls: the first count of a call folds into its own and clears the other.
+struct RadixSummary {
+  unsigned long long all, any;
+};
+struct RadixControl {
+  RadixSummary summary[2];
+  uint32_t totals[256];
+};
+
+// What a pass does, from the digits that vary.  Passes run on alternate
+// buffers and the result belongs in the caller's, so their number is even: an
+// odd count takes in one digit that need not move, and a permutation of keys
+// that are in order already (Iota) is written by two.
+struct RadixPlan {
+  bool run, from_second, first, last;
+};
+template <class T, bool Iota>
+__device__ __forceinline__ RadixPlan radix_plan(const RadixSummary& s, int p) {
+  constexpr int P              = RadixKey<T>::passes;
+  const unsigned long long vary = s.all ^ s.any;
+  unsigned runs                = 0;
+#pragma unroll
+  for (int q = 0; q < P; ++q) runs |= ((vary >> (8 * q)) & 255u) ? 1u << q : 0u;
+  const int want = (Iota && runs == 0) ? 2 : (__builtin_popcount(runs) + 1) & ~1;
+#pragma unroll
+  for (int q = 0; q < P; ++q)
+    if (__builtin_popcount(runs) < want) runs |= 1u << q;
+  const unsigned below = runs & ((1u << p) - 1);
+  return {((runs >> p) & 1u) != 0, (__builtin_popcount(below) & 1) != 0, below == 0, (runs >> p) == 1u};
+}
+
+// Counts of one digit per segment, counts[segment * 256 + d].  It reads at
+// the rate of a copy's read half as long as the LDS atomics keep up, one per
+// key: a bin has 16 counters, adjacent in LDS, one for every 16th lane, so
+// lanes of different groups never meet in a bank, and keys that share a digit
+// (the exponents of floating-point keys, small ranges) only within a group.
+constexpr int kRadixCountLanes = 512;
+template <class T, bool Iota>
+__global__ __launch_bounds__(kRadixCountLanes) void k_radix_count(const int p, const int64_t n, const int64_t segment,
+                                                                  const typename RadixKey<T>::U* k0,
+                                                                  const typename RadixKey<T>::U* k1, RadixControl* ctl,
+                                                                  const int turn, const bool fold, uint32_t* counts) {
+  using R             = RadixKey<T>;
+  using U             = typename R::U;
+  constexpr int C     = 16;
+  constexpr int Items = 64 / sizeof(U);
+  __shared__ uint32_t h[256 * C];
+  __shared__ unsigned long long s_all, s_any;
+  const int t = threadIdx.x, l = t & 63;
+  RadixPlan plan{true, false, true, false};
+  if (!fold) plan = radix_plan<T, Iota>(ctl->summary[turn], p);
+  if (!plan.run) return;
+  const U* in = plan.from_second ? k1 : k0;
+  for (int k = t; k < 256 * C; k += kRadixCountLanes) h[k] = 0;
+  if (t == 0) s_all = ~0ull, s_any = 0ull;
+  __syncthreads();
+  const int c         = l & (C - 1);
+  const int shift     = 8 * p;
+  U all = ~U(0), any = U(0);
+  const int64_t first = int64_t(blockIdx.x) * segment;
+  const int64_t last  = first + segment < n ? first + segment : n;
+  constexpr int Step  = kRadixCountLanes * Items;
+  for (int64_t b = first; b < last; b += Step) {
+    const U* from  = in + b;
+    const int left = last - b < Step ? int(last - b) : Step;
+    U u[Items];
+    if (left == Step) {
+#pragma unroll
+      for (int r = 0; r < Items; ++r) u[r] = from[r * kRadixCountLanes + t];
+    } else {
+#pragma unroll
+      for (int r = 0; r < Items; ++r) u[r] = r * kRadixCountLanes + t < left ? from[r * kRadixCountLanes + t] : U(0);
+    }
+#pragma unroll
+    for (int r = 0; r < Items; ++r) {
+      if (left == Step || r * kRadixCountLanes + t < left) {
+        const U k = R::canon(plan.first ? R::encode(u[r]) : u[r]);
+        atomicAdd(&h[(unsigned(k >> shift) & 255u) * C + c], 1u);
+        if (fold) all &= k, any |= k;
+      }
+    }
+  }
+  if (fold) {
+    atomicAnd(&s_all, (unsigned long long)all);
+    atomicOr(&s_any, (unsigned long long)any);
+  }
+  __syncthreads();
+  if (t < 256) {
+    uint32_t s = 0;
+#pragma unroll
+    for (int q = 0; q < C; ++q) s += h[t * C + ((q + l) & (C - 1))];
+    counts[int64_t(blockIdx.x) * 256 + t] = s;
+  }
+  if (fold && t == 0) {
+    atomicAnd(&ctl->summary[turn].all, s_all);
+    atomicOr(&ctl->summary[turn].any, s_any);
+    if (blockIdx.x == 0) ctl->summary[turn ^ 1] = {~0ull, 0ull};
+  }
+}
+
+// counts[segment * 256 + d] becomes the number of keys with digit d in the
+// segments before; totals[d] their number in all.  One wavefront takes 4
+// digits (16 bytes a segment and lane row) through the segments, 64 of them
+// per round.
+constexpr int kRadixOffsetLanes = 1024;
+template <class T, bool Iota>
+__global__ __launch_bounds__(kRadixOffsetLanes) void k_radix_offsets(const int p, RadixControl* ctl, const int turn,
+                                                                     uint32_t* counts, const int segments) {
+  if (!radix_plan<T, Iota>(ctl->summary[turn], p).run) return;
+  __shared__ uint32_t s_sum[16][4];
+  const int t = threadIdx.x, w = t >> 6, l = t & 63;
+  uint4* col      = reinterpret_cast<uint4*>(counts) + blockIdx.x;  // 4 digits of segment 0
+  const auto plus = [](uint32_t& a, const uint32_t& x) { a += x; };
+  uint4 carry{0, 0, 0, 0};
+  for (int b = 0; b < segments; b += kRadixOffsetLanes) {
+    const int i = b + t;
+    const uint4 x = i < segments ? col[int64_t(i) * 64] : uint4{0, 0, 0, 0};
+    uint4 inc;
+    inc.x = wave::inclusive_scan(x.x, 0u, plus);
+    inc.y = wave::inclusive_scan(x.y, 0u, plus);
+    inc.z = wave::inclusive_scan(x.z, 0u, plus);
+    inc.w = wave::inclusive_scan(x.w, 0u, plus);
+    if (l == 63) s_sum[w][0] = inc.x, s_sum[w][1] = inc.y, s_sum[w][2] = inc.z, s_sum[w][3] = inc.w;
+    __syncthreads();
+    uint4 before = carry;
+    for (int q = 0; q < 16; ++q) {
+      if (q < w) before.x += s_sum[q][0], before.y += s_sum[q][1], before.z += s_sum[q][2], before.w += s_sum[q][3];
+      carry.x += s_sum[q][0], carry.y += s_sum[q][1], carry.z += s_sum[q][2], carry.w += s_sum[q][3];
+    }
+    if (i < segments)
+      col[int64_t(i) * 64] = uint4{before.x + inc.x - x.x, before.y + inc.y - x.y, before.z + inc.z - x.z,
+                                   before.w + inc.w - x.w};
+    __syncthreads();
+  }
+  if (t == 0) reinterpret_cast<uint4*>(ctl->totals)[blockIdx.x] = carry;
+}
+
+// Rank of every key among its wavefront's keys of the same digit, in order of
+// position.  Eight ballots per 64 keys give each lane the lanes that share
+// its digit; the lowest of them adds their number to the wavefront's LDS
+// counter and every lane reads the counter back.  A wavefront's LDS
+// operations execute in order, so the rounds' adds and reads are all in
+// flight together and no round waits for the one before it.
+template <class R, int Items>
+__device__ __forceinline__ void radix_rank(const typename R::U (&u)[Items], uint32_t (&rank)[Items], int shift,
+                                           uint32_t* cnt, int rounds = Items) {
+  uint32_t seen[Items];
+#pragma unroll
+  for (int r = 0; r < Items; ++r) {
+    if (r >= rounds) break;
+    const unsigned d = R::digit(u[r], shift);
+    uint32_t lo = ~0u, hi = ~0u;
+#pragma unroll
+    for (int b = 0; b < 8; ++b) {
+      int32_t xb = __builtin_amdgcn_sbfe(int32_t(d), b, 1);  // 0 or all ones
+      asm("" : "+v"(xb));  // one extract serves the compare and the select
+      const uint64_t m = __builtin_amdgcn_ballot_w64(xb != 0);
+      // lo & ~(m ^ xb): lanes whose bit b is this lane's
+      lo = __builtin_amdgcn_bitop3_b32(lo, uint32_t(m), uint32_t(xb), 0x90);
+      hi = __builtin_amdgcn_bitop3_b32(hi, uint32_t(m >> 32), uint32_t(xb), 0x90);
+    }
+    const uint32_t below = __builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, 0u));
+    const uint32_t total = uint32_t(__popc(lo)) + uint32_t(__popc(hi));
+    if (below == 0) __hip_atomic_fetch_add(&cnt[d], total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    seen[r] = __hip_atomic_load(&cnt[d], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    rank[r] = below - total;
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+  }
+#pragma unroll
+  for (int r = 0; r < Items; ++r)
+    if (r < rounds) rank[r] += seen[r];
+}
+
+// Exclusive prefix over the 256 threads of wavefronts 0-3 (other wavefronts
+// only take part in the barrier).
+template <int NW>
+__device__ __forceinline__ uint32_t radix_prefix256(uint32_t x, uint32_t* s_wave) {
+  const auto plus    = [](uint32_t& a, const uint32_t& y) { a += y; };
+  const int w        = threadIdx.x >> 6;
+  const uint32_t inc = wave::inclusive_scan(x, 0u, plus);
+  if (w < 4 && wave::lane() == 63) s_wave[w] = inc;
+  __syncthreads();
+  uint32_t before = 0;
+#pragma unroll
+  for (int q = 0; q < 3; ++q) before += (q < w) ? s_wave[q] : 0u;
+  return before + inc - x;
+}
+
+// Up to this many segments the scatter adds up the counts before its own by
+// itself, which is shorter than another launch.
+constexpr int kRadixDirect = 48;
+
+// One digit, one segment per block, tile after tile of Lanes x Items keys;
+// wavefront w holds a run of 64 * Items of them.  Thread d < 256 carries digit
+// d's next output position from tile to tile, and the next tile's keys are
+// loaded before this one is written out.
+template <class T, class PT, bool Iota, int Lanes, int Items>
+__global__ __launch_bounds__(Lanes, 4) void k_radix_scatter(
+    const int p, const int64_t n, const int64_t segment, typename RadixKey<T>::U* k0, typename RadixKey<T>::U* k1,
+    PT* p0, PT* p1, const RadixControl* ctl, const int turn, const uint32_t* counts) {
+  using R              = RadixKey<T>;
+  using U              = typename R::U;
+  constexpr bool Pairs = !std::is_same<PT, NoPayload>::value;
+  constexpr int NW     = Lanes / 64;
+  constexpr int Tile   = Lanes * Items;
+  using Wide           = std::conditional_t<(Pairs && sizeof(PT) > sizeof(U)), uint64_t, U>;
+  __shared__ Wide s_tile[Tile];  // the tile's keys, then its payload, in digit order
+  __shared__ uint32_t wcnt[NW][256];
+  __shared__ uint32_t gshift[256];  // output position of tile slot j of digit d: gshift[d] + j
+  __shared__ uint32_t s_wave[4];
+  const RadixPlan plan = radix_plan<T, Iota>(ctl->summary[turn], p);
+  if (!plan.run) return;
+  const U* in     = plan.from_second ? k1 : k0;
+  U* out          = plan.from_second ? k0 : k1;
+  const PT* in_p  = plan.from_second ? p1 : p0;
+  PT* out_p       = plan.from_second ? p0 : p1;
+  U* key_tile     = reinterpret_cast<U*>(s_tile);
+  PT* pay_tile    = reinterpret_cast<PT*>(s_tile);
+  const int shift = 8 * p;
+  const int t = threadIdx.x, l = t & 63;
+  const int w = __builtin_amdgcn_readfirstlane(t >> 6);
+  U u[Items];
+  PT v[Pairs ? Items : 1];
+  // Keys of the tile at `tfirst`; past the end of the last one they are all
+  // ones, which keeps them behind every key of the tile in every pass.
+  const auto load = [&](int64_t tfirst) {
+    const int64_t wfirst = tfirst + w * (64 * Items);
+    const U* from        = in + wfirst;
+    const int left       = n - wfirst < 64 * Items ? int(n - wfirst) : 64 * Items;
+    if (left == 64 * Items) {
+#pragma unroll
+      for (int r = 0; r < Items; ++r) u[r] = from[r * 64 + l];
+    } else {
+#pragma unroll
+      for (int r = 0; r < Items; ++r) u[r] = r * 64 + l < left ? from[r * 64 + l] : R::decode_if(~U(0), plan.first);
+    }
+    if constexpr (Pairs) {
+      if (!(Iota && plan.first)) {
+        const PT* from_p = in_p + wfirst;
+#pragma unroll
+        for (int r = 0; r < Items; ++r) v[r] = r * 64 + l < left ? from_p[r * 64 + l] : PT(0);
+      }
+    }
+  };
+  const int64_t begin = int64_t(blockIdx.x) * segment;
+  const int64_t end   = begin + segment < n ? begin + segment : n;
+  load(begin);
+  for (int k = t; k < NW * 256; k += Lanes) (&wcnt[0][0])[k] = 0;
+  uint32_t next_pos = 0;  // of digit t
+  {
+    uint32_t total = 0;
+    if (t < 256) {
+      if (int(gridDim.x) <= kRadixDirect) {
+#pragma unroll 16
+        for (int q = 0; q < int(gridDim.x); ++q) {
+          const uint32_t x = counts[q * 256 + t];
+          total += x;
+          next_pos += q < int(blockIdx.x) ? x : 0u;
+        }
+      } else {
+        total    = ctl->totals[t];
+        next_pos = counts[int64_t(blockIdx.x) * 256 + t];
+      }
+    }
+    next_pos += radix_prefix256<NW>(total, s_wave);
+    __syncthreads();
+  }
+  for (int64_t tfirst = begin; tfirst < end; tfirst += Tile) {
+    const int have = end - tfirst < Tile ? int(end - tfirst) : Tile;
+    uint32_t slot[Items];
+    if constexpr (Iota) {
+      if (plan.first) {
+#pragma unroll
+        for (int r = 0; r < Items; ++r) v[r] = PT(tfirst + w * (64 * Items) + r * 64 + l);
+      }
+    }
+    if (plan.first) {
+#pragma unroll
+      for (int r = 0; r < Items; ++r) u[r] = R::encode(u[r]);
+    }
+    radix_rank<R>(u, slot, shift, wcnt[w]);
+    __syncthreads();  // the wavefronts' counts are complete
+    uint32_t count = 0;
+    if (t < 256) {
+#pragma unroll
+      for (int q = 0; q < NW; ++q) count += wcnt[q][t];
+    }
+    uint32_t at = radix_prefix256<NW>(count, s_wave);
+    if (t < 256) {
+      gshift[t] = next_pos - at;
+      next_pos += count;
+#pragma unroll 4
+      for (int q = 0; q < NW; ++q) {
+        const uint32_t c = wcnt[q][t];
+        wcnt[q][t]       = at;
+        at += c;
+      }
+    }
+    __syncthreads();  // slot bases and output shifts visible
+#pragma unroll
+    for (int r = 0; r < Items; ++r) {
+      slot[r] += wcnt[w][R::digit(u[r], shift)];
+      key_tile[slot[r]] = u[r];
+    }
+    __syncthreads();  // tile in digit order
+    const bool more = tfirst + Tile < end;
+    for (int k = t; k < NW * 256; k += Lanes) (&wcnt[0][0])[k] = 0;
+    if constexpr (!Pairs) {
+      if (more) load(tfirst + Tile);
+    }
+    if constexpr (!Pairs) {
+#pragma unroll 4
+      for (int r = 0; r < Items; ++r) {
+        const int j = r * Lanes + t;
+        if (j < have) {
+          U k                = key_tile[j];
+          const uint32_t pos = gshift[R::digit(k, shift)] + uint32_t(j);
+          if (plan.last) k = R::decode(k);
+          out[pos] = k;
+        }
+      }
+    } else {
+      uint32_t to[Items];
+#pragma unroll
+      for (int r = 0; r < Items; ++r) {
+        const int j = r * Lanes + t;
+        if (j < have) {
+          U k   = key_tile[j];
+          to[r] = gshift[R::digit(k, shift)] + uint32_t(j);
+          if (plan.last) k = R::decode(k);
+          out[to[r]] = k;
+        }
+      }
+      __syncthreads();  // the keys have left the tile
+#pragma unroll
+      for (int r = 0; r < Items; ++r) pay_tile[slot[r]] = v[r];
+      __syncthreads();
+      if (more) load(tfirst + Tile);
+#pragma unroll
+      for (int r = 0; r < Items; ++r) {
+        const int j = r * Lanes + t;
+        if (j < have) out_p[to[r]] = pay_tile[j];
+      }
+    }
+    __syncthreads();  // the tile has left LDS, the counters are clear
+  }
+}
+
+// Up to kRadixSmall keys, sorted by one block in LDS: every pass ranks the
+// keys the lanes hold, places them in digit order in LDS and takes them back
+// in that order.  Launch latency bounds it below a few thousand keys, then
+// the ranking of one CU.
+constexpr int kRadixSmallLanes = 1024;
+constexpr int kRadixSmallItems = 8;
+constexpr int kRadixSmall      = kRadixSmallLanes * kRadixSmallItems;
+
+template <class T, class PT, bool Iota>
+__global__ __launch_bounds__(kRadixSmallLanes) void k_radix_small(typename RadixKey<T>::U* keys, PT* pay, const int n) {
+  using R              = RadixKey<T>;
+  using U              = typename R::U;
+  constexpr bool Pairs = !std::is_same<PT, NoPayload>::value;
+  constexpr int NW     = kRadixSmallLanes / 64;
+  constexpr int Items  = kRadixSmallItems;
+  using Wide           = std::conditional_t<(Pairs && sizeof(PT) > sizeof(U)), uint64_t, U>;
+  __shared__ Wide s_tile[kRadixSmall];
+  __shared__ uint32_t wcnt[NW][256];
+  __shared__ uint32_t s_wave[4];
+  __shared__ U s_and, s_or;
+  U* key_tile  = reinterpret_cast<U*>(s_tile);
+  PT* pay_tile = reinterpret_cast<PT*>(s_tile);
+  const int t = threadIdx.x, w = t >> 6, l = t & 63;
+  const int rounds = (n + kRadixSmallLanes - 1) / kRadixSmallLanes;  // of 64 keys per wavefront
+  const int wfirst = w * 64 * rounds;
+  if (t == 0) {
+    s_and = ~U(0);
+    s_or  = U(0);
+  }
+  __syncthreads();
+  U u[Items], all = ~U(0), any = U(0);
+  PT v[Pairs ? Items : 1];
+  uint32_t slot[Items];
+#pragma unroll
+  for (int r = 0; r < Items; ++r) {
+    const int i = wfirst + r * 64 + l;
+    u[r]        = ~U(0);  // past the end: stays behind every key
+    if (r < rounds && i < n) {
+      u[r] = R::encode(keys[i]);
+      all &= R::canon(u[r]);
+      any |= R::canon(u[r]);
+      if constexpr (Pairs) {
+        if constexpr (Iota) v[r] = PT(i);
+        else v[r] = pay[i];
+      }
+    }
+  }
+  atomicAnd(&s_and, all);
+  atomicOr(&s_or, any);
+  __syncthreads();
+  const U varying = s_and ^ s_or;
+  for (int p = 0; p < R::passes; ++p) {
+    const int shift = 8 * p;
+    if (((varying >> shift) & U(255)) == 0) continue;  // the same digit in every key
+    for (int k = t; k < NW * 256; k += kRadixSmallLanes) (&wcnt[0][0])[k] = 0;
+    __syncthreads();
+    radix_rank<R>(u, slot, shift, wcnt[w], rounds);
+    __syncthreads();
+    uint32_t count = 0, wc[NW];
+    if (t < 256) {
+#pragma unroll
+      for (int q = 0; q < NW; ++q) {
+        wc[q] = wcnt[q][t];
+        count += wc[q];
+      }
+    }
+    uint32_t at = radix_prefix256<NW>(count, s_wave);
+    if (t < 256) {
+#pragma unroll
+      for (int q = 0; q < NW; ++q) {
+        wcnt[q][t] = at;
+        at += wc[q];
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < Items; ++r) {
+      if (r < rounds) {
+        slot[r] += wcnt[w][R::digit(u[r], shift)];
+        key_tile[slot[r]] = u[r];
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < Items; ++r)
+      if (r < rounds) u[r] = key_tile[wfirst + r * 64 + l];
+    if constexpr (Pairs) {
+      __syncthreads();
+#pragma unroll
+      for (int r = 0; r < Items; ++r)
+        if (r < rounds) pay_tile[slot[r]] = v[r];
+      __syncthreads();
+#pragma unroll
+      for (int r = 0; r < Items; ++r)
+        if (r < rounds) v[r] = pay_tile[wfirst + r * 64 + l];
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < Items; ++r) {
+    const int i = wfirst + r * 64 + l;
+    if (r < rounds && i < n) {
+      keys[i] = R::decode(u[r]);
+      if constexpr (Pairs) pay[i] = v[r];
+    }
+  }
+}
+
+// ------------------------------------------------------------------ host side
+// Device memory of the sort, kept between calls and grown on demand: a fresh
+// allocation per call costs more than the smaller sorts themselves and slows
+// the kernels right after it.  `buf` holds the second copy of keys and
+// payload and the segments' counts, `control` the fixed part.  Calls hold the
+// mutex until their passes have run, so sorts on different instances take
+// turns; Kokkos::finalize frees it.
+struct RadixWorkspace {
+  std::mutex mtx;
+  void* buf             = nullptr;
+  size_t bytes          = 0;
+  RadixControl* control = nullptr;
+  int turn              = 0;
+  bool hooked           = false;
+};
+
+inline RadixWorkspace& radix_workspace() {
+  static RadixWorkspace w;
+  return w;
+}
+
+inline void radix_workspace_release() {
+  RadixWorkspace& w = radix_workspace();
+  std::lock_guard<std::mutex> lock(w.mtx);
+  if (w.buf) KKMX_SAFE_CALL(mx_free(w.buf, nullptr));
+  if (w.control) KKMX_SAFE_CALL(mx_free(w.control, nullptr));
+  w.buf     = nullptr;
+  w.control = nullptr;
+  w.bytes   = 0;
+  w.turn    = 0;
+  w.hooked  = false;
+}
+
+template <class Unused = void>
+__global__ void k_radix_control_init(RadixControl* c) {
+  if (threadIdx.x < 2) c->summary[threadIdx.x] = {~0ull, 0ull};
+}
+
+inline size_t radix_round(size_t bytes) { return (bytes + 255) & ~size_t(255); }
+
+// Tile and resident blocks per CU of the scatter.  From kRadixLarge keys on,
+// larger tiles make longer runs per digit: int32 keys, 2^28 of them, take
+// 0.78 ms a pass with 8192-key tiles, 0.86 with 6144, 1.1 with 4096; (int64,
+// 8-byte value) pairs, 3 M of them, 281 us a sort with 6144-key tiles, 303 with
+// 4096 and 474 with 8192, which no longer fit two blocks' registers.  Below,
+// smaller tiles reach more CUs: 10^6 float64 keys take 159 us with 4096-key
+// tiles, 172 with 6144, 186 with 8192.
+template <class T, class PT, bool Large>
+struct RadixShape {
+  static constexpr int lanes  = 512;
+  static constexpr int items  = !Large ? 8 : std::is_same<PT, NoPayload>::value ? 16 : 12;
+  static constexpr int blocks = Large ? 2 : 4;
+};
+constexpr int64_t kRadixLarge = int64_t(1) << 21;
+
+// The passes of a sort that one block cannot hold.
+template <class T, class PT, bool Iota, class Shape>
+void radix_sort_passes(const MI355X& exec, typename RadixKey<T>::U* k0, int64_t n, PT* payload) {
+  using U              = typename RadixKey<T>::U;
+  constexpr bool pairs = !std::is_same<PT, NoPayload>::value;
+  constexpr int tile   = Shape::lanes * Shape::items;
+  // segments of whole tiles, as many as stay resident
+  const int cus            = MI355X::impl_cu_count() > 0 ? MI355X::impl_cu_count() : 256;
+  const int64_t ntiles     = (n + tile - 1) / tile;
+  const int64_t tpb        = (ntiles + int64_t(cus) * Shape::blocks - 1) / (int64_t(cus) * Shape::blocks);
+  int64_t segment          = tpb * tile;
+  int segments             = int((ntiles + tpb - 1) / tpb);
+  const size_t key_bytes   = radix_round(size_t(n) * sizeof(U));
+  const size_t pay_bytes   = pairs ? radix_round(size_t(n) * sizeof(PT)) : 0;
+  const size_t need        = key_bytes + pay_bytes + radix_round(size_t(segments) * 256 * sizeof(uint32_t));
+  RadixWorkspace& ws       = radix_workspace();
+  std::lock_guard<std::mutex> lock(ws.mtx);
+  if (ws.bytes < need) {
+    if (ws.buf) KKMX_SAFE_CALL(mx_free(ws.buf, nullptr));
+    ws.buf   = nullptr;
+    ws.bytes = 0;
+    KKMX_SAFE_CALL(mx_malloc(&ws.buf, need, nullptr));
+    ws.bytes = need;
+  }
+  if (!ws.control) {
+    void* c = nullptr;
+    KKMX_SAFE_CALL(mx_malloc(&c, sizeof(RadixControl), nullptr));
+    ws.control = static_cast<RadixControl*>(c);
+    mx_launch_kernel(reinterpret_cast<const void*>(&k_radix_control_init<>), 1, 64, 0, exec.stream(), ws.control);
+  }
+  if (!ws.hooked) {
+    push_finalize_hook(&radix_workspace_release);
+    ws.hooked = true;
+  }
+  RadixControl* ctl = ws.control;
+  U* k1             = static_cast<U*>(ws.buf);
+  PT* p1            = pairs ? reinterpret_cast<PT*>(static_cast<char*>(ws.buf) + key_bytes) : nullptr;
+  uint32_t* counts  = reinterpret_cast<uint32_t*>(static_cast<char*>(ws.buf) + key_bytes + pay_bytes);
+  int turn          = ws.turn;
+  ws.turn ^= 1;
+  for (int p = 0; p < RadixKey<T>::passes; ++p) {
+    bool fold = p == 0;
+    mx_launch_kernel(reinterpret_cast<const void*>(&k_radix_count<T, Iota>), unsigned(segments), kRadixCountLanes, 0,
+                     exec.stream(), p, n, segment, k0, k1, ctl, turn, fold, counts);
+    if (segments > kRadixDirect)
+      mx_launch_kernel(reinterpret_cast<const void*>(&k_radix_offsets<T, Iota>), 64, kRadixOffsetLanes, 0,
+                       exec.stream(), p, ctl, turn, counts, segments);
+    mx_launch_kernel(reinterpret_cast<const void*>(&k_radix_scatter<T, PT, Iota, Shape::lanes, Shape::items>),
+                     unsigned(segments), Shape::lanes, 0, exec.stream(), p, n, segment, k0, k1, payload, p1, ctl, turn,
+                     counts);
+  }
+  // the workspace is free for the next call once the stream has run these
+  exec.fence("Kokkos::sort: radix passes");
+}
+
+// Ascending LSD radix sort of n keys in place (device memory), on exec.
+// With a payload (n device words of PT), the sort is of (key, payload)
+// pairs and the payload is permuted with the keys, in place; with iota the
+// payload's input is ignored and it receives the sorting permutation
+// (sorted key i came from position payload[i]).
+template <class T, class PT = NoPayload, bool Iota = false>
+void radix_sort(const MI355X& exec, T* keys, int64_t n, PT* payload = nullptr) {
+  static_assert(std::is_same<PT, NoPayload>::value || sizeof(PT) == 4 || sizeof(PT) == 8,
+                "radix sort payloads are 4- or 8-byte words");
+  static_assert(!Iota || std::is_same<PT, uint32_t>::value, "a permutation payload is 32-bit");
+  if (n > int64_t(0x7fffffff)) throw_runtime_exception("Kokkos::sort: more than 2^31 - 1 keys");
+  if (n < 1 || (n < 2 && !Iota)) return;
+  using U = typename RadixKey<T>::U;
+  U* k0   = reinterpret_cast<U*>(keys);
+  if (n <= kRadixSmall) {
+    int count = int(n);
+    mx_launch_kernel(reinterpret_cast<const void*>(&k_radix_small<T, PT, Iota>), 1, kRadixSmallLanes, 0, exec.stream(),
+                     k0, payload, count);
+    exec.fence("Kokkos::sort: keys of one block");
+    return;
+  }
+  if (n >= kRadixLarge) radix_sort_passes<T, PT, Iota, RadixShape<T, PT, true>>(exec, k0, n, payload);
+  else radix_sort_passes<T, PT, Iota, RadixShape<T, PT, false>>(exec, k0, n, payload);
+}
+
+}  // namespace Impl
+}  // namespace Kokkos
+
+#endif

@@ -11,31 +11,19 @@
 // sort(exec, view), sort(view, comparator), sort(view, begin, end)).
 //
 // Kokkos::sort of a contiguous rank-1 device View of 4- or 8-byte
-// arithmetic keys is an LSD radix sort written for gfx950: 8-bit digits,
-// one histogram pass and one scatter pass per digit over 4096-key tiles of
-// 256 lanes, grouped into one segment of consecutive tiles per block (about
-// four blocks per CU).  The scatter ranks keys with equal digits inside
-// each wavefront from eight ballots, combines the wavefronts through LDS
-// into a digit-sorted copy of the tile in LDS, and writes that copy out so
-// each digit's keys leave as one contiguous run, at offsets from a
-// digit-major exclusive scan of the per-segment histograms: every pass
-// reads its keys twice and writes them once, stably.  The first histogram
-// also folds the AND and OR of all keys, and passes whose digit is the same
-// in every key (the high digits of small-range keys) are skipped.  Signed
-// and floating-point keys are mapped to unsigned order on the first pass
-// that runs and back on the last.  As in the reference's HIP path (thrust::sort, a radix
-// sort for arithmetic keys: algorithms/src/sorting/impl/
-// Kokkos_SortImpl.hpp:222-240), -0.0 and +0.0 compare equal and keep their
-// input order, and NaNs go below -inf (sign bit set) or above +inf.  Other
-// element types, comparators and host Views sort on the host with
-// std::sort (results identical to an ascending sort).
+// arithmetic keys is the LSD radix sort of RadixSort.hpp.  As in the
+// reference's HIP path (thrust::sort, a radix sort for arithmetic keys:
+// algorithms/src/sorting/impl/Kokkos_SortImpl.hpp:222-240), -0.0 and +0.0
+// compare equal and keep their input order, and NaNs go below -inf (sign bit
+// set) or above +inf.  Other element types, comparators and host Views sort
+// on the host with std::sort (results identical to an ascending sort).
 #ifndef KKMX_SORT_HPP
 #define KKMX_SORT_HPP
 
 #include <Kokkos_Core.hpp>
+#include <kkmx/RadixSort.hpp>
 
 #include <algorithm>
-#include <mutex>
 #include <vector>
 
 namespace Kokkos {
@@ -210,384 +198,8 @@ struct CopyRowsF {
 
 }  // namespace Impl
 
-// ------------------------------------------------------------------ radix sort
+// ------------------------------------------------------------------ sort helpers
 namespace Impl {
-
-template <class T>
-struct RadixKey {
-  using U = std::conditional_t<sizeof(T) == 4, uint32_t, uint64_t>;
-  static constexpr U top = U(1) << (8 * sizeof(T) - 1);
-  KOKKOS_FORCEINLINE_FUNCTION static U to(T v) {
-    U u;
-    __builtin_memcpy(&u, &v, sizeof(T));
-    if constexpr (std::is_floating_point<T>::value) return (u & top) ? ~u : (u | top);
-    else if constexpr (std::is_signed<T>::value) return u ^ top;
-    else return u;
-  }
-  // Digit of an encoded key.  -0.0 (encoded ~top) takes the digits of +0.0
-  // (encoded top), so the two compare equal and keep their input order, as
-  // under operator<; the key itself keeps its bits.
-  KOKKOS_FORCEINLINE_FUNCTION static U canon(U u) {
-    if constexpr (std::is_floating_point<T>::value) return u == U(~top) ? top : u;
-    else return u;
-  }
-  KOKKOS_FORCEINLINE_FUNCTION static unsigned digit(U u, int shift) { return unsigned(canon(u) >> shift) & 255u; }
-  KOKKOS_FORCEINLINE_FUNCTION static T from(U u) {
-    if constexpr (std::is_floating_point<T>::value) u = (u & top) ? (u ^ top) : ~u;
-    else if constexpr (std::is_signed<T>::value) u ^= top;
-    T v;
-    __builtin_memcpy(&v, &u, sizeof(T));
-    return v;
-  }
-};
-
-constexpr int kRadixLanes = 256;
-constexpr int kRadixItems = 16;
-constexpr int kRadixTile  = kRadixLanes * kRadixItems;
-
-// Each block owns a segment of `tpb` consecutive tiles of kRadixTile keys
-// (the last segment may be short).  k_radix_hist counts digit
-// R::digit(key, shift) over its segment, in one LDS histogram per wavefront,
-// and stores the counts digit-major: hist[d * nblocks + block].
-//
-// The First variant also folds the bitwise AND and OR of every (canonical)
-// key into summary[0] and summary[1]: digits where the two agree are the
-// same in every key, and their passes move nothing.
-template <class T, bool First>
-__global__ __launch_bounds__(256) void k_radix_hist(const void* in, const int64_t n, const int shift, uint32_t* hist,
-                                                    const int64_t nblocks, const int64_t tpb,
-                                                    typename RadixKey<T>::U* summary) {
-  using R = RadixKey<T>;
-  using U = typename R::U;
-  constexpr int NW = kRadixLanes / 64;
-  __shared__ uint32_t h[NW][256];
-  __shared__ U s_and, s_or;
-  const int t = threadIdx.x, w = t >> 6;
-#pragma unroll
-  for (int k = 0; k < NW; ++k) h[k][t] = 0;
-  if (First && t == 0) {
-    s_and = ~U(0);
-    s_or  = U(0);
-  }
-  U all_and = ~U(0), any_or = U(0);
-  __syncthreads();
-  const int64_t first = int64_t(blockIdx.x) * tpb * kRadixTile;
-  const int64_t last  = first + tpb * kRadixTile < n ? first + tpb * kRadixTile : n;
-  for (int64_t tb = first; tb < last; tb += kRadixTile) {
-    U u[kRadixItems];
-#pragma unroll
-    for (int r = 0; r < kRadixItems; ++r) {
-      const int64_t i = tb + int64_t(r) * kRadixLanes + t;
-      u[r]            = 0;
-      if (i < last) u[r] = First ? R::to(static_cast<const T*>(in)[i]) : static_cast<const U*>(in)[i];
-    }
-#pragma unroll
-    for (int r = 0; r < kRadixItems; ++r) {
-      if (tb + int64_t(r) * kRadixLanes + t < last) {
-        atomicAdd(&h[w][R::digit(u[r], shift)], 1u);
-        if (First) {
-          all_and &= R::canon(u[r]);
-          any_or |= R::canon(u[r]);
-        }
-      }
-    }
-  }
-  if (First) {
-    atomicAnd(&s_and, all_and);
-    atomicOr(&s_or, any_or);
-  }
-  __syncthreads();
-  uint32_t c = 0;
-#pragma unroll
-  for (int k = 0; k < NW; ++k) c += h[k][t];
-  hist[int64_t(t) * nblocks + blockIdx.x] = c;
-  if (First && t == 0) {
-    atomicAnd(&summary[0], s_and);
-    atomicOr(&summary[1], s_or);
-  }
-}
-
-// Stable placement of a segment's keys at their digit's offsets, one tile at
-// a time.  Wavefront w ranks keys [w * 1024, (w + 1) * 1024) of the tile with
-// eight ballots per 64 keys and its own LDS digit counters (no block barrier
-// per round), the block turns the per-wavefront counts into slots of a
-// digit-sorted copy of the tile in LDS, and writes that copy out so each
-// digit's keys leave as one contiguous run.  Lane t carries digit t's next
-// output position from tile to tile in a register.
-//
-// A payload word PT (4 or 8 bytes) can travel with each key through the same
-// slots: the values of a sort by key, or with Iota the key's input position,
-// generated on the first pass, so the last pass leaves the sorting
-// permutation.  NoPayload sorts keys alone.
-struct NoPayload {};
-
-template <class T, bool First, bool Last, class PT, bool Iota>
-__global__ __launch_bounds__(256) void k_radix_scatter(const void* in, void* out, const PT* in_p, PT* out_p,
-                                                       const int64_t n, const int shift, const uint32_t* offsets,
-                                                       const int64_t nblocks, const int64_t tpb) {
-  constexpr bool Pairs = !std::is_same<PT, NoPayload>::value;
-  using R = RadixKey<T>;
-  using U = typename R::U;
-  constexpr int NW   = kRadixLanes / 64;
-  constexpr int WKEY = kRadixTile / NW;  // keys per wavefront per tile
-  static_assert(WKEY == 64 * kRadixItems, "each lane ranks kRadixItems keys per tile");
-  __shared__ uint32_t gshift[256];  // output position of tile slot j of digit d: gshift[d] + j
-  __shared__ uint32_t wcnt[NW][256];
-  __shared__ uint32_t wsum[NW];
-  __shared__ U tile[kRadixTile];
-  __shared__ PT ptile[Pairs ? kRadixTile : 1];
-  const int t = threadIdx.x, w = t >> 6, l = t & 63;
-  const uint64_t lt = (uint64_t(1) << l) - 1;
-  uint32_t gnext    = offsets[int64_t(t) * nblocks + blockIdx.x];  // digit t's next output position
-  const int64_t seg = int64_t(blockIdx.x) * tpb * kRadixTile;
-  for (int64_t k = 0; k < tpb; ++k) {
-    const int64_t tfirst = seg + k * kRadixTile;
-    if (tfirst >= n) break;
-#pragma unroll
-    for (int q = 0; q < NW; ++q) wcnt[q][t] = 0;
-    __syncthreads();  // counters cleared; the previous tile is fully written out
-    const int64_t wfirst = tfirst + int64_t(w) * WKEY;
-    U u[kRadixItems];
-    PT ix[Pairs ? kRadixItems : 1];
-#pragma unroll
-    for (int r = 0; r < kRadixItems; ++r) {
-      const int64_t i = wfirst + int64_t(r) * 64 + l;
-      u[r]            = 0;
-      if (i < n) u[r] = First ? R::to(static_cast<const T*>(in)[i]) : static_cast<const U*>(in)[i];
-      if constexpr (Pairs) {
-        if constexpr (First && Iota) ix[r] = PT(i);
-        else if (i < n) ix[r] = in_p[i];
-      }
-    }
-    uint32_t rk[kRadixItems];
-#pragma unroll
-    for (int r = 0; r < kRadixItems; ++r) {
-      const bool valid = wfirst + int64_t(r) * 64 + l < n;
-      const unsigned d = R::digit(u[r], shift);
-      // lanes differing from this lane in some digit bit; the ballot mask of
-      // a bit doubles as the per-lane select between it and its complement
-      const uint64_t vm = __builtin_amdgcn_ballot_w64(valid);
-      uint32_t dlo = ~uint32_t(vm), dhi = ~uint32_t(vm >> 32);
-#pragma unroll
-      for (int b = 0; b < 8; ++b) {
-        const int32_t xb = int32_t(d << (31 - b)) >> 31;  // 0 or all ones
-        const uint64_t m = __builtin_amdgcn_ballot_w64(xb != 0);
-        dlo |= uint32_t(m) ^ uint32_t(xb);
-        dhi |= uint32_t(m >> 32) ^ uint32_t(xb);
-      }
-      const uint64_t peers = ~((uint64_t(dhi) << 32) | dlo);
-      const uint32_t below = __popcll(peers & lt);
-      const uint32_t prior = wcnt[w][d];
-      rk[r]                = prior + below;
-      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-      if (valid && below == 0) wcnt[w][d] = prior + uint32_t(__popcll(peers));
-      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    }
-    __syncthreads();  // per-wavefront counts complete
-    uint32_t total = 0;
-#pragma unroll
-    for (int q = 0; q < NW; ++q) {
-      const uint32_t c = wcnt[q][t];
-      wcnt[q][t]       = total;
-      total += c;
-    }
-    {
-      const auto plus    = [](uint32_t& a, const uint32_t& b) { a += b; };
-      const uint32_t inc = wave::inclusive_scan(total, 0u, plus);
-      if (l == 63) wsum[w] = inc;
-      __syncthreads();
-      uint32_t before = 0;
-#pragma unroll
-      for (int q = 0; q < NW; ++q) before += q < w ? wsum[q] : 0u;
-      // digit t's first slot in the tile; fold it into the per-wavefront
-      // prefixes and into the output shift, so placement and write-out
-      // read one LDS word per key each
-      const uint32_t first = before + inc - total;
-#pragma unroll
-      for (int q = 0; q < NW; ++q) wcnt[q][t] += first;
-      gshift[t] = gnext - first;
-      gnext += total;
-    }
-    __syncthreads();  // slot bases and output shifts visible
-#pragma unroll
-    for (int r = 0; r < kRadixItems; ++r) {
-      if (wfirst + int64_t(r) * 64 + l < n) {
-        const uint32_t slot = wcnt[w][R::digit(u[r], shift)] + rk[r];
-        tile[slot]          = u[r];
-        if constexpr (Pairs) ptile[slot] = ix[r];
-      }
-    }
-    __syncthreads();  // tile sorted by digit
-    const int64_t left = n - tfirst;
-    const int count    = left < kRadixTile ? int(left) : kRadixTile;
-    for (int j = t; j < count; j += kRadixLanes) {
-      const U v          = tile[j];
-      const uint32_t pos = gshift[R::digit(v, shift)] + uint32_t(j);
-      if (Last) static_cast<T*>(out)[pos] = R::from(v);
-      else static_cast<U*>(out)[pos] = v;
-      if constexpr (Pairs) out_p[pos] = ptile[j];
-    }
-    // the next tile writes tile, wcnt and gshift only after its first
-    // barrier, which every lane reaches after this write-out
-  }
-}
-
-struct ExclusiveScanU32 {
-  const uint32_t* in;
-  uint32_t* out;
-  KOKKOS_INLINE_FUNCTION void operator()(const int64_t i, uint32_t& upd, const bool final) const {
-    const uint32_t x = in[i];
-    if (final) out[i] = upd;
-    upd += x;
-  }
-};
-
-// Device workspace of the radix sort (ping-pong keys and the two digit
-// tables), kept between calls and grown on demand: a fresh allocation per
-// call costs more than the smaller sorts themselves and slows the kernels
-// right after it.  Calls hold the mutex until their passes have run, so
-// sorts on different instances take turns; Kokkos::finalize frees it.
-struct RadixWorkspace {
-  std::mutex mtx;
-  void* buf    = nullptr;
-  size_t bytes = 0;
-  bool hooked  = false;
-};
-
-inline RadixWorkspace& radix_workspace() {
-  static RadixWorkspace w;
-  return w;
-}
-
-inline void radix_workspace_release() {
-  RadixWorkspace& w = radix_workspace();
-  std::lock_guard<std::mutex> lock(w.mtx);
-  if (w.buf) KKMX_SAFE_CALL(mx_free(w.buf, nullptr));
-  w.buf    = nullptr;
-  w.bytes  = 0;
-  w.hooked = false;
-}
-
-struct IotaU32 {
-  uint32_t* p;
-  KOKKOS_INLINE_FUNCTION void operator()(const int64_t i) const { p[i] = uint32_t(i); }
-};
-
-template <class T, class PT, bool Iota>
-const void* radix_scatter_kernel(bool first, bool last) {
-  if (first) return last ? reinterpret_cast<const void*>(&k_radix_scatter<T, true, true, PT, Iota>)
-                         : reinterpret_cast<const void*>(&k_radix_scatter<T, true, false, PT, Iota>);
-  return last ? reinterpret_cast<const void*>(&k_radix_scatter<T, false, true, PT, Iota>)
-              : reinterpret_cast<const void*>(&k_radix_scatter<T, false, false, PT, Iota>);
-}
-
-// Ascending LSD radix sort of n keys in place (device memory), on exec.
-// With a payload (n device words of PT), the sort is of (key, payload)
-// pairs and the payload is permuted with the keys, in place; with iota the
-// payload's input is ignored and it receives the sorting permutation
-// (sorted key i came from position payload[i]).
-template <class T, class PT = NoPayload, bool Iota = false>
-void radix_sort(const MI355X& exec, T* keys, int64_t n, PT* payload = nullptr) {
-  static_assert(std::is_same<PT, NoPayload>::value || sizeof(PT) == 4 || sizeof(PT) == 8,
-                "radix sort payloads are 4- or 8-byte words");
-  static_assert(!Iota || std::is_same<PT, uint32_t>::value, "a permutation payload is 32-bit");
-  if (n > int64_t(0x7fffffff)) throw_runtime_exception("Kokkos::sort: more than 2^31 - 1 keys");
-  if (n < 2) {
-    if constexpr (Iota) {
-      if (n == 1) {
-        const uint32_t zero = 0;
-        KKMX_SAFE_CALL(mx_memcpy_async(payload, &zero, sizeof(zero), exec.stream()));
-        exec.fence("Kokkos::sort: one key");
-      }
-    }
-    return;
-  }
-  using U              = typename RadixKey<T>::U;
-  const int64_t ntiles = (n + kRadixTile - 1) / kRadixTile;
-  // segments of whole tiles, about four blocks per CU
-  const int cus        = MI355X::impl_cu_count() > 0 ? MI355X::impl_cu_count() : 256;
-  const int64_t want   = int64_t(cus) * 4;
-  const int64_t tpb    = (ntiles + want - 1) / want;
-  const int64_t nblk   = (ntiles + tpb - 1) / tpb;
-  const int passes     = int(sizeof(T));
-  const size_t key_bytes   = (size_t(n) * sizeof(U) + 255) & ~size_t(255);
-  const size_t table_bytes = size_t(256 * nblk) * sizeof(uint32_t);
-  constexpr bool pairs     = !std::is_same<PT, NoPayload>::value;
-  const size_t idx_bytes   = pairs ? (size_t(n) * sizeof(PT) + 255) & ~size_t(255) : 0;
-  const size_t need        = key_bytes + 2 * table_bytes + idx_bytes + 256;
-  RadixWorkspace& ws       = radix_workspace();
-  std::lock_guard<std::mutex> lock(ws.mtx);
-  if (ws.bytes < need) {
-    if (ws.buf) KKMX_SAFE_CALL(mx_free(ws.buf, nullptr));
-    ws.buf   = nullptr;
-    ws.bytes = 0;
-    KKMX_SAFE_CALL(mx_malloc(&ws.buf, need, nullptr));
-    ws.bytes = need;
-  }
-  if (!ws.hooked) {
-    push_finalize_hook(&radix_workspace_release);
-    ws.hooked = true;
-  }
-  char* base   = static_cast<char*>(ws.buf);
-  void* buf[2] = {static_cast<void*>(keys), static_cast<void*>(base)};
-  uint32_t* hp = reinterpret_cast<uint32_t*>(base + key_bytes);
-  uint32_t* op = reinterpret_cast<uint32_t*>(base + key_bytes + table_bytes);
-  PT* ibuf[2]   = {payload, pairs ? reinterpret_cast<PT*>(base + key_bytes + 2 * table_bytes) : nullptr};
-  U* summary    = reinterpret_cast<U*>(base + key_bytes + 2 * table_bytes + idx_bytes);
-  int64_t nb = nblk, tp = tpb;
-
-  // Pass 0's histogram, with the AND / OR summary of all keys; passes whose
-  // digit is the same in every key are identity permutations and are skipped.
-  const U init[2] = {~U(0), U(0)};
-  KKMX_SAFE_CALL(mx_memcpy_async(summary, init, sizeof(init), exec.stream()));
-  const void* keys_in = keys;
-  int shift0          = 0;
-  mx_launch_kernel(reinterpret_cast<const void*>(&k_radix_hist<T, true>), unsigned(nblk), kRadixLanes, 0,
-                   exec.stream(), keys_in, n, shift0, hp, nb, tp, summary);
-  U got[2] = {0, 0};
-  KKMX_SAFE_CALL(mx_memcpy_async(got, summary, sizeof(got), exec.stream()));
-  exec.fence("Kokkos::sort: key summary");
-  const U varying = got[0] ^ got[1];
-  int run[8], nrun = 0;
-  for (int p = 0; p < passes; ++p)
-    if ((varying >> (8 * p)) & U(255)) run[nrun++] = p;
-
-  if (nrun == 0) {  // every key has the same digits: the keys are sorted
-    if constexpr (Iota)
-      parallel_for("Kokkos::sort::identity_permutation", RangePolicy<MI355X, IndexType<int64_t>>(exec, 0, n),
-                   IotaU32{payload});
-    exec.fence("Kokkos::sort: nothing to move");
-    return;
-  }
-  for (int k = 0; k < nrun; ++k) {
-    const int p      = run[k];
-    const void* in   = buf[k & 1];
-    void* out        = buf[(k + 1) & 1];
-    int shift        = 8 * p;
-    const bool first = k == 0, last = k == nrun - 1;
-    if (!(first && p == 0)) {  // pass 0's histogram is already there
-      const void* kh = first ? reinterpret_cast<const void*>(&k_radix_hist<T, true>)
-                             : reinterpret_cast<const void*>(&k_radix_hist<T, false>);
-      mx_launch_kernel(kh, unsigned(nblk), kRadixLanes, 0, exec.stream(), in, n, shift, hp, nb, tp, summary);
-    }
-    parallel_scan("Kokkos::sort::radix_offsets", RangePolicy<MI355X, IndexType<int64_t>>(exec, 0, 256 * nblk),
-                  ExclusiveScanU32{hp, op});
-    const void* ks      = radix_scatter_kernel<T, PT, Iota>(first, last);
-    const uint32_t* cop = op;
-    const PT* iin       = ibuf[k & 1];
-    PT* iout            = ibuf[(k + 1) & 1];
-    mx_launch_kernel(ks, unsigned(nblk), kRadixLanes, 0, exec.stream(), in, out, iin, iout, n, shift, cop, nb, tp);
-  }
-  if (nrun & 1) {  // an odd number of passes left the result in the workspace
-    parallel_for("Kokkos::sort::copy_back", RangePolicy<MI355X, IndexType<int64_t>>(exec, 0, n),
-                 CopyElems<U>{static_cast<const U*>(buf[1]), reinterpret_cast<U*>(keys)});
-    if constexpr (pairs)
-      parallel_for("Kokkos::sort::copy_back_payload", RangePolicy<MI355X, IndexType<int64_t>>(exec, 0, n),
-                   CopyElems<PT>{ibuf[1], payload});
-  }
-  // the workspace is free for the next call once the stream has run these
-  exec.fence("Kokkos::sort: radix passes");
-}
 
 template <class V>
 constexpr bool radix_sortable() {

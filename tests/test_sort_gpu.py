@@ -108,6 +108,30 @@ def test_sort_by_key_is_stable(paths, oracle, code, n, vbytes):
     assert np.array_equal(Dv.download(vdt, n), vals[order])
 
 
+# Edges of the radix sort's forms: rounds of the one-block sort and its limit
+# (8192 keys), one tile more than a block's (4096), the last size whose
+# segments add up their counts themselves and the first that does not (48
+# tiles of 4096), several tiles per segment with a ragged last one, and both
+# sides of the switch to larger tiles (2^21 keys).
+@pytest.mark.parametrize("n", [1023, 1025, 8191, 8192, 8193, 12289, 48 * 4096, 48 * 4096 + 1, 1024 * 4096 + 5,
+                               (1 << 21) - 1, 1 << 21, 3000017])
+@pytest.mark.parametrize("code,vbytes", [(0, 0), (3, 0), (4, 4), (2, 8), (1, 8), (3, 4)])
+def test_sort_edges(paths, oracle, n, code, vbytes):
+    P = paths
+    x = keys_for(oracle, code, n, 400 + code)
+    bits = {4: np.uint32, 8: np.uint64}[x.dtype.itemsize]
+    order = np.argsort(x, kind="stable")
+    Dk = K.DeviceBuffer.from_array(x)
+    if vbytes == 0:
+        run(P, P.kkmx_sort(Dk.ptr, n, code))
+    else:
+        vdt = np.uint32 if vbytes == 4 else np.uint64
+        Dv = K.DeviceBuffer.from_array(np.arange(n, dtype=vdt))
+        run(P, P.kkmx_sort_by_key(Dk.ptr, Dv.ptr, n, code, vbytes, 0))
+        assert np.array_equal(Dv.download(vdt, n), order.astype(vdt))
+    assert np.array_equal(Dk.download(TYPES[code], n).view(bits), x[order].view(bits))
+
+
 @pytest.mark.parametrize("code", [0, 3])
 def test_sort_by_key_with_comparator(paths, oracle, code):
     """The comparator overload (Kokkos_SortByKeyPublicAPI.hpp:67-108) with a
@@ -129,8 +153,8 @@ def test_sort_by_key_with_comparator(paths, oracle, code):
 @pytest.mark.parametrize("n", [4097, 1 << 20])
 def test_small_range_keys_skip_constant_digits(paths, oracle, code, lo, hi, n):
     """Keys whose high (or all) digits are the same everywhere: those passes
-    are skipped, with an odd or even number of passes left (the odd case ends
-    with a copy back), or none at all; results equal numpy's stable sort and,
+    are skipped, with an odd or even number of passes left (the odd case takes
+    in one skipped digit), or none at all; results equal numpy's stable sort and,
     for sort_by_key, its stable argsort."""
     P = paths
     dt = TYPES[code]
