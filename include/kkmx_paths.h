@@ -182,7 +182,11 @@ int kkmx_spmv_csr(const int64_t* rowptr_dev, const int32_t* col_dev, const doubl
  *   atomics in mode 3; the workspace, teams x nbins int32, is kept between
  *   calls and released by kkmx_finalize.  Modes 2 and 3 lower lds_bins to
  *   what fits in LDS beside the replicas.  Every mode adds into bins.
- * kkmx_scatter_add_f64: bins[idx[i]] += vals[i] with FP64 atomic_add. */
+ * kkmx_scatter_add_f64: bins[idx[i]] += vals[i] with FP64 atomic_add; from
+ *   2^20 values (2^18 into at most 4096 bins) and up to 2^21 bins, values of
+ *   one bin are first added up in LDS.  That form keeps a workspace of up to
+ *   194 MiB between calls, released by kkmx_finalize; under stream capture the
+ *   atomics run directly.  Every form only adds to bins. */
 int kkmx_xorshift64_stream(uint64_t* out_dev, int64_t n, uint64_t seed);
 int kkmx_gups(int64_t* table_dev, int64_t table_size, const uint64_t* stream_dev, int64_t nupdates);
 int kkmx_zipf_keys(int32_t* keys_dev, int64_t n, double s, int32_t nbins, uint64_t seed);

@@ -75,8 +75,11 @@ struct RadixControl {
 struct RadixPlan {
   bool run, from_second, first, last;
 };
+// p < 0 is a single pass of its own, outside a sort: from the first buffers to
+// the second, keys as they are.
 template <class T, bool Iota>
 __device__ __forceinline__ RadixPlan radix_plan(const RadixSummary& s, int p) {
+  if (p < 0) return {true, false, false, false};
   constexpr int P              = RadixKey<T>::passes;
   const unsigned long long vary = s.all ^ s.any;
   unsigned runs                = 0;
@@ -97,7 +100,8 @@ __device__ __forceinline__ RadixPlan radix_plan(const RadixSummary& s, int p) {
 // (the exponents of floating-point keys, small ranges) only within a group.
 constexpr int kRadixCountLanes = 512;
 template <class T, bool Iota>
-__global__ __launch_bounds__(kRadixCountLanes) void k_radix_count(const int p, const int64_t n, const int64_t segment,
+__global__ __launch_bounds__(kRadixCountLanes) void k_radix_count(const int p, const int shift,
+                                                                  const int64_t n, const int64_t segment,
                                                                   const typename RadixKey<T>::U* k0,
                                                                   const typename RadixKey<T>::U* k1, RadixControl* ctl,
                                                                   const int turn, const bool fold, uint32_t* counts) {
@@ -115,8 +119,7 @@ __global__ __launch_bounds__(kRadixCountLanes) void k_radix_count(const int p, c
   for (int k = t; k < 256 * C; k += kRadixCountLanes) h[k] = 0;
   if (t == 0) s_all = ~0ull, s_any = 0ull;
   __syncthreads();
-  const int c         = l & (C - 1);
-  const int shift     = 8 * p;
+  const int c = l & (C - 1);
   U all = ~U(0), any = U(0);
   const int64_t first = int64_t(blockIdx.x) * segment;
   const int64_t last  = first + segment < n ? first + segment : n;
@@ -258,8 +261,8 @@ constexpr int kRadixDirect = 48;
 // loaded before this one is written out.
 template <class T, class PT, bool Iota, int Lanes, int Items>
 __global__ __launch_bounds__(Lanes, 4) void k_radix_scatter(
-    const int p, const int64_t n, const int64_t segment, typename RadixKey<T>::U* k0, typename RadixKey<T>::U* k1,
-    PT* p0, PT* p1, const RadixControl* ctl, const int turn, const uint32_t* counts) {
+    const int p, const int shift, const int64_t n, const int64_t segment, const typename RadixKey<T>::U* k0,
+    typename RadixKey<T>::U* k1, const PT* p0, PT* p1, const RadixControl* ctl, const int turn, const uint32_t* counts) {
   using R              = RadixKey<T>;
   using U              = typename R::U;
   constexpr bool Pairs = !std::is_same<PT, NoPayload>::value;
@@ -272,13 +275,13 @@ __global__ __launch_bounds__(Lanes, 4) void k_radix_scatter(
   __shared__ uint32_t s_wave[4];
   const RadixPlan plan = radix_plan<T, Iota>(ctl->summary[turn], p);
   if (!plan.run) return;
-  const U* in     = plan.from_second ? k1 : k0;
-  U* out          = plan.from_second ? k0 : k1;
-  const PT* in_p  = plan.from_second ? p1 : p0;
-  PT* out_p       = plan.from_second ? p0 : p1;
-  U* key_tile     = reinterpret_cast<U*>(s_tile);
-  PT* pay_tile    = reinterpret_cast<PT*>(s_tile);
-  const int shift = 8 * p;
+  // k0 and p0 are only written by passes that read the second buffers
+  const U* in    = plan.from_second ? k1 : k0;
+  U* out         = plan.from_second ? const_cast<U*>(k0) : k1;
+  const PT* in_p = plan.from_second ? p1 : p0;
+  PT* out_p      = plan.from_second ? const_cast<PT*>(p0) : p1;
+  U* key_tile    = reinterpret_cast<U*>(s_tile);
+  PT* pay_tile   = reinterpret_cast<PT*>(s_tile);
   const int t = threadIdx.x, l = t & 63;
   const int w = __builtin_amdgcn_readfirstlane(t >> 6);
   U u[Items];
@@ -612,13 +615,14 @@ void radix_sort_passes(const MI355X& exec, typename RadixKey<T>::U* k0, int64_t 
   ws.turn ^= 1;
   for (int p = 0; p < RadixKey<T>::passes; ++p) {
     bool fold = p == 0;
+    int shift = 8 * p;
     mx_launch_kernel(reinterpret_cast<const void*>(&k_radix_count<T, Iota>), unsigned(segments), kRadixCountLanes, 0,
-                     exec.stream(), p, n, segment, k0, k1, ctl, turn, fold, counts);
+                     exec.stream(), p, shift, n, segment, k0, k1, ctl, turn, fold, counts);
     if (segments > kRadixDirect)
       mx_launch_kernel(reinterpret_cast<const void*>(&k_radix_offsets<T, Iota>), 64, kRadixOffsetLanes, 0,
                        exec.stream(), p, ctl, turn, counts, segments);
     mx_launch_kernel(reinterpret_cast<const void*>(&k_radix_scatter<T, PT, Iota, Shape::lanes, Shape::items>),
-                     unsigned(segments), Shape::lanes, 0, exec.stream(), p, n, segment, k0, k1, payload, p1, ctl, turn,
+                     unsigned(segments), Shape::lanes, 0, exec.stream(), p, shift, n, segment, k0, k1, payload, p1, ctl, turn,
                      counts);
   }
   // the workspace is free for the next call once the stream has run these

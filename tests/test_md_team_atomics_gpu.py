@@ -10,6 +10,8 @@ Tolerances, stated per result:
   * GUPS, histogram: bit-exact (integer atomics commute);
   * FP64 scatter: per-bin relative error <= 1e-10 against compensated sums.
 """
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -269,3 +271,55 @@ def test_scatter_f64_within_1e10(paths, oracle, n, nbins):
     print(f"scatter n={n} bins={nbins} max rel err {err:.2e}")
     assert err <= 1e-10
     assert np.all(got[~nz] == 0.0)
+
+
+# Forms of the scatter: LDS bins directly (at most 4096 bins, from 2^18
+# values), runs of at least 1024 bins moved together first (from 2^20 values,
+# up to 2^21 bins, pieces of 2^24 values), plain atomics on the other side of
+# each line.
+@pytest.mark.parametrize("n,nbins,skew", [((1 << 18) - 1, 4096, False), (1 << 18, 4096, False), ((1 << 18) + 5, 1, False),
+                                          ((1 << 20) - 1, 4097, False), (1 << 20, 4097, False), (1 << 20, 1 << 21, False),
+                                          (1 << 20, (1 << 21) + 1, False), ((1 << 21) + 13, 262145, True),
+                                          ((1 << 24) + 7, 100003, False), ((1 << 25) + 1, 1 << 20, True)])
+def test_scatter_f64_forms(paths, oracle, n, nbins, skew):
+    P = paths
+    vals = oracle.fill_uniform_f64(n, 21, -1.0, 1.0)
+    idx = oracle.fill_uniform_i32(n, 22, 0, nbins - 1)
+    if skew:  # most values in few bins: runs of several parts
+        idx = ((idx / nbins) ** 4 * nbins).astype(np.int32)
+    if nbins > 8:
+        idx[idx == nbins // 2] = 3  # one bin stays untouched
+    start = np.where(np.arange(nbins) % 3 == 0, -0.0, 0.5)
+    V, I, B = dev(vals), dev(idx), dev(start)
+    run(P, P.kkmx_scatter_add_f64(V.ptr, I.ptr, n, B.ptr, nbins))
+    got = B.download(np.float64, nbins)
+    ref, absb = oracle.scatter_f64(vals, idx, nbins)
+    count = np.bincount(idx, minlength=nbins)
+    # m + 1 terms in any order are within m roundings of the sum of magnitudes
+    bound = (count + 1) * 2.0**-53 * (absb + np.abs(start)) * 1.01 + np.spacing(np.abs(ref))
+    assert np.all(np.abs(got - (ref + start)) <= 2 * bound)
+    untouched = count == 0
+    assert np.array_equal(got[untouched].view(np.uint64), start[untouched].view(np.uint64))
+
+
+def test_scatter_f64_captured(paths, oracle):
+    """Captured into a graph and replayed with eager calls between: every
+    replay adds the same values again."""
+    P, rt = paths, K.load("kkmx_rt")
+    n, nbins = 1 << 20, 5000
+    vals = np.floor(oracle.fill_uniform_f64(n, 23, 0.0, 16.0))  # whole: sums are exact
+    idx = oracle.fill_uniform_i32(n, 24, 0, nbins - 1)
+    V, I, B = dev(vals), dev(idx), dev(np.zeros(nbins))
+    s = P.kkmx_stream()
+    graph, ex = C.c_void_p(), C.c_void_p()
+    K.check(rt.mx_graph_capture_begin(C.c_void_p(s)))
+    K.check(P.kkmx_scatter_add_f64(V.ptr, I.ptr, n, B.ptr, nbins), P)
+    K.check(rt.mx_graph_capture_end(C.c_void_p(s), C.byref(graph)))
+    K.check(rt.mx_graph_instantiate(C.byref(ex), graph))
+    ref, _ = oracle.scatter_f64(vals, idx, nbins)
+    for k in range(3):
+        K.check(rt.mx_graph_launch(ex, C.c_void_p(s)))
+        run(P, P.kkmx_scatter_add_f64(V.ptr, I.ptr, n, B.ptr, nbins))
+        assert np.array_equal(B.download(np.float64, nbins), ref * (2 * k + 2))
+    K.check(rt.mx_graph_exec_destroy(ex))
+    K.check(rt.mx_graph_destroy(graph))
