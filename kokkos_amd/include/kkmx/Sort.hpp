@@ -140,6 +140,195 @@ struct BinShiftF {
   KOKKOS_INLINE_FUNCTION void operator()(const int i) const { order(i) += begin; }
 };
 
+// ---- BinOp1D order by quantised keys
+// A key's bin is the whole part of x = mul * (key - min), and x never
+// decreases as the key grows, so floor(x * 2^frac) orders keys as they are,
+// up to keys that share a cell of 1 / 2^frac bins, and its upper bits are the
+// bin.  Four 8-bit passes over such 32-bit codes replace the eight of the
+// float64 keys; BinRunsF then finds runs of one code whose keys are not in
+// order and BinRunSortF orders them by the keys.
+//
+// flags: [0] number of runs listed, [1] whether some key falls in no bin, [2]
+// whether a run is too long; the last two send the call to the sort of the
+// keys.
+constexpr int kBinRunMax = 64;
+template <class Keys>
+struct BinQuantiseF {
+  Keys keys;
+  double mul, min, scale, bins;
+  uint32_t* code;
+  uint32_t* flags;
+  int begin;
+  KOKKOS_INLINE_FUNCTION void operator()(const int i) const {
+    const double x = mul * (static_cast<double>(keys(begin + i)) - min);
+    const bool in  = x >= 0.0 && x < bins;  // false for NaN
+    if (!in) flags[1] = 1;
+    code[i] = in ? static_cast<uint32_t>(x * scale) : 0u;
+  }
+};
+template <class Keys>
+struct BinRunsF {
+  Keys keys;
+  const uint32_t* code;  // sorted
+  const uint32_t* order;
+  uint32_t* flags;
+  uint32_t* runs;
+  int begin, n;
+  KOKKOS_INLINE_FUNCTION bool descends(int i) const {
+    return keys(begin + int(order[i])) < keys(begin + int(order[i - 1]));
+  }
+  KOKKOS_INLINE_FUNCTION void operator()(const int i) const {
+    if (i == 0 || code[i] != code[i - 1] || !descends(i)) return;
+    int first = i - 1;  // the run's first descent lists it
+    while (first > 0 && code[first - 1] == code[i]) {
+      if (i - first >= kBinRunMax) {
+        flags[2] = 1;
+        return;
+      }
+      if (descends(first)) return;
+      --first;
+    }
+    runs[atomic_fetch_add(&flags[0], 1u)] = uint32_t(first);
+  }
+};
+template <class Keys>
+struct BinRunSortF {
+  Keys keys;
+  const uint32_t* code;
+  uint32_t* order;
+  uint32_t* flags;
+  const uint32_t* runs;
+  int begin, n;
+  KOKKOS_INLINE_FUNCTION void operator()(const int start) const {
+    const int listed = int(flags[0]);
+    for (int r = start; r < listed; r += kRunLanes) {
+      const int lo = int(runs[r]);
+      for (int k = lo + 1; k < n && code[k] == code[lo]; ++k) {
+        if (k - lo >= kBinRunMax) {
+          flags[2] = 1;
+          break;
+        }
+        const uint32_t cur = order[k];
+        int j              = k - 1;
+        while (j >= lo && keys(begin + int(cur)) < keys(begin + int(order[j]))) {
+          order[j + 1] = order[j];
+          --j;
+        }
+        order[j + 1] = cur;
+      }
+    }
+  }
+  static constexpr int kRunLanes = 1 << 16;
+};
+// First position of each bin: the first sorted code that is not below it.
+struct BinStartF {
+  const uint32_t* code;
+  View<int*, MI355XSpace, MemoryTraits<Unmanaged>> offsets;
+  int n, frac;
+  KOKKOS_INLINE_FUNCTION void operator()(const int b) const {
+    const uint32_t want = uint32_t(b) << frac;
+    int lo = 0, hi = n;
+    while (lo < hi) {
+      const int mid = lo + (hi - lo) / 2;
+      if (code[mid] < want) lo = mid + 1;
+      else hi = mid;
+    }
+    offsets(b) = lo;
+  }
+};
+struct BinExtentF {
+  View<const int*, MI355XSpace, MemoryTraits<Unmanaged>> offsets;
+  View<int*, MI355XSpace, MemoryTraits<Unmanaged>> count;
+  int n, bins;
+  KOKKOS_INLINE_FUNCTION void operator()(const int b) const {
+    count(b) = (b + 1 < bins ? offsets(b + 1) : n) - offsets(b);
+  }
+};
+
+// Device scratch of BinSort, kept between calls and grown on demand: held by
+// its mutex until the stream has run what uses it; freed by Kokkos::finalize.
+struct BinWorkspace {
+  std::mutex mtx;
+  void* buf    = nullptr;
+  size_t bytes = 0;
+  bool hooked  = false;
+  void* space(size_t need);
+};
+inline BinWorkspace& bin_workspace() {
+  static BinWorkspace w;
+  return w;
+}
+inline void bin_workspace_release() {
+  BinWorkspace& w = bin_workspace();
+  std::lock_guard<std::mutex> lock(w.mtx);
+  if (w.buf) KKMX_SAFE_CALL(mx_free(w.buf, nullptr));
+  w.buf    = nullptr;
+  w.bytes  = 0;
+  w.hooked = false;
+}
+inline void* BinWorkspace::space(size_t need) {
+  if (bytes < need) {
+    if (buf) KKMX_SAFE_CALL(mx_free(buf, nullptr));
+    buf   = nullptr;
+    bytes = 0;
+    KKMX_SAFE_CALL(mx_malloc(&buf, need, nullptr));
+    bytes = need;
+  }
+  if (!hooked) {
+    push_finalize_hook(&bin_workspace_release);
+    hooked = true;
+  }
+  return buf;
+}
+
+// The permutation of "by bin, then by key, equal keys in index order", bin
+// counts and offsets, for len > 0.  False, with nothing defined, when some key
+// falls in no bin.  Where more than kBinRunMax keys that are not in order
+// share a code (keys crowded into a few cells), the keys themselves are
+// sorted, which a BinOp1D never decreasing in the key makes the same order.
+template <class Keys, class Op>
+bool bin_order_by_code(const MI355X& exec, const Keys& keys, const Op& op, int begin, int len, int bins, int* order,
+                       int* count, int* offsets) {
+  using T = typename Keys::non_const_value_type;
+  if (!(op.mul_ > 0.0) || bins < 1) return false;  // also a range that is no number
+  int frac = 31;
+  while (frac > 0 && (uint64_t(bins) << frac) > (uint64_t(1) << 32)) --frac;
+  BinWorkspace& ws = bin_workspace();
+  std::lock_guard<std::mutex> lock(ws.mtx);
+  const size_t code_bytes = radix_round(size_t(len) * 4);
+  char* base              = static_cast<char*>(ws.space(2 * code_bytes + 256));
+  uint32_t* code          = reinterpret_cast<uint32_t*>(base);
+  uint32_t* runs          = reinterpret_cast<uint32_t*>(base + code_bytes);
+  uint32_t* flags         = reinterpret_cast<uint32_t*>(base + 2 * code_bytes);
+  uint32_t* perm          = reinterpret_cast<uint32_t*>(order);
+  clear_words_async(flags, 16, exec.stream());
+  parallel_for("Kokkos::Sort::BinQuantise", RangePolicy<MI355X>(exec, 0, len),
+               BinQuantiseF<Keys>{keys, op.mul_, op.min_, double(uint64_t(1) << frac), double(bins), code, flags, begin});
+  radix_sort<uint32_t, uint32_t, true>(exec, code, int64_t(len), perm);
+  parallel_for("Kokkos::Sort::BinRuns", RangePolicy<MI355X>(exec, 0, len),
+               BinRunsF<Keys>{keys, code, perm, flags, runs, begin, len});
+  const int lanes = len < BinRunSortF<Keys>::kRunLanes ? len : BinRunSortF<Keys>::kRunLanes;
+  parallel_for("Kokkos::Sort::BinRunSort", RangePolicy<MI355X>(exec, 0, lanes),
+               BinRunSortF<Keys>{keys, code, perm, flags, runs, begin, len});
+  using U  = View<int*, MI355XSpace, MemoryTraits<Unmanaged>>;
+  using CU = View<const int*, MI355XSpace, MemoryTraits<Unmanaged>>;
+  parallel_for("Kokkos::Sort::BinStart", RangePolicy<MI355X>(exec, 0, bins),
+               BinStartF{code, U(offsets, size_t(bins)), len, frac});
+  parallel_for("Kokkos::Sort::BinExtent", RangePolicy<MI355X>(exec, 0, bins),
+               BinExtentF{CU(offsets, size_t(bins)), U(count, size_t(bins)), len, bins});
+  uint32_t got[4] = {0, 0, 0, 0};
+  KKMX_SAFE_CALL(mx_memcpy_async(got, flags, sizeof(got), exec.stream()));
+  exec.fence("Kokkos::BinSort: keys in order");
+  if (got[1]) return false;
+  if (got[2]) {
+    View<T*, MI355XSpace> copy(view_alloc(WithoutInitializing, std::string("Kokkos::BinSort::key_copy")), size_t(len));
+    parallel_for("Kokkos::Sort::BinKeyCopy", RangePolicy<MI355X>(exec, 0, len),
+                 BinKeyCopyF<View<T*, MI355XSpace>, Keys>{copy, keys, begin});
+    radix_sort<T, uint32_t, true>(exec, copy.data(), int64_t(len), perm);
+  }
+  return true;
+}
+
 // Insertion sort of one bin's indices by one thread, as the reference does on
 // devices (quadratic in the bin size: meant for the small bins BinSort is
 // used with); equal keys keep index order, so the result does not depend on
@@ -259,7 +448,6 @@ class BinSort {
     if (range_begin > range_end) Kokkos::abort("BinSort: range_begin > range_end");
     sort_order  = offset_type("Kokkos::BinSort::sort_order", size_t(range_end - range_begin));
     bin_count   = View<int*, MI355XSpace>("Kokkos::BinSort::bin_count", size_t(bin_op.max_bins()));
-    bin_fill    = View<int*, MI355XSpace>("Kokkos::BinSort::bin_fill", size_t(bin_op.max_bins()));
     bin_offsets = offset_type("Kokkos::BinSort::bin_offsets", size_t(bin_op.max_bins()));
     (void)exec;
   }
@@ -278,10 +466,21 @@ class BinSort {
     using CU       = View<const int*, MI355XSpace, MemoryTraits<Unmanaged>>;
     const int len  = range_end - range_begin;
     const int bins = bin_op.max_bins();
+    U cnt(bin_count.data(), size_t(bins));
+    U off(bin_offsets.data(), size_t(bins)), order(sort_order.data(), size_t(len));
+    if constexpr (Impl::is_bin_op_1d<BinSortOp>::value && KeyViewType::rank == 1 &&
+                  Impl::radix_sortable<KeyViewType>()) {
+      if (sort_within_bins && len > 0 &&
+          Impl::bin_order_by_code(exec, keys, bin_op, range_begin, len, bins, order.data(), cnt.data(), off.data())) {
+        if (range_begin != 0)
+          parallel_for("Kokkos::Sort::BinShift", RangePolicy<MI355X>(exec, 0, len), Impl::BinShiftF{order, range_begin});
+        return;
+      }
+    }
+    if (bin_fill.extent(0) != size_t(bins)) bin_fill = View<int*, MI355XSpace>("Kokkos::BinSort::bin_fill", size_t(bins));
+    U fill(bin_fill.data(), size_t(bins));
     deep_copy(exec, bin_count, 0);
     deep_copy(exec, bin_fill, 0);
-    U cnt(bin_count.data(), size_t(bins)), fill(bin_fill.data(), size_t(bins));
-    U off(bin_offsets.data(), size_t(bins)), order(sort_order.data(), size_t(len));
     parallel_for("Kokkos::Sort::BinCount", RangePolicy<MI355X>(exec, 0, len),
                  Impl::BinCountF<const_key_view_type, BinSortOp>{keys, bin_op, cnt, range_begin});
     parallel_scan("Kokkos::Sort::BinOffset", RangePolicy<MI355X>(exec, 0, bins), Impl::BinOffsetF{CU(cnt), off});
@@ -324,10 +523,24 @@ class BinSort {
     const int len = range_end - range_begin;
     if (values_range_end - values_range_begin != len)
       Kokkos::abort("BinSort::sort: values range length != permutation vector length");
+    View<const int*, MI355XSpace, MemoryTraits<Unmanaged>> order(sort_order.data(), size_t(len));
+    using W = typename ValuesViewType::non_const_value_type;
+    if constexpr (ValuesViewType::rank == 1 && std::is_trivially_copyable<W>::value) {
+      // through the kept scratch, which is free again once the stream is done
+      using Rows               = View<W*, MI355XSpace, MemoryTraits<Unmanaged>>;
+      Impl::BinWorkspace& ws   = Impl::bin_workspace();
+      std::lock_guard<std::mutex> lock(ws.mtx);
+      Rows rows(static_cast<W*>(ws.space(size_t(len) * sizeof(W))), size_t(len));
+      parallel_for("Kokkos::Sort::CopyPermute", RangePolicy<MI355X>(exec, 0, len),
+                   Impl::PermuteRowsF<Rows, ValuesViewType>{rows, values, order, values_range_begin - range_begin});
+      parallel_for("Kokkos::Sort::Copy", RangePolicy<MI355X>(exec, 0, len),
+                   Impl::CopyRowsF<ValuesViewType, Rows>{values, rows, range_begin});
+      exec.fence("Kokkos::BinSort::sort: values in place");
+      return;
+    }
     using Tmp = View<typename ValuesViewType::non_const_data_type, typename ValuesViewType::array_layout, MI355XSpace>;
     Tmp tmp(std::string("Kokkos::SortImpl::BinSortFunctor::sorted_values"), size_t(len),
             ValuesViewType::rank > 1 ? values.extent(1) : ~size_t(0));  // ~0: no extent
-    View<const int*, MI355XSpace, MemoryTraits<Unmanaged>> order(sort_order.data(), size_t(len));
     parallel_for("Kokkos::Sort::CopyPermute", RangePolicy<MI355X>(exec, 0, len),
                  Impl::PermuteRowsF<Tmp, ValuesViewType>{tmp, values, order, values_range_begin - range_begin});
     parallel_for("Kokkos::Sort::Copy", RangePolicy<MI355X>(exec, 0, len),

@@ -2817,6 +2817,51 @@ KKMX_TEST(binsort_subrange_and_strided_values) {
   CHECK(got == want);
 }
 
+// Within-bin order, counts and offsets where the quantised keys take each of
+// their forms: spread keys, equal keys, cells of several keys out of order,
+// keys crowded into one cell, the range's ends and signed zeros.
+KKMX_TEST(binsort_quantised_forms) {
+  const int n = 20011;
+  using DV    = Kokkos::View<double*, Exec>;
+  for (int form = 0; form < 5; ++form) {
+    std::vector<double> h(n);
+    for (int i = 0; i < n; ++i) {
+      const double u = double((int64_t(i) * 2654435761ll + 12345) % 1000003) / 1000003.0;
+      const double w = u * 0x1.0p-40;
+      h[i]           = form == 0 ? u
+                       : form == 1 ? double(int(u * 50)) / 50
+                       : form == 2 ? double((i * 7919) % 5003) / 5003 + w  // 4 keys a cell
+                       : form == 3 ? 0.5 + w
+                                   : (i % 3 == 0 ? 1.0 : i % 3 == 1 ? 0.0 : -0.0);
+    }
+    DV keys("keys", n);
+    auto m = Kokkos::create_mirror_view(keys);
+    for (int i = 0; i < n; ++i) m(i) = h[i];
+    Kokkos::deep_copy(keys, m);
+    for (int nbins : {1, 17, 4096}) {
+      Kokkos::BinOp1D<DV> op(nbins, 0.0, 1.0);
+      Kokkos::BinSort<DV, Kokkos::BinOp1D<DV>> sorter(keys, 0, n, op, true);
+      sorter.create_permute_vector(Exec());
+      auto perm = Kokkos::create_mirror_view_and_copy(Kokkos::HostSpace(), sorter.get_permute_vector());
+      auto cnt  = Kokkos::create_mirror_view_and_copy(Kokkos::HostSpace(), sorter.get_bin_count());
+      auto off  = Kokkos::create_mirror_view_and_copy(Kokkos::HostSpace(), sorter.get_bin_offsets());
+      std::vector<int> order(n), want(nbins + 1, 0);
+      for (int i = 0; i < n; ++i) {
+        order[i] = i;
+        ++want[op.bin(m, i)];
+      }
+      std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return h[x] < h[y]; });
+      for (int i = 0; i < n; ++i) CHECK_EQ(perm(i), order[i]);
+      int total = 0;
+      for (int k = 0; k <= nbins; ++k) {
+        CHECK_EQ(off(k), total);
+        CHECK_EQ(cnt(k), want[k]);
+        total += want[k];
+      }
+    }
+  }
+}
+
 // =========================================================================
 // Kokkos::sort of strided keys (TestSort.hpp sorts subviews): every third
 // element of a buffer, whole and over [begin, end), on the device; the

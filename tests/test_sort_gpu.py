@@ -75,6 +75,28 @@ def test_binsort_within_bins_is_stable_argsort(paths, oracle, n, nbins):
     assert np.array_equal(Vd.download(np.int64, n), vals[ref])
 
 
+@pytest.mark.parametrize("n", [1, 8193, (1 << 21) + 3])
+@pytest.mark.parametrize("form", ["crowded", "pairs", "outside"])
+def test_binsort_within_bins_forms(paths, oracle, n, form):
+    """Keys crowded into one cell of the quantised range, keys that meet in
+    pairs there, and keys that fall in no bin (NaN): the permutation is the
+    stable order of the keys in every form (numpy puts NaN last, too)."""
+    P = paths
+    keys = oracle.fill_uniform_f64(n, 83, 0.0, 1.0)
+    if form == "crowded":
+        keys = 0.5 + keys * 1e-12
+    elif form == "pairs":
+        keys[1::2] = np.nextafter(keys[: n - n // 2][: len(keys[1::2])], -1.0)
+    else:
+        keys[n // 2] = np.nan
+    vals = np.arange(n, dtype=np.int64) * 3
+    Kd, Vd, Pd = K.DeviceBuffer.from_array(keys), K.DeviceBuffer.from_array(vals), K.DeviceBuffer(n * 4)
+    run(P, P.kkmx_binsort_f64(Kd.ptr, Vd.ptr, n, 1000, 0.0, 1.0, 1, Pd.ptr))
+    ref = np.argsort(keys, kind="stable")
+    assert np.array_equal(Pd.download(np.int32, n), ref)
+    assert np.array_equal(Vd.download(np.int64, n), vals[ref])
+
+
 def test_binsort_without_bin_sort_is_bin_monotone(paths, oracle):
     P = paths
     n, nbins = 1 << 18, 1000
