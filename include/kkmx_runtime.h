@@ -72,6 +72,10 @@ int mx_current_device(int* device);
 /* Device memory, stream ordered when a stream is given (NULL = synchronous). */
 int mx_malloc(void** ptr, size_t bytes, mx_stream_t stream);
 int mx_free(void* ptr, mx_stream_t stream);
+/* Blocks freed without a stream, after the device has run everything queued,
+ * are kept for later allocations, at most 512 MiB in all and 256 MiB each;
+ * mx_trim gives the kept ones back to the device. */
+int mx_trim(void);
 /* Pinned, device-mapped host memory. */
 int mx_host_alloc(void** ptr, size_t bytes);
 int mx_host_free(void* ptr);

@@ -83,6 +83,7 @@ inline void MI355X::impl_finalize() {
   if (!g.default_instance) return;
   (void)mx_device_sync();
   g.default_instance.reset();
+  (void)mx_trim();
 }
 inline void MI355X::print_configuration(std::ostream& os, bool verbose) const {
   const auto& p = Impl::mi355x_globals().props;
