@@ -8,9 +8,12 @@
 // ranks a tile's keys in LDS and writes them out as one contiguous run per
 // digit, stably; up to kRadixDirect segments it adds up the counts by itself.
 // The first count also folds the AND and OR of all keys: digits where the two
-// agree are the same in every key, and their passes end at once.  All of that
-// is decided on the device, so a sort is a fixed sequence of launches and one
-// wait.  Up to kRadixSmall keys are sorted by one block in LDS.
+// agree are the same in every key and need no pass, which the device decides by
+// itself.  8-byte keys are sorted by their five highest digits that vary where a
+// sample shows those to tell them apart (k_radix_sample), and neighbours that
+// share them are put right on the way back (k_radix_finish).  A sort is a fixed
+// sequence of launches and one wait, two for 8-byte keys that are not trimmed.
+// Up to kRadixSmall keys are sorted by one block in LDS.
 //
 // Reading the keys twice a pass costs less than learning the positions in one
 // sweep: a decoupled look-back over tiles took 0.42 ms of a 1.0 ms pass over
@@ -66,31 +69,64 @@ struct RadixSummary {
 struct RadixControl {
   RadixSummary summary[2];
   uint32_t totals[256];
+  uint32_t trim;  // 8-byte keys: only the kRadixTrim highest digits that vary are sorted
 };
+
+// Random 8-byte keys differ in their highest five or so digits: sorting by
+// those leaves a few neighbours that share them out of order, which
+// k_radix_finish puts right.  The digits are trimmed where at least two more
+// would be sorted and a sample of the keys shows no crowding.
+constexpr int kRadixTrim = 5;
 
 // What a pass does, from the digits that vary.  Passes run on alternate
 // buffers and the result belongs in the caller's, so their number is even: an
 // odd count takes in one digit that need not move, and a permutation of keys
-// that are in order already (Iota) is written by two.
+// that are in order already (Iota) is written by two.  Trimmed passes end in
+// the second buffers, still encoded, and k_radix_finish takes them back.
 struct RadixPlan {
   bool run, from_second, first, last;
+  int digit;
 };
-// p < 0 is a single pass of its own, outside a sort: from the first buffers to
-// the second, keys as they are.
-template <class T, bool Iota>
-__device__ __forceinline__ RadixPlan radix_plan(const RadixSummary& s, int p) {
-  if (p < 0) return {true, false, false, false};
-  constexpr int P              = RadixKey<T>::passes;
+template <class T>
+__device__ __forceinline__ unsigned radix_varying(const RadixSummary& s) {
   const unsigned long long vary = s.all ^ s.any;
-  unsigned runs                = 0;
+  unsigned digits               = 0;
 #pragma unroll
-  for (int q = 0; q < P; ++q) runs |= ((vary >> (8 * q)) & 255u) ? 1u << q : 0u;
+  for (int q = 0; q < RadixKey<T>::passes; ++q) digits |= ((vary >> (8 * q)) & 255u) ? 1u << q : 0u;
+  return digits;
+}
+// The digits that passes sort by.
+template <class T, bool Iota>
+__device__ __forceinline__ unsigned radix_digits(const RadixSummary& s, bool trim) {
+  unsigned runs = radix_varying<T>(s);
+  if (trim) {
+    while (__builtin_popcount(runs) > kRadixTrim) runs &= runs - 1;
+    return runs;
+  }
   const int want = (Iota && runs == 0) ? 2 : (__builtin_popcount(runs) + 1) & ~1;
 #pragma unroll
-  for (int q = 0; q < P; ++q)
+  for (int q = 0; q < RadixKey<T>::passes; ++q)
     if (__builtin_popcount(runs) < want) runs |= 1u << q;
-  const unsigned below = runs & ((1u << p) - 1);
-  return {((runs >> p) & 1u) != 0, (__builtin_popcount(below) & 1) != 0, below == 0, (runs >> p) == 1u};
+  return runs;
+}
+// Pass p of a sort: digit p of 4-byte keys, the p-th digit to be sorted of
+// 8-byte keys.  p < 0 is a single pass of its own, outside a sort: from the
+// first buffers to the second, keys as they are.
+template <class T, bool Iota>
+__device__ __forceinline__ RadixPlan radix_plan(const RadixControl* ctl, int turn, int p) {
+  if (p < 0) return {true, false, false, false, 0};
+  const bool trim     = sizeof(T) == 8 && ctl->trim != 0;
+  const unsigned runs = radix_digits<T, Iota>(ctl->summary[turn], trim);
+  int digit           = p;
+  if constexpr (sizeof(T) == 8) {
+    unsigned left = runs;
+    for (int q = 0; q < p; ++q) left &= left - 1;
+    if (left == 0) return {false, false, false, false, 0};
+    digit = __builtin_ctz(left);
+  }
+  const unsigned below = runs & ((1u << digit) - 1);
+  return {((runs >> digit) & 1u) != 0, (__builtin_popcount(below) & 1) != 0, below == 0,
+          !trim && (runs >> digit) == 1u, digit};
 }
 
 // Counts of one digit per segment, counts[segment * 256 + d].  It reads at
@@ -100,7 +136,7 @@ __device__ __forceinline__ RadixPlan radix_plan(const RadixSummary& s, int p) {
 // (the exponents of floating-point keys, small ranges) only within a group.
 constexpr int kRadixCountLanes = 512;
 template <class T, bool Iota>
-__global__ __launch_bounds__(kRadixCountLanes) void k_radix_count(const int p, const int shift,
+__global__ __launch_bounds__(kRadixCountLanes) void k_radix_count(const int p, const int pass_shift,
                                                                   const int64_t n, const int64_t segment,
                                                                   const typename RadixKey<T>::U* k0,
                                                                   const typename RadixKey<T>::U* k1, RadixControl* ctl,
@@ -112,9 +148,11 @@ __global__ __launch_bounds__(kRadixCountLanes) void k_radix_count(const int p, c
   __shared__ uint32_t h[256 * C];
   __shared__ unsigned long long s_all, s_any;
   const int t = threadIdx.x, l = t & 63;
-  RadixPlan plan{true, false, true, false};
-  if (!fold) plan = radix_plan<T, Iota>(ctl->summary[turn], p);
+  RadixPlan plan{true, false, true, false, 0};
+  if (!fold) plan = radix_plan<T, Iota>(ctl, turn, p);
   if (!plan.run) return;
+  if (!fold && p == 0 && plan.digit == 0) return;  // counted by the fold
+  const int shift = p < 0 ? pass_shift : 8 * plan.digit;
   const U* in = plan.from_second ? k1 : k0;
   for (int k = t; k < 256 * C; k += kRadixCountLanes) h[k] = 0;
   if (t == 0) s_all = ~0ull, s_any = 0ull;
@@ -170,7 +208,7 @@ constexpr int kRadixOffsetLanes = 1024;
 template <class T, bool Iota>
 __global__ __launch_bounds__(kRadixOffsetLanes) void k_radix_offsets(const int p, RadixControl* ctl, const int turn,
                                                                      uint32_t* counts, const int segments) {
-  if (!radix_plan<T, Iota>(ctl->summary[turn], p).run) return;
+  if (!radix_plan<T, Iota>(ctl, turn, p).run) return;
   __shared__ uint32_t s_sum[16][4];
   const int t = threadIdx.x, w = t >> 6, l = t & 63;
   uint4* col      = reinterpret_cast<uint4*>(counts) + blockIdx.x;  // 4 digits of segment 0
@@ -261,7 +299,7 @@ constexpr int kRadixDirect = 48;
 // loaded before this one is written out.
 template <class T, class PT, bool Iota, int Lanes, int Items>
 __global__ __launch_bounds__(Lanes, 4) void k_radix_scatter(
-    const int p, const int shift, const int64_t n, const int64_t segment, const typename RadixKey<T>::U* k0,
+    const int p, const int pass_shift, const int64_t n, const int64_t segment, const typename RadixKey<T>::U* k0,
     typename RadixKey<T>::U* k1, const PT* p0, PT* p1, const RadixControl* ctl, const int turn, const uint32_t* counts) {
   using R              = RadixKey<T>;
   using U              = typename R::U;
@@ -273,8 +311,9 @@ __global__ __launch_bounds__(Lanes, 4) void k_radix_scatter(
   __shared__ uint32_t wcnt[NW][256];
   __shared__ uint32_t gshift[256];  // output position of tile slot j of digit d: gshift[d] + j
   __shared__ uint32_t s_wave[4];
-  const RadixPlan plan = radix_plan<T, Iota>(ctl->summary[turn], p);
+  const RadixPlan plan = radix_plan<T, Iota>(ctl, turn, p);
   if (!plan.run) return;
+  const int shift = p < 0 ? pass_shift : 8 * plan.digit;
   // k0 and p0 are only written by passes that read the second buffers
   const U* in    = plan.from_second ? k1 : k0;
   U* out         = plan.from_second ? const_cast<U*>(k0) : k1;
@@ -411,6 +450,165 @@ __global__ __launch_bounds__(Lanes, 4) void k_radix_scatter(
   }
 }
 
+// Whether the digits of 8-byte keys are trimmed: 4096 keys, evenly spaced, go
+// into an LDS hash table by their trimmed digits, and different keys that meet
+// there are counted.  If all of n keys lie in runs of 64, which is more than
+// k_radix_finish takes, 4096^2 / 2 * 64 / n meet: 8 at n = 2^26, more below.
+constexpr int kRadixSample = 4096;
+template <class T>
+__global__ __launch_bounds__(1024) void k_radix_sample(const typename RadixKey<T>::U* in, const int64_t n,
+                                                       RadixControl* ctl, const int turn, const bool allow) {
+  using R = RadixKey<T>;
+  using U = typename R::U;
+  __shared__ unsigned long long table[2 * kRadixSample];
+  __shared__ unsigned met;
+  const int t            = threadIdx.x;
+  const unsigned digits  = radix_digits<T, false>(ctl->summary[turn], true);
+  const bool worth       = allow && __builtin_popcount(radix_varying<T>(ctl->summary[turn])) >= kRadixTrim + 2;
+  if (!worth) {
+    if (t == 0) ctl->trim = 0;
+    return;
+  }
+  const int low = 8 * __builtin_ctz(digits);
+  for (int k = t; k < 2 * kRadixSample; k += 1024) table[k] = ~0ull;
+  if (t == 0) met = 0;
+  __syncthreads();
+  const int64_t step = n / kRadixSample;
+  for (int k = t; k < kRadixSample; k += 1024) {
+    const unsigned long long key = R::canon(R::encode(in[k * step]));
+    if (key == ~0ull) continue;
+    unsigned at = unsigned(((key >> low) * 0x9E3779B97F4A7C15ull) >> 51);  // 13 bits
+    for (int probe = 0; probe < 32; ++probe, at = (at + 1) & (2 * kRadixSample - 1)) {
+      const unsigned long long was = atomicCAS(&table[at], ~0ull, key);
+      if (was == ~0ull || was == key) break;
+      if ((was >> low) == (key >> low)) {
+        atomicAdd(&met, 1u);
+        break;
+      }
+    }
+  }
+  __syncthreads();
+  if (t == 0) ctl->trim = met <= 4 ? 1 : 0;
+}
+
+// Takes keys sorted by their trimmed digits from the second buffers to the
+// caller's.  Neighbours that share those digits form a run; a key's place in
+// its run is the number of keys before it there, by value, then by position.
+// Most keys have no such neighbour, or a run already in order, which a
+// wavefront sees from its own and the neighbouring wavefronts' ballots.  A run
+// of 64 keys or more (every key of it sees that) is left as it is, and reported
+// where it is out of order (status 1): the caller's keys are then still a
+// stable order by the trimmed digits, and all digits are sorted over.  Status 2
+// reports digits left to sort where nothing was trimmed.
+constexpr int kRadixRun         = 64;
+constexpr int kRadixFinishLanes = 1024;
+constexpr int kRadixFinishTile  = 4096;
+// How far key j moves within its run.
+template <class R, class U, class Tied>
+__device__ __forceinline__ int radix_place_in_run(const U* s_key, const int j, const Tied& tied, bool& broken) {
+  const U key = R::canon(s_key[j]);
+  int lo = j, hi = j + 1;  // the run, as far as 64 keys to each side
+  while (j - lo < kRadixRun - 1 && tied(lo)) --lo;
+  while (hi - j < kRadixRun && tied(hi)) ++hi;
+  if (tied(lo) || hi - j == kRadixRun || hi - lo >= kRadixRun) {
+    for (int k = lo + 1; k < hi; ++k) broken = broken || R::canon(s_key[k]) < R::canon(s_key[k - 1]);
+    return 0;
+  }
+  int before = 0;
+  for (int k = lo; k < hi; ++k) {
+    const U x = R::canon(s_key[k]);
+    before += (x < key || (x == key && k < j)) ? 1 : 0;
+  }
+  return lo + before - j;
+}
+
+template <class T, class PT>
+__global__ __launch_bounds__(kRadixFinishLanes) void k_radix_finish(const int64_t n, typename RadixKey<T>::U* k0,
+                                                                    const typename RadixKey<T>::U* k1, PT* p0,
+                                                                    const PT* p1, const RadixControl* ctl,
+                                                                    const int turn, uint32_t* status) {
+  using R              = RadixKey<T>;
+  using U              = typename R::U;
+  constexpr bool Pairs = !std::is_same<PT, NoPayload>::value;
+  constexpr int NW     = kRadixFinishLanes / 64;
+  constexpr int Items  = kRadixFinishTile / kRadixFinishLanes;
+  const unsigned runs  = radix_digits<T, false>(ctl->summary[turn], ctl->trim != 0);
+  const int t = threadIdx.x, w = t >> 6, l = t & 63;
+  if (!ctl->trim) {
+    if (blockIdx.x == 0 && t == 0 && __builtin_popcount(runs) > kRadixTrim) *status = 2;
+    return;
+  }
+  const int low = 8 * __builtin_ctz(runs);
+  // key base + x is s_key[x + kRadixRun + 1]; [0] is one before the halo
+  __shared__ U s_key[kRadixFinishTile + 2 * kRadixRun + 1];
+  // keys tied to the one before, and descents there, 64 keys a word, with a
+  // word for each halo
+  __shared__ uint64_t s_tied[kRadixFinishTile / 64 + 2], s_down[kRadixFinishTile / 64 + 2];
+  bool broken = false;
+  for (int64_t base = int64_t(blockIdx.x) * kRadixFinishTile; base < n; base += int64_t(gridDim.x) * kRadixFinishTile) {
+    U raw[Items], halo = U(0);
+    PT v[Pairs ? Items : 1];
+#pragma unroll
+    for (int r = 0; r < Items; ++r) {
+      const int64_t i = base + r * kRadixFinishLanes + t;
+      raw[r]          = i < n ? k1[i] : U(0);
+      if constexpr (Pairs) {
+        if (i < n) v[r] = p1[i];
+      }
+    }
+    const int hj = t <= kRadixRun ? t : kRadixFinishTile + t;  // lanes 0-64 before the tile, 65-128 after it
+    if (t <= 2 * kRadixRun) {
+      const int64_t i = base - kRadixRun - 1 + hj;
+      if (i >= 0 && i < n) halo = k1[i];
+    }
+#pragma unroll
+    for (int r = 0; r < Items; ++r) s_key[1 + kRadixRun + r * kRadixFinishLanes + t] = raw[r];
+    if (t <= 2 * kRadixRun) s_key[hj] = halo;
+    __syncthreads();
+    const auto tied = [&](int j) {
+      const int64_t i = base - kRadixRun - 1 + j;
+      return i > 0 && i < n && (R::canon(s_key[j]) >> low) == (R::canon(s_key[j - 1]) >> low);
+    };
+    for (int q = w; q < kRadixFinishTile / 64 + 2; q += NW) {
+      const int j         = 1 + q * 64 + l;
+      const bool tie      = tied(j);
+      const uint64_t ties = __builtin_amdgcn_ballot_w64(tie);
+      const uint64_t down = __builtin_amdgcn_ballot_w64(tie && R::canon(s_key[j]) < R::canon(s_key[j - 1]));
+      if (l == 0) s_tied[q] = ties, s_down[q] = down;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < Items; ++r) {
+      const int64_t i = base + r * kRadixFinishLanes + t;
+      if (i >= n) break;
+      const int j   = 1 + kRadixRun + r * kRadixFinishLanes + t;
+      const int q   = w + r * NW;
+      int64_t place = i;
+      const uint64_t d1 = s_down[q + 1], d2 = s_down[q + 2];
+      if (s_down[q] | d1 | d2) {
+        // bits 0-2: this key and the two after it
+        const uint64_t t1 = s_tied[q + 1], t2 = s_tied[q + 2];
+        const unsigned tie  = unsigned((t1 >> l) | (l ? t2 << (64 - l) : 0)) & 7u;
+        const unsigned down = unsigned((d1 >> l) | (l ? d2 << (64 - l) : 0)) & 3u;
+        const bool tie_back = l ? ((t1 >> (l - 1)) & 1) != 0 : (s_tied[q] >> 63) != 0;
+        if ((tie & 3u) == 0) {
+          // no such neighbour
+        } else if (tie == 2u) {  // the first of two
+          place = i + (down >> 1);
+        } else if ((tie & 3u) == 1u && !tie_back) {  // the second of two
+          place = i - (down & 1u);
+        } else {
+          place = i + radix_place_in_run<R>(s_key, j, tied, broken);
+        }
+      }
+      k0[place] = R::decode(raw[r]);
+      if constexpr (Pairs) p0[place] = v[r];
+    }
+    __syncthreads();
+  }
+  if (broken) *status = 1;
+}
+
 // Up to kRadixSmall keys, sorted by one block in LDS: every pass ranks the
 // keys the lanes hold, places them in digit order in LDS and takes them back
 // in that order.  Launch latency bounds it below a few thousand keys, then
@@ -530,6 +728,7 @@ struct RadixWorkspace {
   void* buf             = nullptr;
   size_t bytes          = 0;
   RadixControl* control = nullptr;
+  uint32_t* status      = nullptr;  // pinned host word that k_radix_finish reports to
   int turn              = 0;
   bool hooked           = false;
 };
@@ -544,8 +743,10 @@ inline void radix_workspace_release() {
   std::lock_guard<std::mutex> lock(w.mtx);
   if (w.buf) KKMX_SAFE_CALL(mx_free(w.buf, nullptr));
   if (w.control) KKMX_SAFE_CALL(mx_free(w.control, nullptr));
+  if (w.status) KKMX_SAFE_CALL(mx_host_free(w.status));
   w.buf     = nullptr;
   w.control = nullptr;
+  w.status  = nullptr;
   w.bytes   = 0;
   w.turn    = 0;
   w.hooked  = false;
@@ -554,6 +755,7 @@ inline void radix_workspace_release() {
 template <class Unused = void>
 __global__ void k_radix_control_init(RadixControl* c) {
   if (threadIdx.x < 2) c->summary[threadIdx.x] = {~0ull, 0ull};
+  if (threadIdx.x == 2) c->trim = 0;
 }
 
 inline size_t radix_round(size_t bytes) { return (bytes + 255) & ~size_t(255); }
@@ -572,6 +774,53 @@ struct RadixShape {
   static constexpr int blocks = Large ? 2 : 4;
 };
 constexpr int64_t kRadixLarge = int64_t(1) << 21;
+
+// The launches of one sort.
+template <class T, class PT>
+struct RadixRun {
+  using U = typename RadixKey<T>::U;
+  mx_stream_t stream;
+  int64_t n, segment;
+  int segments;
+  U *k0, *k1;
+  PT *p0, *p1;
+  RadixControl* ctl;
+  int turn;
+  uint32_t* counts;
+
+  // Digit 0's counts, and the AND and OR of all keys.
+  template <bool Iota>
+  void fold() {
+    int p = 0, shift = 0;
+    bool yes = true;
+    mx_launch_kernel(reinterpret_cast<const void*>(&k_radix_count<T, Iota>), unsigned(segments), kRadixCountLanes, 0,
+                     stream, p, shift, n, segment, k0, k1, ctl, turn, yes, counts);
+  }
+  template <bool Iota, class Shape>
+  void passes(int first, int last) {
+    bool no   = false;
+    int shift = 0;
+    for (int p = first; p < last; ++p) {
+      if (p > 0 || sizeof(T) == 8)  // digit 0 of 4-byte keys is counted by the fold
+        mx_launch_kernel(reinterpret_cast<const void*>(&k_radix_count<T, Iota>), unsigned(segments), kRadixCountLanes,
+                         0, stream, p, shift, n, segment, k0, k1, ctl, turn, no, counts);
+      if (segments > kRadixDirect)
+        mx_launch_kernel(reinterpret_cast<const void*>(&k_radix_offsets<T, Iota>), 64, kRadixOffsetLanes, 0, stream, p,
+                         ctl, turn, counts, segments);
+      mx_launch_kernel(reinterpret_cast<const void*>(&k_radix_scatter<T, PT, Iota, Shape::lanes, Shape::items>),
+                       unsigned(segments), Shape::lanes, 0, stream, p, shift, n, segment, k0, k1, p0, p1, ctl, turn,
+                       counts);
+    }
+  }
+  void sample(bool allow) {
+    mx_launch_kernel(reinterpret_cast<const void*>(&k_radix_sample<T>), 1, 1024, 0, stream, k0, n, ctl, turn, allow);
+  }
+  void finish(uint32_t* status, int cus) {
+    const int64_t tiles = (n + kRadixFinishTile - 1) / kRadixFinishTile;
+    mx_launch_kernel(reinterpret_cast<const void*>(&k_radix_finish<T, PT>), unsigned(tiles < 2 * cus ? tiles : 2 * cus),
+                     kRadixFinishLanes, 0, stream, n, k0, k1, p0, p1, ctl, turn, status);
+  }
+};
 
 // The passes of a sort that one block cannot hold.
 template <class T, class PT, bool Iota, class Shape>
@@ -607,26 +856,49 @@ void radix_sort_passes(const MI355X& exec, typename RadixKey<T>::U* k0, int64_t 
     push_finalize_hook(&radix_workspace_release);
     ws.hooked = true;
   }
-  RadixControl* ctl = ws.control;
-  U* k1             = static_cast<U*>(ws.buf);
-  PT* p1            = pairs ? reinterpret_cast<PT*>(static_cast<char*>(ws.buf) + key_bytes) : nullptr;
-  uint32_t* counts  = reinterpret_cast<uint32_t*>(static_cast<char*>(ws.buf) + key_bytes + pay_bytes);
-  int turn          = ws.turn;
-  ws.turn ^= 1;
-  for (int p = 0; p < RadixKey<T>::passes; ++p) {
-    bool fold = p == 0;
-    int shift = 8 * p;
-    mx_launch_kernel(reinterpret_cast<const void*>(&k_radix_count<T, Iota>), unsigned(segments), kRadixCountLanes, 0,
-                     exec.stream(), p, shift, n, segment, k0, k1, ctl, turn, fold, counts);
-    if (segments > kRadixDirect)
-      mx_launch_kernel(reinterpret_cast<const void*>(&k_radix_offsets<T, Iota>), 64, kRadixOffsetLanes, 0,
-                       exec.stream(), p, ctl, turn, counts, segments);
-    mx_launch_kernel(reinterpret_cast<const void*>(&k_radix_scatter<T, PT, Iota, Shape::lanes, Shape::items>),
-                     unsigned(segments), Shape::lanes, 0, exec.stream(), p, shift, n, segment, k0, k1, payload, p1, ctl, turn,
-                     counts);
+  if (!ws.status) {
+    void* h = nullptr;
+    KKMX_SAFE_CALL(mx_host_alloc(&h, 64));
+    ws.status = static_cast<uint32_t*>(h);
   }
-  // the workspace is free for the next call once the stream has run these
-  exec.fence("Kokkos::sort: radix passes");
+  RadixRun<T, PT> r{exec.stream(),
+                    n,
+                    segment,
+                    segments,
+                    k0,
+                    static_cast<U*>(ws.buf),
+                    payload,
+                    pairs ? reinterpret_cast<PT*>(static_cast<char*>(ws.buf) + key_bytes) : nullptr,
+                    ws.control,
+                    ws.turn,
+                    reinterpret_cast<uint32_t*>(static_cast<char*>(ws.buf) + key_bytes + pay_bytes)};
+  ws.turn ^= 1;
+  if constexpr (sizeof(T) == 4) {
+    r.template fold<Iota>();
+    r.template passes<Iota, Shape>(0, 4);
+    // the workspace is free for the next call once the stream has run these
+    exec.fence("Kokkos::sort: radix passes");
+  } else {
+    uint32_t* status = ws.status;
+    *status          = 0;
+    r.template fold<Iota>();
+    r.sample(true);
+    r.template passes<Iota, Shape>(0, kRadixTrim);
+    r.finish(status, cus);
+    exec.fence("Kokkos::sort: radix passes");
+    if (*static_cast<volatile uint32_t*>(status) == 2) {
+      r.template passes<Iota, Shape>(kRadixTrim, 8);
+      exec.fence("Kokkos::sort: remaining radix passes");
+    } else if (*static_cast<volatile uint32_t*>(status) == 1) {
+      // the payload holds the permutation so far, also with Iota
+      r.turn = ws.turn;
+      ws.turn ^= 1;
+      r.template fold<false>();
+      r.sample(false);
+      r.template passes<false, Shape>(0, 8);
+      exec.fence("Kokkos::sort: all radix passes");
+    }
+  }
 }
 
 // Ascending LSD radix sort of n keys in place (device memory), on exec.

@@ -154,6 +154,47 @@ def test_sort_edges(paths, oracle, n, code, vbytes):
     assert np.array_equal(Dk.download(TYPES[code], n).view(bits), x[order].view(bits))
 
 
+@pytest.mark.parametrize("form", ["spread", "runs", "crowd", "one_long_run", "equal", "six_digits"])
+@pytest.mark.parametrize("n", [8193, 100003, (1 << 21) + 5])
+@pytest.mark.parametrize("code,vbytes", [(1, 0), (3, 0), (5, 8), (3, 4)])
+def test_sort_of_8_byte_keys_by_their_highest_digits(paths, oracle, n, code, vbytes, form):
+    """8-byte keys are sorted by their five highest digits that vary where
+    those tell them apart: spread keys (no digits to spare), runs of up to 40
+    keys that share them out of order, keys all crowded into few runs (seen in
+    the sample: all digits), one run of 300 among spread keys (not seen, found
+    at the end: sorted over), many equal keys, and keys of six digits."""
+    P = paths
+    r = oracle.fill_uniform_i64(n, 500 + code, -(1 << 62), 1 << 62)
+    low = oracle.fill_uniform_i64(n, 600 + code, 0, (1 << 20) - 1)
+    if form == "runs":
+        k = np.arange(n) // 40 % 997
+        r = np.where(k < 20, (r[k] & ~np.int64((1 << 20) - 1)) | low, r)[np.argsort(low, kind="stable")]
+    elif form == "crowd":
+        r = (r[np.arange(n) % 7] & ~np.int64((1 << 20) - 1)) | low
+        r[0] = -(1 << 62)
+        r[1] = (1 << 62) - 1
+    elif form == "one_long_run":
+        at = np.argsort(low, kind="stable")[:300]
+        r[at] = (r[0] & ~np.int64((1 << 20) - 1)) | low[at]
+    elif form == "equal":
+        r = r[np.arange(n) % 1009]
+    elif form == "six_digits":
+        r = r & ((1 << 48) - 1)
+    x = r.view(np.float64) if code == 3 else r.astype(TYPES[code])
+    if code == 3:
+        x = np.where(np.isnan(x), 1.5, x)
+    order = np.argsort(x, kind="stable")
+    Dk = K.DeviceBuffer.from_array(x)
+    if vbytes:
+        vdt = np.uint32 if vbytes == 4 else np.uint64
+        Dv = K.DeviceBuffer.from_array(np.arange(n, dtype=vdt))
+        run(P, P.kkmx_sort_by_key(Dk.ptr, Dv.ptr, n, code, vbytes, 0))
+        assert np.array_equal(Dv.download(vdt, n), order.astype(vdt))
+    else:
+        run(P, P.kkmx_sort(Dk.ptr, n, code))
+    assert np.array_equal(Dk.download(TYPES[code], n).view(np.uint64), x[order].view(np.uint64))
+
+
 @pytest.mark.parametrize("code", [0, 3])
 def test_sort_by_key_with_comparator(paths, oracle, code):
     """The comparator overload (Kokkos_SortByKeyPublicAPI.hpp:67-108) with a
