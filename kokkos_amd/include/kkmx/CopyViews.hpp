@@ -99,48 +99,53 @@ struct ElementCopy {
 };
 
 // ViewCopy between LayoutLeft and LayoutRight (both contiguous, rank >= 2)
-// as an LDS-tiled transpose on gfx950: each 512-lane workgroup moves a
-// 64 x 64 tile of (first index, last index) for one multi-index of the
-// middle dimensions.  It reads along the source's contiguous dimension and
-// writes along the destination's, both coalesced; the tile sits in LDS with
-// a 65-element row pitch so neither pass has bank conflicts.  Consecutive
-// workgroups take consecutive tiles of the last index, and the destination
-// is written with nontemporal stores (a copy's output is not read back by
-// the copy).  512^3 doubles: 0.452 ms; 0.522 ms with 256 lanes, 0.483 ms
-// with 1024, 0.549 ms with 256 lanes, the first index fastest and ordinary
-// stores.
+// as an LDS-tiled transpose on gfx950: each 512-lane workgroup moves a tile of
+// (first index, last index) for one multi-index of the middle dimensions, 64
+// long in the source's contiguous dimension and in the destination's 64, for
+// 8-byte words 32, which leaves room for twice the workgroups.  It reads along
+// the source's contiguous dimension and writes along the destination's, both
+// coalesced; the tile sits in LDS with an odd row pitch so neither pass has
+// bank conflicts.  Consecutive workgroups take consecutive tiles of the last
+// index, and the destination is written with nontemporal stores (a copy's
+// output is not read back by the copy).  512^3 doubles: 0.421 ms with 64 x 32
+// tiles, 0.435 with 64 x 64 (0.449 with 64-bit index arithmetic), 0.51-0.64
+// with 128 in either direction, 0.65 with the middle index fastest.
 //   LayoutLeft  offset of (i, mid, k) = i + e0 * (midL + M * k)
 //   LayoutRight offset of (i, mid, k) = (i * M + midR) * e_last + k
 // midL / midR: the middle indices flattened left-first / right-first, M
 // their product.
 struct TransposeShape {
   int64_t e0, elast, M;
-  int64_t mid[4];  // extents of the middle dimensions (1 when absent)
+  uint32_t mid[4];  // extents of the middle dimensions (1 when absent)
   int nmid;
-  int64_t tiles0, tileslast;
+  uint32_t tiles0, tileslast;  // their product with M is below 2^31
 };
+// Tile extent along the destination's contiguous dimension.
+template <class W>
+constexpr int transpose_narrow = sizeof(W) == 8 ? 32 : 64;
 template <class W, bool SrcLeft>
 __global__ __launch_bounds__(512) void k_layout_transpose(W* __restrict__ dst, const W* __restrict__ src,
                                                           const TransposeShape sh) {
-  __shared__ W tile[64][65];
-  const int64_t b  = blockIdx.x;
-  const int64_t tk = b % sh.tileslast;
-  const int64_t t0 = (b / sh.tileslast) % sh.tiles0;
-  int64_t g        = b / (sh.tiles0 * sh.tileslast);  // middle multi-index, flattened left-first
+  constexpr int N = transpose_narrow<W>;
+  __shared__ W tile[N][65];
+  const uint32_t b  = blockIdx.x;
+  const uint32_t tk = b % sh.tileslast;
+  const uint32_t t0 = (b / sh.tileslast) % sh.tiles0;
+  uint32_t g        = b / (sh.tiles0 * sh.tileslast);  // middle multi-index, flattened left-first
   int64_t midL = g, midR = 0;
   {
-    int64_t idx[4] = {0, 0, 0, 0};
+    uint32_t idx[4] = {0, 0, 0, 0};
     for (int d = 0; d < sh.nmid; ++d) {
       idx[d] = g % sh.mid[d];
       g /= sh.mid[d];
     }
     for (int d = 0; d < sh.nmid; ++d) midR = midR * sh.mid[d] + idx[d];
   }
-  const int lane = threadIdx.x & 63, row = threadIdx.x >> 6;
-  const int64_t i0 = t0 * 64, k0 = tk * 64;
   // load along the source's contiguous dimension
+  const int lane = threadIdx.x & 63, row = threadIdx.x >> 6;
+  const int64_t i0 = int64_t(t0) * (SrcLeft ? 64 : N), k0 = int64_t(tk) * (SrcLeft ? N : 64);
 #pragma unroll
-  for (int r = 0; r < 8; ++r) {
+  for (int r = 0; r < N / 8; ++r) {
     const int q = row + 8 * r;
     if (SrcLeft) {
       const int64_t i = i0 + lane, k = k0 + q;
@@ -152,15 +157,16 @@ __global__ __launch_bounds__(512) void k_layout_transpose(W* __restrict__ dst, c
   }
   __syncthreads();
   // store along the destination's contiguous dimension
+  const int near = threadIdx.x % N, far = threadIdx.x / N;
 #pragma unroll
-  for (int r = 0; r < 8; ++r) {
-    const int q = row + 8 * r;
+  for (int r = 0; r < N / 8; ++r) {
+    const int q = far + 512 / N * r;
     if (SrcLeft) {  // destination LayoutRight: k fastest; tile[k_local][i_local]
-      const int64_t k = k0 + lane, i = i0 + q;
-      if (i < sh.e0 && k < sh.elast) __builtin_nontemporal_store(tile[lane][q], &dst[(i * sh.M + midR) * sh.elast + k]);
+      const int64_t k = k0 + near, i = i0 + q;
+      if (i < sh.e0 && k < sh.elast) __builtin_nontemporal_store(tile[near][q], &dst[(i * sh.M + midR) * sh.elast + k]);
     } else {  // destination LayoutLeft: i fastest; tile[i_local][k_local]
-      const int64_t i = i0 + lane, k = k0 + q;
-      if (i < sh.e0 && k < sh.elast) __builtin_nontemporal_store(tile[lane][q], &dst[i + sh.e0 * (midL + sh.M * k)]);
+      const int64_t i = i0 + near, k = k0 + q;
+      if (i < sh.e0 && k < sh.elast) __builtin_nontemporal_store(tile[near][q], &dst[i + sh.e0 * (midL + sh.M * k)]);
     }
   }
 }
@@ -193,15 +199,18 @@ bool layout_transpose(const MI355X& exec, const DV& dst, const SV& src) {
     sh.nmid = int(R) - 2;
     for (int d = 0; d < 4; ++d) sh.mid[d] = 1;
     for (int d = 0; d < sh.nmid; ++d) {
-      sh.mid[d] = int64_t(dst.extent(d + 1));
-      sh.M *= sh.mid[d];
+      sh.M *= int64_t(dst.extent(d + 1));
+      sh.mid[d] = uint32_t(dst.extent(d + 1));
     }
     if (sh.M == 0) return true;
-    sh.tiles0    = (sh.e0 + 63) / 64;
-    sh.tileslast = (sh.elast + 63) / 64;
-    const int64_t blocks = sh.tiles0 * sh.tileslast * sh.M;
-    if (blocks > 0x7fffffff) return false;
-    using W  = transpose_word_t<T>;
+    using W                 = transpose_word_t<T>;
+    constexpr int64_t N     = transpose_narrow<W>;
+    const int64_t tiles0    = lr ? (sh.e0 + 63) / 64 : (sh.e0 + N - 1) / N;
+    const int64_t tileslast = lr ? (sh.elast + N - 1) / N : (sh.elast + 63) / 64;
+    if (tiles0 > 0x7fffffff || tileslast > 0x7fffffff / tiles0 || sh.M > 0x7fffffff / (tiles0 * tileslast)) return false;
+    const int64_t blocks = tiles0 * tileslast * sh.M;
+    sh.tiles0            = uint32_t(tiles0);
+    sh.tileslast         = uint32_t(tileslast);
     W* d     = reinterpret_cast<W*>(dst.data());
     const W* s_ = reinterpret_cast<const W*>(src.data());
     const void* k = lr ? reinterpret_cast<const void*>(&k_layout_transpose<W, true>)

@@ -49,6 +49,13 @@ def test_layout_copy(paths, oracle, shape, dst_layout, src_layout):
     assert np.array_equal(dst, src)
 
 
+@pytest.mark.parametrize("shape", [(33, 2, 65), (31, 5, 32), (32, 1, 33), (64, 3, 31), (129, 2, 96), (16, 1, 16)])
+@pytest.mark.parametrize("dst_layout,src_layout", [(1, 0), (0, 1)])
+def test_layout_copy_tile_edges(paths, oracle, shape, dst_layout, src_layout):
+    """Both sides of the transpose's 64 x 32 tiles, in either direction."""
+    test_layout_copy(paths, oracle, shape, dst_layout, src_layout)
+
+
 def test_transpose_512_cubed(paths, oracle):
     """The measured case: 512^3 doubles, LayoutLeft -> LayoutRight."""
     P = paths
