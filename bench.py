@@ -253,7 +253,8 @@ def leg_md_team(K, P, timer):
     U, V = K.DeviceBuffer(m**3 * 8), K.DeviceBuffer(m**3 * 8)
     chk(P.kkmx_fill_uniform_f64(U.ptr, m**3, 5, 0.0, 1.0))
     chk(P.kkmx_fill_uniform_f64(V.ptr, m**3, 5, 0.0, 1.0))
-    st = _timeit(K, timer, lambda: chk(P.kkmx_stencil7_sweeps(U.ptr, V.ptr, n, 10, 0.4, 0.1, 0, 0, 0)), reps=3, warm=1)
+    # the default tile by name: ten MDRange dispatches, none of them in pairs
+    st = _timeit(K, timer, lambda: chk(P.kkmx_stencil7_sweeps(U.ptr, V.ptr, n, 10, 0.4, 0.1, 64, 4, 1)), reps=3, warm=1)
     del U, V
     nrows = 1 << 20
     rp = K.DeviceBuffer((nrows + 1) * 8)

@@ -144,7 +144,10 @@ int kkmx_scan_excl_f64(const double* in_dev, double* out_dev, int64_t n, double*
  * u_dev, v_dev: (n+2)^3 doubles, LayoutLeft (first index fastest), 1-cell
  * halo; v(i,j,k) = c0*u(i,j,k) + c1*(sum of the 6 neighbours) for the
  * interior.  t0..t2 = tile shape (0 = the space's default).  The sweeps
- * variant ping-pongs u -> v -> u ...  (reference: core/src/KokkosExp_MDRangePolicy.hpp:158-426) */
+ * variant leaves both grids as sweeps u -> v -> u ... do, with the same bits;
+ * with the default tile, at least 96 points a side and at least 5 sweeps it
+ * takes them in pairs, each one pass over memory (a TeamPolicy dispatch in
+ * place of two MDRange ones).  (reference: core/src/KokkosExp_MDRangePolicy.hpp:158-426) */
 int kkmx_stencil7(const double* u_dev, double* v_dev, int64_t n, double c0, double c1, int t0, int t1, int t2);
 int kkmx_stencil7_sweeps(double* u_dev, double* v_dev, int64_t n, int sweeps, double c0, double c1, int t0, int t1,
                          int t2);

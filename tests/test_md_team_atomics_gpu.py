@@ -54,6 +54,24 @@ def test_stencil7_matches_oracle(paths, oracle, n, sweeps, tile):
     assert err <= 1e-12
 
 
+# Sweeps in pairs against single ones, which a tile by name asks for: the
+# smallest size that pairs, one tile less and more than whole 60 x 28 tiles,
+# more and fewer sweeps than whole pairs, and the last size without pairs.
+@pytest.mark.parametrize("n,sweeps", [(95, 7), (96, 5), (97, 4), (112, 9), (113, 10), (119, 6), (120, 7), (121, 5),
+                                      (200, 13), (257, 8)])
+def test_stencil7_sweeps_in_pairs(paths, oracle, n, sweeps):
+    P = paths
+    m = n + 2
+    u0, v0 = oracle.fill_uniform_f64(m**3, 5, -1.0, 1.0), oracle.fill_uniform_f64(m**3, 6, -1.0, 1.0)
+    got = []
+    for tile in ((0, 0, 0), (64, 4, 1)):  # the grids' boundary values differ
+        U, V = dev(u0), dev(v0)
+        run(P, P.kkmx_stencil7_sweeps(U.ptr, V.ptr, n, sweeps, C0, C1, *tile))
+        got.append([U.download(np.float64, m**3), V.download(np.float64, m**3)])
+    for a, b in zip(*got):
+        assert np.array_equal(a.view(np.uint64), b.view(np.uint64))
+
+
 def test_stencil7_full_size_config3(paths, oracle):
     """512^3 interior, 10 sweeps, input U[0,1) seed 5."""
     P = paths
