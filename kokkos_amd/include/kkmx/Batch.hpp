@@ -74,6 +74,7 @@ constexpr int kBatchShapes = 8;
 constexpr BatchShape kBatchShape[kBatchShapes] = {{256, 1, 16}, {256, 4, 4}, {256, 4, 8},  {512, 4, 4},
                                                   {1024, 1, 16}, {512, 4, 8}, {1024, 4, 4}, {512, 1, 32}};
 constexpr int kBatchDefaultShape = 5;
+constexpr int kBatchSmallShape   = 3;
 static_assert(kBatchShapes == kBatchShapeCandidates, "the batch_shape tuning variable lists every tile shape");
 constexpr int64_t kBatchDetTiles = 2048;
 
@@ -658,12 +659,27 @@ class BatchDispatch {
     (void)mx_free(m_control, nullptr);
     m_desc = nullptr;
   }
+  // The default tile shape: 16384-element tiles, unless all tiles of half that
+  // size run at once, two a CU.  Such a batch takes as long as its longest tile
+  // with its claim and look-back: 64 ops of 2^8..2^16 elements 17.4 us with the
+  // large tiles and 11.8 with the small ones, 16 of 2^4..2^12 12.0 and 7.7; with
+  // more tiles the large ones' fewer claims pay, 34.2 us and 36.0 for 64 ops of
+  // 2^8..2^20.
+  int default_shape() const {
+    const int64_t tile = Impl::kBatchShape[Impl::kBatchSmallShape].tile();
+    int64_t tiles      = 0;
+    for (const auto& d : m_ops) tiles += (d.n + tile - 1) / tile;
+    const int64_t cus = MI355X::impl_cu_count() > 0 ? MI355X::impl_cu_count() : 256;
+    return tiles <= 2 * cus ? Impl::kBatchSmallShape : Impl::kBatchDefaultShape;
+  }
   // The tile shape: the learned tuner's answer when a tuning tool is
   // loaded, else the default.
   int tuned_shape() const {
-    if (m_ops.empty() || !Tools::Experimental::have_tuning_tool()) return Impl::kBatchDefaultShape;
-    const int c = Impl::request_launch_candidate(Impl::LaunchVar::Batch, tuning_features(), Impl::kBatchDefaultShape);
-    return (c >= 0 && c < Impl::kBatchShapes) ? c : Impl::kBatchDefaultShape;
+    if (m_ops.empty()) return Impl::kBatchDefaultShape;
+    const int dflt = default_shape();
+    if (!Tools::Experimental::have_tuning_tool()) return dflt;
+    const int c = Impl::request_launch_candidate(Impl::LaunchVar::Batch, tuning_features(), dflt);
+    return (c >= 0 && c < Impl::kBatchShapes) ? c : dflt;
   }
   MI355X m_exec;
   std::vector<Impl::BatchDesc> m_ops;

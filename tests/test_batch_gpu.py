@@ -212,3 +212,16 @@ def test_batch_full_workload_4096_ops(paths, oracle):
     K.fence()
     check_run(run, oracle, wl, exp)
     run.close()
+
+
+@pytest.mark.parametrize("nops,shape", [(1, 3), (512, 3), (513, 5)])
+def test_batch_default_shape(paths, oracle, nops, shape):
+    """Without a tuning tool: the small tiles while all of them run at once,
+    two a CU of 256, and the large ones beyond; both give the oracle's results."""
+    wl = small_workload(nops, 13, 0, 12)
+    run = B.BatchRun(wl)
+    assert run.shape == shape
+    run.run(B.MODE_FUSED, 1)
+    K.fence()
+    check_run(run, oracle, wl, expected(oracle, wl, run.inputs()))
+    run.close()
