@@ -816,6 +816,13 @@ int32_t* hist_rows_space(size_t elems) {
         Kokkos::view_alloc(Kokkos::WithoutInitializing, std::string("kkmx_hist_rows")), elems);
   return rows->data();
 }
+// Teams, and rows of the table, for n keys: one per CU, fewer where a team would
+// have less than 16384 keys.  A team pays for its bins whatever its keys, in
+// LDS and with a row written and read again: 65536 bins cost 256 rows 40 us.
+int hist_teams(int64_t n, int cus) {
+  const int64_t want = (n + 16383) / 16384;
+  return int(want < 1 ? 1 : want < cus ? want : cus);
+}
 struct ScatterAdd {
   DevView<const double> vals;
   DevView<const int32_t> idx;
@@ -1461,15 +1468,16 @@ int kkmx_histogram(const int32_t* keys, int64_t n, int32_t* bins, int32_t nbins,
       const int cus_ = Kokkos::MI355X::impl_cu_count();
       const size_t budget = Kokkos::TeamPolicy<Kokkos::MI355X>(cus_, 1024).scratch_size_max(0);
       if (HistPacked::scratch_words(nbins) * 4 <= budget && n / cus_ < HistPacked::kMaxKeysPerTeam - 4096) {
-        int32_t* rows = hist_rows_space(size_t(cus_) * nbins);
+        const int teams = hist_teams(n, cus_);
+        int32_t* rows   = hist_rows_space(size_t(teams) * nbins);
         using Rows = Kokkos::View<int32_t**, Kokkos::LayoutRight, Kokkos::MI355XSpace, Kokkos::MemoryTraits<Kokkos::Unmanaged>>;
-        auto pol = Kokkos::TeamPolicy<Kokkos::MI355X>(cus_, 1024)
+        auto pol = Kokkos::TeamPolicy<Kokkos::MI355X>(teams, 1024)
                        .set_scratch_size(0, Kokkos::PerTeam(HistPacked::scratch_words(nbins) * 4));
-        Kokkos::parallel_for("kkmx::hist_packed", pol, HistPacked{K, Rows(rows, cus_, nbins), n, nbins});
+        Kokkos::parallel_for("kkmx::hist_packed", pol, HistPacked{K, Rows(rows, teams, nbins), n, nbins});
         const int sum_teams = (nbins + HistRowSum::kBins - 1) / HistRowSum::kBins;
         auto sum_pol = Kokkos::TeamPolicy<Kokkos::MI355X>(sum_teams, HistRowSum::kBins * HistRowSum::kWaves)
                            .set_scratch_size(0, Kokkos::PerTeam(size_t(HistRowSum::kBins) * HistRowSum::kWaves * 4));
-        Kokkos::parallel_for("kkmx::hist_row_sum", sum_pol, HistRowSum{decltype(HistRowSum::rows)(rows, cus_, nbins), B});
+        Kokkos::parallel_for("kkmx::hist_row_sum", sum_pol, HistRowSum{decltype(HistRowSum::rows)(rows, teams, nbins), B});
         return;
       }
     }
@@ -1480,15 +1488,16 @@ int kkmx_histogram(const int32_t* keys, int64_t n, int32_t* bins, int32_t nbins,
       const size_t budget = Kokkos::TeamPolicy<Kokkos::MI355X>(cus, 1024).scratch_size_max(0);
       const int64_t fit   = int64_t(budget / 4) - int64_t(HistRows::kHotCopies) * (hot + 1);
       if (lb3 > fit) lb3 = int32_t(fit);
-      int32_t* rows = hist_rows_space(size_t(cus) * nbins);
+      const int teams = hist_teams(n, cus);
+      int32_t* rows   = hist_rows_space(size_t(teams) * nbins);
       using Rows = Kokkos::View<int32_t**, Kokkos::LayoutRight, Kokkos::MI355XSpace, Kokkos::MemoryTraits<Kokkos::Unmanaged>>;
-      auto pol = Kokkos::TeamPolicy<Kokkos::MI355X>(cus, 1024)
+      auto pol = Kokkos::TeamPolicy<Kokkos::MI355X>(teams, 1024)
                      .set_scratch_size(0, Kokkos::PerTeam(HistRows::scratch_bytes(lb3, hot)));
-      Kokkos::parallel_for("kkmx::hist_rows", pol, HistRows{K, Rows(rows, cus, nbins), n, nbins, lb3, hot});
+      Kokkos::parallel_for("kkmx::hist_rows", pol, HistRows{K, Rows(rows, teams, nbins), n, nbins, lb3, hot});
       const int sum_teams = (nbins + HistRowSum::kBins - 1) / HistRowSum::kBins;
       auto sum_pol = Kokkos::TeamPolicy<Kokkos::MI355X>(sum_teams, HistRowSum::kBins * HistRowSum::kWaves)
                          .set_scratch_size(0, Kokkos::PerTeam(size_t(HistRowSum::kBins) * HistRowSum::kWaves * 4));
-      Kokkos::parallel_for("kkmx::hist_row_sum", sum_pol, HistRowSum{decltype(HistRowSum::rows)(rows, cus, nbins), B});
+      Kokkos::parallel_for("kkmx::hist_row_sum", sum_pol, HistRowSum{decltype(HistRowSum::rows)(rows, teams, nbins), B});
       return;
     }
     if (mode >= 2 && reinterpret_cast<uintptr_t>(keys) % 16 == 0) {

@@ -341,3 +341,16 @@ def test_scatter_f64_captured(paths, oracle):
         assert np.array_equal(B.download(np.float64, nbins), ref * (2 * k + 2))
     K.check(rt.mx_graph_exec_destroy(ex))
     K.check(rt.mx_graph_destroy(graph))
+
+
+@pytest.mark.parametrize("n", [1, 3, 16384, 16385, 100003, 256 * 16384, 256 * 16384 + 1])
+@pytest.mark.parametrize("nb", [100, 300, 65536, 100000])
+def test_histogram_mode3_team_counts(paths, oracle, n, nb):
+    """One team, two, several and all of them, in the packed layout, with all
+    bins replicated and with bins above the LDS range."""
+    P = paths
+    keys = oracle.fill_uniform_i32(n, 95, 0, nb - 1)
+    keys[: n // 3] %= 7
+    Kb, Bb = dev(keys), dev(np.full(nb, 5, np.int32))
+    run(P, P.kkmx_histogram(Kb.ptr, n, Bb.ptr, nb, 3, 0))
+    assert np.array_equal(Bb.download(np.int32, nb), oracle.histogram(keys, nb) + 5)
