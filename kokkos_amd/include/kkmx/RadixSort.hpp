@@ -13,7 +13,9 @@
 // sample shows those to tell them apart (k_radix_sample), and neighbours that
 // share them are put right on the way back (k_radix_finish).  A sort is a fixed
 // sequence of launches and one wait, two for 8-byte keys that are not trimmed.
-// Up to kRadixSmall keys are sorted by one block in LDS.
+// Few keys are sorted in LDS: those of one block by a single launch
+// (k_radix_small), those of several blocks' runs by one more that places every
+// key among the other runs (k_radix_merge).
 //
 // Reading the keys twice a pass costs less than learning the positions in one
 // sweep: a decoupled look-back over tiles took 0.42 ms of a 1.0 ms pass over
@@ -609,26 +611,31 @@ __global__ __launch_bounds__(kRadixFinishLanes) void k_radix_finish(const int64_
   if (broken) *status = 1;
 }
 
-// Up to kRadixSmall keys, sorted by one block in LDS: every pass ranks the
-// keys the lanes hold, places them in digit order in LDS and takes them back
-// in that order.  Launch latency bounds it below a few thousand keys, then
-// the ranking of one CU.
+// Runs of at most 1024 x Items keys, each sorted by one block in LDS: every
+// pass ranks the keys the lanes hold, places them in digit order in LDS and
+// takes them back in that order.  One run is a whole sort, in place; more of
+// them go to `out` and `pay_out`, encoded, for k_radix_merge.  Launch latency
+// and the digits' chain of barriers bound it, about 2.5 us a digit at one key a
+// lane and 5 at eight.
 constexpr int kRadixSmallLanes = 1024;
-constexpr int kRadixSmallItems = 8;
-constexpr int kRadixSmall      = kRadixSmallLanes * kRadixSmallItems;
 
-template <class T, class PT, bool Iota>
-__global__ __launch_bounds__(kRadixSmallLanes) void k_radix_small(typename RadixKey<T>::U* keys, PT* pay, const int n) {
+template <class T, class PT, bool Iota, int Items, bool Whole>
+__global__ __launch_bounds__(kRadixSmallLanes) void k_radix_small(typename RadixKey<T>::U* keys, PT* pay, const int all_n,
+                                                                  typename RadixKey<T>::U* out, PT* pay_out) {
   using R              = RadixKey<T>;
   using U              = typename R::U;
   constexpr bool Pairs = !std::is_same<PT, NoPayload>::value;
   constexpr int NW     = kRadixSmallLanes / 64;
-  constexpr int Items  = kRadixSmallItems;
+  constexpr int Run    = kRadixSmallLanes * Items;
   using Wide           = std::conditional_t<(Pairs && sizeof(PT) > sizeof(U)), uint64_t, U>;
-  __shared__ Wide s_tile[kRadixSmall];
+  __shared__ Wide s_tile[Run];
   __shared__ uint32_t wcnt[NW][256];
   __shared__ uint32_t s_wave[4];
   __shared__ U s_and, s_or;
+  const int first = Whole ? 0 : int(blockIdx.x) * Run;
+  const int n     = Whole || all_n - first < Run ? all_n - first : Run;
+  keys += first;
+  if constexpr (Pairs) pay += first;
   U* key_tile  = reinterpret_cast<U*>(s_tile);
   PT* pay_tile = reinterpret_cast<PT*>(s_tile);
   const int t = threadIdx.x, w = t >> 6, l = t & 63;
@@ -651,7 +658,7 @@ __global__ __launch_bounds__(kRadixSmallLanes) void k_radix_small(typename Radix
       all &= R::canon(u[r]);
       any |= R::canon(u[r]);
       if constexpr (Pairs) {
-        if constexpr (Iota) v[r] = PT(i);
+        if constexpr (Iota) v[r] = PT(first + i);
         else v[r] = pay[i];
       }
     }
@@ -710,10 +717,72 @@ __global__ __launch_bounds__(kRadixSmallLanes) void k_radix_small(typename Radix
   for (int r = 0; r < Items; ++r) {
     const int i = wfirst + r * 64 + l;
     if (r < rounds && i < n) {
-      keys[i] = R::decode(u[r]);
-      if constexpr (Pairs) pay[i] = v[r];
+      if constexpr (Whole) {
+        keys[i] = R::decode(u[r]);
+        if constexpr (Pairs) pay[i] = v[r];
+      } else {
+        out[first + i] = u[r];
+        if constexpr (Pairs) pay_out[first + i] = v[r];
+      }
     }
   }
+}
+
+// Places the keys of several sorted runs: a key's position is its own in its
+// run and, for every other run, the number of keys there that go before it,
+// those of earlier runs also where they are equal.  The searches' latency
+// bounds it, so a block takes 64 keys only, neighbours in order that read the
+// same lines, its wavefronts search different runs and each kRadixAbreast of
+// them at once: 64 runs of 1024 (int64, 8-byte value) pairs take 79 us with
+// their sort, 157 with one wavefront for all runs; 8 or 16 at once are no
+// faster.
+constexpr int kRadixAbreast    = 4;
+constexpr int kRadixMergeWaves = 4;
+
+template <class T, class PT, int Run>
+__global__ __launch_bounds__(64 * kRadixMergeWaves) void k_radix_merge(const typename RadixKey<T>::U* in,
+                                                                       const PT* pay_in, const int n,
+                                                                       typename RadixKey<T>::U* keys, PT* pay) {
+  using R = RadixKey<T>;
+  using U = typename R::U;
+  __shared__ int s_at[kRadixMergeWaves][64];
+  const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int i    = int(blockIdx.x) * 64 + l;
+  const int own  = int(blockIdx.x) / (Run / 64);
+  const int runs = (n + Run - 1) / Run;
+  const U u      = in[i < n ? i : n - 1];
+  const U key    = R::canon(u);
+  int at         = 0;
+  for (int q = w; q < runs; q += kRadixAbreast * kRadixMergeWaves) {
+    int pos[kRadixAbreast], len[kRadixAbreast];
+#pragma unroll
+    for (int c = 0; c < kRadixAbreast; ++c) {
+      const int run = q + c * kRadixMergeWaves;
+      pos[c]        = 0;
+      len[c]        = run >= runs || run == own ? 0 : n - run * Run < Run ? n - run * Run : Run;
+    }
+    // the keys below pos go before, those from pos + 2 * step - 1 on do not
+    for (int step = Run; step > 0; step >>= 1) {
+#pragma unroll
+      for (int c = 0; c < kRadixAbreast; ++c) {
+        const int run = q + c * kRadixMergeWaves, k = pos[c] + step;
+        if (k <= len[c]) {
+          const U other = R::canon(in[run * Run + k - 1]);
+          if (other < key || (other == key && run < own)) pos[c] = k;
+        }
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < kRadixAbreast; ++c) at += pos[c];
+  }
+  s_at[w][l] = at;
+  __syncthreads();
+  if (w > 0 || i >= n) return;
+  at = i - own * Run;
+#pragma unroll
+  for (int q = 0; q < kRadixMergeWaves; ++q) at += s_at[q][l];
+  keys[at] = R::decode(u);
+  if constexpr (!std::is_same<PT, NoPayload>::value) pay[at] = pay_in[i];
 }
 
 // ------------------------------------------------------------------ host side
@@ -731,6 +800,9 @@ struct RadixWorkspace {
   uint32_t* status      = nullptr;  // pinned host word that k_radix_finish reports to
   int turn              = 0;
   bool hooked           = false;
+  // under the mutex
+  void hook();
+  void fit(size_t need);
 };
 
 inline RadixWorkspace& radix_workspace() {
@@ -738,7 +810,26 @@ inline RadixWorkspace& radix_workspace() {
   return w;
 }
 
+// Where merged sorts keep their runs: several, as such sorts on different
+// streams may well run side by side, and a device runs about four at once.
+// A call holds one until its kernels have run.
+struct RadixMergeSpace {
+  std::mutex mtx;
+  void* buf = nullptr;
+};
+constexpr int kRadixMergeSpaces = 4;
+inline RadixMergeSpace* radix_merge_spaces() {
+  static RadixMergeSpace s[kRadixMergeSpaces];
+  return s;
+}
+
 inline void radix_workspace_release() {
+  for (int q = 0; q < kRadixMergeSpaces; ++q) {
+    RadixMergeSpace& s = radix_merge_spaces()[q];
+    std::lock_guard<std::mutex> lock(s.mtx);
+    if (s.buf) KKMX_SAFE_CALL(mx_free(s.buf, nullptr));
+    s.buf = nullptr;
+  }
   RadixWorkspace& w = radix_workspace();
   std::lock_guard<std::mutex> lock(w.mtx);
   if (w.buf) KKMX_SAFE_CALL(mx_free(w.buf, nullptr));
@@ -750,6 +841,20 @@ inline void radix_workspace_release() {
   w.bytes   = 0;
   w.turn    = 0;
   w.hooked  = false;
+}
+
+inline void RadixWorkspace::hook() {
+  if (!hooked) push_finalize_hook(&radix_workspace_release);
+  hooked = true;
+}
+
+inline void RadixWorkspace::fit(size_t need) {
+  if (bytes >= need) return;
+  if (buf) KKMX_SAFE_CALL(mx_free(buf, nullptr));
+  buf   = nullptr;
+  bytes = 0;
+  KKMX_SAFE_CALL(mx_malloc(&buf, need, nullptr));
+  bytes = need;
 }
 
 template <class Unused = void>
@@ -839,22 +944,13 @@ void radix_sort_passes(const MI355X& exec, typename RadixKey<T>::U* k0, int64_t 
   const size_t need        = key_bytes + pay_bytes + radix_round(size_t(segments) * 256 * sizeof(uint32_t));
   RadixWorkspace& ws       = radix_workspace();
   std::lock_guard<std::mutex> lock(ws.mtx);
-  if (ws.bytes < need) {
-    if (ws.buf) KKMX_SAFE_CALL(mx_free(ws.buf, nullptr));
-    ws.buf   = nullptr;
-    ws.bytes = 0;
-    KKMX_SAFE_CALL(mx_malloc(&ws.buf, need, nullptr));
-    ws.bytes = need;
-  }
+  ws.hook();
+  ws.fit(need);
   if (!ws.control) {
     void* c = nullptr;
     KKMX_SAFE_CALL(mx_malloc(&c, sizeof(RadixControl), nullptr));
     ws.control = static_cast<RadixControl*>(c);
     mx_launch_kernel(reinterpret_cast<const void*>(&k_radix_control_init<>), 1, 64, 0, exec.stream(), ws.control);
-  }
-  if (!ws.hooked) {
-    push_finalize_hook(&radix_workspace_release);
-    ws.hooked = true;
   }
   if (!ws.status) {
     void* h = nullptr;
@@ -901,6 +997,51 @@ void radix_sort_passes(const MI355X& exec, typename RadixKey<T>::U* k0, int64_t 
   }
 }
 
+// One block sorts up to 16 KiB of keys.  Up to kRadixMerged keys are sorted in
+// runs that k_radix_merge puts together, at most 24 of 1024 keys and then at
+// most 24 of 4096; more keys go through the passes, which launch two or three
+// kernels a digit but do not read every run for every key.  In us, one block /
+// runs of 1024 / of 4096 / passes, int32 keys: 29 / 29 / 32 at 3000, 38 / 30 /
+// 36 at 8192, runs 33 / 37 and passes 55 at 16384, 45 / 39 and 61 at 32768, 66 /
+// 46 and 54 at 65536, 122 / 63 and 57 at 131072; (int64, 8-byte value) pairs:
+// 37 / 37 / 39 at 1500, 43 / 37 / 45 at 3000, 65 / 38 / 54 at 8192, 43 / 53 and
+// 94 at 16384, 55 / 56 and 100 at 32768, 79 / 65 and 94 at 65536, 143 / 84 and
+// 98 at 131072, where pairs of few digits already gain from the passes.
+template <class U>
+constexpr int kRadixSmallItems    = sizeof(U) == 4 ? 4 : 2;
+constexpr int kRadixMergeRuns     = 24;
+constexpr int kRadixMerged        = kRadixMergeRuns * 4 * kRadixSmallLanes;
+constexpr size_t kRadixMergeBytes = size_t(kRadixMerged) * 16;  // 8-byte keys and payload
+
+template <class T, class PT, bool Iota, int Items>
+void radix_sort_merged(const MI355X& exec, typename RadixKey<T>::U* k0, int n, PT* payload) {
+  using U              = typename RadixKey<T>::U;
+  constexpr bool pairs = !std::is_same<PT, NoPayload>::value;
+  constexpr int run    = kRadixSmallLanes * Items;
+  std::unique_lock<std::mutex> lock;
+  RadixMergeSpace* space = radix_merge_spaces();
+  for (int q = 0; q < kRadixMergeSpaces && !lock.owns_lock(); ++q) {
+    space = radix_merge_spaces() + q;
+    lock  = std::unique_lock<std::mutex>(space->mtx, std::try_to_lock);
+  }
+  if (!lock.owns_lock()) lock.lock();
+  if (!space->buf) {
+    {
+      std::lock_guard<std::mutex> hooks(radix_workspace().mtx);
+      radix_workspace().hook();
+    }
+    KKMX_SAFE_CALL(mx_malloc(&space->buf, kRadixMergeBytes, nullptr));
+  }
+  U* k1  = static_cast<U*>(space->buf);
+  PT* p1 = pairs ? reinterpret_cast<PT*>(static_cast<char*>(space->buf) + kRadixMergeBytes / 2) : nullptr;
+  mx_launch_kernel(reinterpret_cast<const void*>(&k_radix_small<T, PT, Iota, Items, false>), unsigned((n + run - 1) / run),
+                   kRadixSmallLanes, 0, exec.stream(), k0, payload, n, k1, p1);
+  mx_launch_kernel(reinterpret_cast<const void*>(&k_radix_merge<T, PT, run>), unsigned((n + 63) / 64),
+                   64 * kRadixMergeWaves, 0, exec.stream(), k1, p1, n, k0, payload);
+  // the space is free for the next call once the stream has run these
+  exec.fence("Kokkos::sort: merged runs");
+}
+
 // Ascending LSD radix sort of n keys in place (device memory), on exec.
 // With a payload (n device words of PT), the sort is of (key, payload)
 // pairs and the payload is permuted with the keys, in place; with iota the
@@ -915,11 +1056,18 @@ void radix_sort(const MI355X& exec, T* keys, int64_t n, PT* payload = nullptr) {
   if (n < 1 || (n < 2 && !Iota)) return;
   using U = typename RadixKey<T>::U;
   U* k0   = reinterpret_cast<U*>(keys);
-  if (n <= kRadixSmall) {
-    int count = int(n);
-    mx_launch_kernel(reinterpret_cast<const void*>(&k_radix_small<T, PT, Iota>), 1, kRadixSmallLanes, 0, exec.stream(),
-                     k0, payload, count);
+  if (n <= kRadixSmallLanes * kRadixSmallItems<U>) {
+    int count  = int(n);
+    U* no_out  = nullptr;
+    PT* no_pay = nullptr;
+    mx_launch_kernel(reinterpret_cast<const void*>(&k_radix_small<T, PT, Iota, kRadixSmallItems<U>, true>), 1,
+                     kRadixSmallLanes, 0, exec.stream(), k0, payload, count, no_out, no_pay);
     exec.fence("Kokkos::sort: keys of one block");
+    return;
+  }
+  if (n <= kRadixMerged) {
+    if (n <= kRadixMergeRuns * kRadixSmallLanes) radix_sort_merged<T, PT, Iota, 1>(exec, k0, int(n), payload);
+    else radix_sort_merged<T, PT, Iota, 4>(exec, k0, int(n), payload);
     return;
   }
   if (n >= kRadixLarge) radix_sort_passes<T, PT, Iota, RadixShape<T, PT, true>>(exec, k0, n, payload);

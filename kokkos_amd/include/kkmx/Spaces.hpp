@@ -84,7 +84,11 @@ inline GlobalState& global_state() {
 
 inline bool is_initialized() noexcept { return Impl::global_state().state.load() == 1; }
 inline bool is_finalized() noexcept { return Impl::global_state().state.load() == 2; }
-inline void push_finalize_hook(void (*f)()) { Impl::global_state().finalize_hooks.push_back(f); }
+inline void push_finalize_hook(void (*f)()) {
+  static std::mutex mtx;  // workspaces register from any thread
+  std::lock_guard<std::mutex> lock(mtx);
+  Impl::global_state().finalize_hooks.push_back(f);
+}
 namespace Impl {
 inline bool& tune_internals() noexcept { return global_state().tune_internals; }
 }  // namespace Impl

@@ -154,6 +154,33 @@ def test_sort_edges(paths, oracle, n, code, vbytes):
     assert np.array_equal(Dk.download(TYPES[code], n).view(bits), x[order].view(bits))
 
 
+@pytest.mark.parametrize("form", ["any", "few", "equal", "ascending", "descending"])
+@pytest.mark.parametrize("n", [2048, 2049, 4096, 4097, 24 * 1024, 24 * 1024 + 1, 7 * 4096 + 1, 24 * 4096, 24 * 4096 + 1])
+@pytest.mark.parametrize("code,vbytes", [(0, 0), (1, 8), (2, 8), (3, 4), (4, 4), (5, 0)])
+def test_sort_in_runs(paths, oracle, n, code, vbytes, form):
+    """Either side of one block, of 24 runs of 1024 keys and of 24 runs of 4096;
+    equal keys keep their order across runs."""
+    P = paths
+    x = keys_for(oracle, code, n, 500 + code)
+    if form == "few":
+        x = x[np.arange(n) * 7919 % 5]
+    elif form == "equal":
+        x[:] = x[0]
+    elif form != "any":
+        x = np.sort(x)[:: 1 if form == "ascending" else -1].copy()
+    order = np.argsort(x, kind="stable")
+    bits = {4: np.uint32, 8: np.uint64}[x.dtype.itemsize]
+    Dk = K.DeviceBuffer.from_array(x)
+    if vbytes == 0:
+        run(P, P.kkmx_sort(Dk.ptr, n, code))
+    else:
+        vdt = np.uint32 if vbytes == 4 else np.uint64
+        Dv = K.DeviceBuffer.from_array(np.arange(n, dtype=vdt))
+        run(P, P.kkmx_sort_by_key(Dk.ptr, Dv.ptr, n, code, vbytes, 0))
+        assert np.array_equal(Dv.download(vdt, n), order.astype(vdt))
+    assert np.array_equal(Dk.download(TYPES[code], n).view(bits), x[order].view(bits))
+
+
 @pytest.mark.parametrize("form", ["spread", "runs", "crowd", "one_long_run", "equal", "six_digits"])
 @pytest.mark.parametrize("n", [8193, 100003, (1 << 21) + 5])
 @pytest.mark.parametrize("code,vbytes", [(1, 0), (3, 0), (5, 8), (3, 4)])
