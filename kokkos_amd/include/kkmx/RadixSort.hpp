@@ -1013,12 +1013,34 @@ constexpr int kRadixMergeRuns     = 24;
 constexpr int kRadixMerged        = kRadixMergeRuns * 4 * kRadixSmallLanes;
 constexpr size_t kRadixMergeBytes = size_t(kRadixMerged) * 16;  // 8-byte keys and payload
 
-template <class T, class PT, bool Iota, int Items>
-void radix_sort_merged(const MI355X& exec, typename RadixKey<T>::U* k0, int n, PT* payload) {
-  using U              = typename RadixKey<T>::U;
-  constexpr bool pairs = !std::is_same<PT, NoPayload>::value;
-  constexpr int run    = kRadixSmallLanes * Items;
-  std::unique_lock<std::mutex> lock;
+// The launches of a sort of at most kRadixMerged keys, which are in order, and
+// `space` free again, once the stream has run them.  `space` holds
+// kRadixMergeBytes; one block's keys leave it alone.
+template <class T, class PT, bool Iota>
+void radix_sort_few(const MI355X& exec, typename RadixKey<T>::U* k0, int n, PT* payload, void* space) {
+  using U = typename RadixKey<T>::U;
+  U* k1   = static_cast<U*>(space);
+  PT* p1  = nullptr;
+  if constexpr (!std::is_same<PT, NoPayload>::value)
+    p1 = reinterpret_cast<PT*>(static_cast<char*>(space) + kRadixMergeBytes / 2);
+  const auto runs = [&](const void* sort, const void* merge, int run) {
+    mx_launch_kernel(sort, unsigned((n + run - 1) / run), kRadixSmallLanes, 0, exec.stream(), k0, payload, n, k1, p1);
+    mx_launch_kernel(merge, unsigned((n + 63) / 64), 64 * kRadixMergeWaves, 0, exec.stream(), k1, p1, n, k0, payload);
+  };
+  constexpr int R = kRadixSmallLanes;
+  if (n <= R * kRadixSmallItems<U>)
+    mx_launch_kernel(reinterpret_cast<const void*>(&k_radix_small<T, PT, Iota, kRadixSmallItems<U>, true>), 1, R, 0,
+                     exec.stream(), k0, payload, n, k1, p1);
+  else if (n <= kRadixMergeRuns * R)
+    runs(reinterpret_cast<const void*>(&k_radix_small<T, PT, Iota, 1, false>),
+         reinterpret_cast<const void*>(&k_radix_merge<T, PT, R>), R);
+  else
+    runs(reinterpret_cast<const void*>(&k_radix_small<T, PT, Iota, 4, false>),
+         reinterpret_cast<const void*>(&k_radix_merge<T, PT, 4 * R>), 4 * R);
+}
+
+// A space for a merged sort, held until its owner is done with it.
+inline void* radix_merge_space(std::unique_lock<std::mutex>& lock) {
   RadixMergeSpace* space = radix_merge_spaces();
   for (int q = 0; q < kRadixMergeSpaces && !lock.owns_lock(); ++q) {
     space = radix_merge_spaces() + q;
@@ -1032,14 +1054,7 @@ void radix_sort_merged(const MI355X& exec, typename RadixKey<T>::U* k0, int n, P
     }
     KKMX_SAFE_CALL(mx_malloc(&space->buf, kRadixMergeBytes, nullptr));
   }
-  U* k1  = static_cast<U*>(space->buf);
-  PT* p1 = pairs ? reinterpret_cast<PT*>(static_cast<char*>(space->buf) + kRadixMergeBytes / 2) : nullptr;
-  mx_launch_kernel(reinterpret_cast<const void*>(&k_radix_small<T, PT, Iota, Items, false>), unsigned((n + run - 1) / run),
-                   kRadixSmallLanes, 0, exec.stream(), k0, payload, n, k1, p1);
-  mx_launch_kernel(reinterpret_cast<const void*>(&k_radix_merge<T, PT, run>), unsigned((n + 63) / 64),
-                   64 * kRadixMergeWaves, 0, exec.stream(), k1, p1, n, k0, payload);
-  // the space is free for the next call once the stream has run these
-  exec.fence("Kokkos::sort: merged runs");
+  return space->buf;
 }
 
 // Ascending LSD radix sort of n keys in place (device memory), on exec.
@@ -1056,18 +1071,11 @@ void radix_sort(const MI355X& exec, T* keys, int64_t n, PT* payload = nullptr) {
   if (n < 1 || (n < 2 && !Iota)) return;
   using U = typename RadixKey<T>::U;
   U* k0   = reinterpret_cast<U*>(keys);
-  if (n <= kRadixSmallLanes * kRadixSmallItems<U>) {
-    int count  = int(n);
-    U* no_out  = nullptr;
-    PT* no_pay = nullptr;
-    mx_launch_kernel(reinterpret_cast<const void*>(&k_radix_small<T, PT, Iota, kRadixSmallItems<U>, true>), 1,
-                     kRadixSmallLanes, 0, exec.stream(), k0, payload, count, no_out, no_pay);
-    exec.fence("Kokkos::sort: keys of one block");
-    return;
-  }
   if (n <= kRadixMerged) {
-    if (n <= kRadixMergeRuns * kRadixSmallLanes) radix_sort_merged<T, PT, Iota, 1>(exec, k0, int(n), payload);
-    else radix_sort_merged<T, PT, Iota, 4>(exec, k0, int(n), payload);
+    std::unique_lock<std::mutex> lock;
+    void* space = n <= kRadixSmallLanes * kRadixSmallItems<U> ? nullptr : radix_merge_space(lock);
+    radix_sort_few<T, PT, Iota>(exec, k0, int(n), payload, space);
+    exec.fence("Kokkos::sort: few keys");
     return;
   }
   if (n >= kRadixLarge) radix_sort_passes<T, PT, Iota, RadixShape<T, PT, true>>(exec, k0, n, payload);

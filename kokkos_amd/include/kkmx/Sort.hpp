@@ -220,38 +220,52 @@ struct BinRunSortF {
   }
   static constexpr int kRunLanes = 1 << 16;
 };
-// First position of each bin: the first sorted code that is not below it.
+// Each bin's first position, that of the first sorted code that is not below
+// it, and its count, from the next bin's, by two searches side by side.  Bin 0
+// hands the flags to the host and clears them for the next call.
 struct BinStartF {
   const uint32_t* code;
-  View<int*, MI355XSpace, MemoryTraits<Unmanaged>> offsets;
-  int n, frac;
+  View<int*, MI355XSpace, MemoryTraits<Unmanaged>> offsets, count;
+  int n, frac, bins;
+  uint32_t* flags;
+  uint32_t* host;
   KOKKOS_INLINE_FUNCTION void operator()(const int b) const {
-    const uint32_t want = uint32_t(b) << frac;
-    int lo = 0, hi = n;
-    while (lo < hi) {
-      const int mid = lo + (hi - lo) / 2;
-      if (code[mid] < want) lo = mid + 1;
-      else hi = mid;
+    const uint32_t want = uint32_t(b) << frac, next = uint32_t(b + 1) << frac;
+    int lo = 0, hi = n, lo1 = 0, hi1 = n;
+    while (lo < hi || lo1 < hi1) {
+      const int mid = lo + (hi - lo) / 2, mid1 = lo1 + (hi1 - lo1) / 2;
+      const uint32_t c = code[mid < n ? mid : n - 1], c1 = code[mid1 < n ? mid1 : n - 1];
+      if (lo < hi) (c < want ? lo : hi) = c < want ? mid + 1 : mid;
+      if (lo1 < hi1) (c1 < next ? lo1 : hi1) = c1 < next ? mid1 + 1 : mid1;
     }
     offsets(b) = lo;
+    count(b)   = (b + 1 < bins ? lo1 : n) - lo;  // the last bin's next may not fit 32 bits
+    if (b == 0) {
+      for (int k = 1; k < 3; ++k) host[k] = flags[k];
+      for (int k = 0; k < 3; ++k) flags[k] = 0;
+    }
   }
 };
-struct BinExtentF {
-  View<const int*, MI355XSpace, MemoryTraits<Unmanaged>> offsets;
-  View<int*, MI355XSpace, MemoryTraits<Unmanaged>> count;
-  int n, bins;
-  KOKKOS_INLINE_FUNCTION void operator()(const int b) const {
-    count(b) = (b + 1 < bins ? offsets(b + 1) : n) - offsets(b);
+struct BinZeroF {
+  View<int*, MI355XSpace, MemoryTraits<Unmanaged>> order, count, offsets;
+  KOKKOS_INLINE_FUNCTION void operator()(const size_t i) const {
+    if (i < order.extent(0)) order(i) = 0;
+    if (i < count.extent(0)) count(i) = offsets(i) = 0;
   }
 };
 
 // Device scratch of BinSort, kept between calls and grown on demand: held by
 // its mutex until the stream has run what uses it; freed by Kokkos::finalize.
+// `flags` are the ordering's, all zero between calls unless one was cut off by
+// an error (clear is false then), `host` its pinned copy.
 struct BinWorkspace {
   std::mutex mtx;
-  void* buf    = nullptr;
-  size_t bytes = 0;
-  bool hooked  = false;
+  void* buf       = nullptr;
+  size_t bytes    = 0;
+  bool hooked     = false;
+  void* flags     = nullptr;
+  uint32_t* host  = nullptr;
+  bool clear      = false;
   void* space(size_t need);
 };
 inline BinWorkspace& bin_workspace() {
@@ -262,8 +276,13 @@ inline void bin_workspace_release() {
   BinWorkspace& w = bin_workspace();
   std::lock_guard<std::mutex> lock(w.mtx);
   if (w.buf) KKMX_SAFE_CALL(mx_free(w.buf, nullptr));
+  if (w.flags) KKMX_SAFE_CALL(mx_free(w.flags, nullptr));
+  if (w.host) KKMX_SAFE_CALL(mx_host_free(w.host));
   w.buf    = nullptr;
+  w.flags  = nullptr;
+  w.host   = nullptr;
   w.bytes  = 0;
+  w.clear  = false;
   w.hooked = false;
 }
 inline void* BinWorkspace::space(size_t need) {
@@ -295,30 +314,36 @@ bool bin_order_by_code(const MI355X& exec, const Keys& keys, const Op& op, int b
   while (frac > 0 && (uint64_t(bins) << frac) > (uint64_t(1) << 32)) --frac;
   BinWorkspace& ws = bin_workspace();
   std::lock_guard<std::mutex> lock(ws.mtx);
+  const bool few          = len <= kRadixMerged;
   const size_t code_bytes = radix_round(size_t(len) * 4);
-  char* base              = static_cast<char*>(ws.space(2 * code_bytes + 256));
+  char* base              = static_cast<char*>(ws.space(2 * code_bytes + (few ? kRadixMergeBytes : 0)));
   uint32_t* code          = reinterpret_cast<uint32_t*>(base);
   uint32_t* runs          = reinterpret_cast<uint32_t*>(base + code_bytes);
-  uint32_t* flags         = reinterpret_cast<uint32_t*>(base + 2 * code_bytes);
   uint32_t* perm          = reinterpret_cast<uint32_t*>(order);
-  clear_words_async(flags, 16, exec.stream());
+  if (!ws.flags) KKMX_SAFE_CALL(mx_malloc(&ws.flags, 64, nullptr));
+  if (!ws.host) {
+    void* h = nullptr;
+    KKMX_SAFE_CALL(mx_host_alloc(&h, 64));
+    ws.host = static_cast<uint32_t*>(h);
+  }
+  uint32_t* flags = static_cast<uint32_t*>(ws.flags);
+  if (!ws.clear) clear_words_async(flags, 16, exec.stream());
+  ws.clear = false;
   parallel_for("Kokkos::Sort::BinQuantise", RangePolicy<MI355X>(exec, 0, len),
                BinQuantiseF<Keys>{keys, op.mul_, op.min_, double(uint64_t(1) << frac), double(bins), code, flags, begin});
-  radix_sort<uint32_t, uint32_t, true>(exec, code, int64_t(len), perm);
+  if (few) radix_sort_few<uint32_t, uint32_t, true>(exec, code, len, perm, base + 2 * code_bytes);
+  else radix_sort<uint32_t, uint32_t, true>(exec, code, int64_t(len), perm);
   parallel_for("Kokkos::Sort::BinRuns", RangePolicy<MI355X>(exec, 0, len),
                BinRunsF<Keys>{keys, code, perm, flags, runs, begin, len});
   const int lanes = len < BinRunSortF<Keys>::kRunLanes ? len : BinRunSortF<Keys>::kRunLanes;
   parallel_for("Kokkos::Sort::BinRunSort", RangePolicy<MI355X>(exec, 0, lanes),
                BinRunSortF<Keys>{keys, code, perm, flags, runs, begin, len});
-  using U  = View<int*, MI355XSpace, MemoryTraits<Unmanaged>>;
-  using CU = View<const int*, MI355XSpace, MemoryTraits<Unmanaged>>;
+  using U = View<int*, MI355XSpace, MemoryTraits<Unmanaged>>;
   parallel_for("Kokkos::Sort::BinStart", RangePolicy<MI355X>(exec, 0, bins),
-               BinStartF{code, U(offsets, size_t(bins)), len, frac});
-  parallel_for("Kokkos::Sort::BinExtent", RangePolicy<MI355X>(exec, 0, bins),
-               BinExtentF{CU(offsets, size_t(bins)), U(count, size_t(bins)), len, bins});
-  uint32_t got[4] = {0, 0, 0, 0};
-  KKMX_SAFE_CALL(mx_memcpy_async(got, flags, sizeof(got), exec.stream()));
+               BinStartF{code, U(offsets, size_t(bins)), U(count, size_t(bins)), len, frac, bins, flags, ws.host});
   exec.fence("Kokkos::BinSort: keys in order");
+  ws.clear                     = true;
+  const volatile uint32_t* got = ws.host;
   if (got[1]) return false;
   if (got[2]) {
     View<T*, MI355XSpace> copy(view_alloc(WithoutInitializing, std::string("Kokkos::BinSort::key_copy")), size_t(len));
@@ -446,10 +471,15 @@ class BinSort {
         sort_within_bins(sort_within_bins_) {
     static_assert(std::is_same<ExecutionSpace, MI355X>::value, "BinSort runs on the MI355X execution space");
     if (range_begin > range_end) Kokkos::abort("BinSort: range_begin > range_end");
-    sort_order  = offset_type("Kokkos::BinSort::sort_order", size_t(range_end - range_begin));
-    bin_count   = View<int*, MI355XSpace>("Kokkos::BinSort::bin_count", size_t(bin_op.max_bins()));
-    bin_offsets = offset_type("Kokkos::BinSort::bin_offsets", size_t(bin_op.max_bins()));
-    (void)exec;
+    const size_t len = size_t(range_end - range_begin), bins = size_t(bin_op.max_bins());
+    sort_order  = offset_type(view_alloc(WithoutInitializing, std::string("Kokkos::BinSort::sort_order")), len);
+    bin_count   = View<int*, MI355XSpace>(view_alloc(WithoutInitializing, std::string("Kokkos::BinSort::bin_count")), bins);
+    bin_offsets = offset_type(view_alloc(WithoutInitializing, std::string("Kokkos::BinSort::bin_offsets")), bins);
+    // one launch and one wait for all three
+    using U = View<int*, MI355XSpace, MemoryTraits<Unmanaged>>;
+    parallel_for("Kokkos::Sort::BinZero", RangePolicy<MI355X, IndexType<size_t>>(exec, 0, len > bins ? len : bins),
+                 Impl::BinZeroF{U(sort_order.data(), len), U(bin_count.data(), bins), U(bin_offsets.data(), bins)});
+    exec.fence("Kokkos::BinSort: Views set to zero");
   }
   BinSort(const_key_view_type keys_, int range_begin_, int range_end_, BinSortOp bin_op_, bool sort_within_bins_ = false)
       : BinSort(exec_space{}, keys_, range_begin_, range_end_, bin_op_, sort_within_bins_) {}

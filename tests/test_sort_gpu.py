@@ -97,6 +97,24 @@ def test_binsort_within_bins_forms(paths, oracle, n, form):
     assert np.array_equal(Vd.download(np.int64, n), vals[ref])
 
 
+@pytest.mark.parametrize("nbins", [1, 3, 5000, 1 << 20])
+@pytest.mark.parametrize("n", [2, 4096, 4097, 24 * 1024 + 1, 24 * 4096, 24 * 4096 + 1])
+def test_binsort_sizes(paths, oracle, n, nbins):
+    """Either side of the codes' sorts, each size right after a call that met a
+    key in no bin."""
+    P = paths
+    for form in ("outside", "any"):
+        keys = np.floor(oracle.fill_uniform_f64(n, 84, 0.0, 1.0) * 30000.0) / 30000.0
+        if form == "outside":
+            keys[0] = np.nan
+        vals = np.arange(n, dtype=np.int64) * 3
+        Kd, Vd, Pd = K.DeviceBuffer.from_array(keys), K.DeviceBuffer.from_array(vals), K.DeviceBuffer(n * 4)
+        run(P, P.kkmx_binsort_f64(Kd.ptr, Vd.ptr, n, nbins, 0.0, 1.0, 1, Pd.ptr))
+        ref = np.argsort(keys, kind="stable")
+        assert np.array_equal(Pd.download(np.int32, n), ref)
+        assert np.array_equal(Vd.download(np.int64, n), vals[ref])
+
+
 def test_binsort_without_bin_sort_is_bin_monotone(paths, oracle):
     P = paths
     n, nbins = 1 << 18, 1000
