@@ -456,6 +456,7 @@ __global__ __launch_bounds__(Lanes, 4) void k_radix_scatter(
 // into an LDS hash table by their trimmed digits, and different keys that meet
 // there are counted.  If all of n keys lie in runs of 64, which is more than
 // k_radix_finish takes, 4096^2 / 2 * 64 / n meet: 8 at n = 2^26, more below.
+// One block, bound by its loads' latency.
 constexpr int kRadixSample = 4096;
 template <class T>
 __global__ __launch_bounds__(1024) void k_radix_sample(const typename RadixKey<T>::U* in, const int64_t n,
@@ -868,8 +869,8 @@ inline size_t radix_round(size_t bytes) { return (bytes + 255) & ~size_t(255); }
 // Tile and resident blocks per CU of the scatter.  From kRadixLarge keys on,
 // larger tiles make longer runs per digit: int32 keys, 2^28 of them, take
 // 0.78 ms a pass with 8192-key tiles, 0.86 with 6144, 1.1 with 4096; (int64,
-// 8-byte value) pairs, 3 M of them, 281 us a sort with 6144-key tiles, 303 with
-// 4096 and 474 with 8192, which no longer fit two blocks' registers.  Below,
+// 8-byte value) pairs, 3 M of them, 281 us all eight passes with 6144-key tiles, 303
+// with 4096 and 474 with 8192, which no longer fit two blocks' registers.  Below,
 // smaller tiles reach more CUs: 10^6 float64 keys take 159 us with 4096-key
 // tiles, 172 with 6144, 186 with 8192.
 template <class T, class PT, bool Large>

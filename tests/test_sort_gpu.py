@@ -148,10 +148,9 @@ def test_sort_by_key_is_stable(paths, oracle, code, n, vbytes):
     assert np.array_equal(Dv.download(vdt, n), vals[order])
 
 
-# Edges of the radix sort's forms: rounds of the one-block sort and its limit
-# (8192 keys), one tile more than a block's (4096), the last size whose
-# segments add up their counts themselves and the first that does not (48
-# tiles of 4096), several tiles per segment with a ragged last one, and both
+# Edges of the radix sort's forms: rounds of a block's sort, runs with a ragged
+# last one, the last size of the passes whose segments add up their counts
+# themselves and the first that does not (48 tiles of 4096), several tiles per segment with a ragged last one, and both
 # sides of the switch to larger tiles (2^21 keys).
 @pytest.mark.parametrize("n", [1023, 1025, 8191, 8192, 8193, 12289, 48 * 4096, 48 * 4096 + 1, 1024 * 4096 + 5,
                                (1 << 21) - 1, 1 << 21, 3000017])
