@@ -9,16 +9,15 @@
 //  * Allocation is stream ordered (hipMallocAsync) when a stream is given, like
 //    the reference's HIPSpace::impl_allocate (Kokkos_HIP_Space.cpp:92-131).
 //  * Blocks of device memory that are freed without a stream are kept for the
-//    next allocation of about their size (BlockCache below).
+//    next allocation of about their size (block_cache.hpp).
 //  * Streams keep the default priority.
 #include <hip/hip_runtime.h>
 
 #include <cstdio>
 #include <cstring>
-#include <map>
 #include <mutex>
-#include <unordered_map>
 
+#include "block_cache.hpp"
 #include "kkmx_runtime.h"
 
 namespace {
@@ -38,82 +37,14 @@ RuntimeState& state() {
 
 inline int rc(hipError_t e) { return static_cast<int>(e); }
 
-// Device blocks allocated without a stream (Views, workspaces, buffers of C
-// callers).  hipMalloc and hipFree map and unmap the block's pages: a BinSort
-// of 2^24 keys, which makes and releases Views of 64, 4 and 4 MiB, takes 1.97
-// ms with them and 1.40 without.  A freed block is therefore kept, up to
-// kIdleBytes in all and kBlockBytes each, and handed out again for a request
-// of 80-100 % of its size.
-//  * mx_free without a stream keeps hipFree's meaning: it returns when the
-//    device has run everything queued before it, on any stream, so a kept
-//    block is idle whoever takes it next.
-//  * Kept blocks go back to the device when an allocation fails, by mx_trim
-//    (Kokkos::finalize calls it) and at mx_finalize.
-//  * A thread that is recording a stream goes to hipFree as before: waiting
-//    for the device is not allowed there.
-struct BlockCache {
-  static constexpr size_t kBlockBytes = size_t(256) << 20;
-  static constexpr size_t kIdleBytes  = size_t(512) << 20;
-  std::mutex mtx;
-  std::unordered_map<void*, size_t> live;
-  std::multimap<size_t, void*> idle;
-  size_t idle_bytes = 0;
-
-  static size_t rounded(size_t n) {
-    const size_t unit = n <= (size_t(1) << 20) ? size_t(4) << 10 : size_t(64) << 10;
-    return (n + unit - 1) / unit * unit;
-  }
-  // with mtx held
-  void release_idle() {
-    for (auto& b : idle) (void)hipFree(b.second);
-    idle.clear();
-    idle_bytes = 0;
-  }
-  hipError_t take(void** ptr, size_t bytes) {
-    const size_t want = rounded(bytes);
-    std::lock_guard<std::mutex> lk(mtx);
-    auto it = idle.lower_bound(want);
-    if (it != idle.end() && it->first <= want + want / 4) {
-      *ptr       = it->second;
-      live[*ptr] = it->first;
-      idle_bytes -= it->first;
-      idle.erase(it);
-      return hipSuccess;
-    }
-    hipError_t e = hipMalloc(ptr, want);
-    if (e != hipSuccess && !idle.empty()) {
-      (void)hipGetLastError();
-      release_idle();
-      e = hipMalloc(ptr, want);
-    }
-    if (e == hipSuccess) live[*ptr] = want;
-    else *ptr = nullptr;
-    return e;
-  }
-  hipError_t give(void* ptr, bool recording) {
-    size_t bytes = 0;
-    {
-      std::lock_guard<std::mutex> lk(mtx);
-      auto it = live.find(ptr);
-      if (it != live.end()) {
-        bytes = it->second;
-        live.erase(it);
-      }
-    }
-    if (bytes == 0 || bytes > kBlockBytes || recording) return hipFree(ptr);
-    if (hipDeviceSynchronize() != hipSuccess) {
-      (void)hipGetLastError();
-      return hipFree(ptr);
-    }
-    std::lock_guard<std::mutex> lk(mtx);
-    if (idle_bytes + bytes > kIdleBytes) return hipFree(ptr);
-    idle.emplace(bytes, ptr);
-    idle_bytes += bytes;
-    return hipSuccess;
-  }
+struct HipBlocks {
+  static int alloc(void** ptr, size_t bytes) { return rc(hipMalloc(ptr, bytes)); }
+  static int free(void* ptr) { return rc(hipFree(ptr)); }
+  static int sync() { return rc(hipDeviceSynchronize()); }
+  static void clear_error() { (void)hipGetLastError(); }
 };
-BlockCache& blocks() {
-  static BlockCache* c = new BlockCache;  // outlives every static that frees a block
+BlockCache<HipBlocks>& blocks() {
+  static BlockCache<HipBlocks>* c = new BlockCache<HipBlocks>;  // outlives every static that frees a block
   return *c;
 }
 thread_local int g_recording = 0;
@@ -177,11 +108,7 @@ int mx_finalize(void) {
   std::lock_guard<std::mutex> lk(s.mtx);
   if (!s.initialized) return 0;
   hipError_t e = hipStreamSynchronize(s.stream);
-  {
-    BlockCache& c = blocks();
-    std::lock_guard<std::mutex> cl(c.mtx);
-    c.release_idle();
-  }
+  blocks().trim();
   hipError_t e2 = hipStreamDestroy(s.stream);
   s.stream      = nullptr;
   s.initialized = false;
@@ -211,19 +138,17 @@ int mx_malloc(void** ptr, size_t bytes, mx_stream_t stream) {
   if (bytes == 0) return 0;
   if (stream)
     return rc(hipMallocAsync(ptr, bytes, static_cast<hipStream_t>(stream)));
-  return rc(blocks().take(ptr, bytes));
+  return blocks().take(ptr, bytes);
 }
 
 int mx_free(void* ptr, mx_stream_t stream) {
   if (!ptr) return 0;
   if (stream) return rc(hipFreeAsync(ptr, static_cast<hipStream_t>(stream)));
-  return rc(blocks().give(ptr, g_recording > 0));
+  return blocks().give(ptr, g_recording > 0);
 }
 
 int mx_trim(void) {
-  BlockCache& c = blocks();
-  std::lock_guard<std::mutex> lk(c.mtx);
-  c.release_idle();
+  blocks().trim();
   return 0;
 }
 
