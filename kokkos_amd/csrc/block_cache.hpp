@@ -5,15 +5,18 @@
 // kIdleBytes in all and kBlockBytes each, and handed out again for a request
 // of 80-100 % of its size.
 //  * mx_free without a stream keeps hipFree's meaning: it returns when the
-//    device has run everything queued before it, on any stream, so a kept
-//    block is idle whoever takes it next.
+//    block's device has run everything queued before it, on any stream, so a
+//    kept block is idle whoever takes it next.  That device need not be the
+//    freeing thread's own: a thread starts on device 0, whichever mx_init chose.
+//  * A block is handed out only to threads on its device.
 //  * Kept blocks go back to the device when an allocation fails, by mx_trim
 //    (Kokkos::finalize calls it) and at mx_finalize.
 //  * A thread that is recording a stream goes to hipFree as before: waiting
 //    for the device is not allowed there.
 //
 // Api stands for the HIP calls, as static functions that return 0 or an error:
-//   alloc(ptr*, bytes), free(ptr), sync(), clear_error()
+//   alloc(ptr*, bytes), free(ptr), device(id*), set_device(id), sync(), clear_error()
+// alloc, sync and set_device are about the calling thread's device.
 #ifndef KKMX_BLOCK_CACHE_HPP
 #define KKMX_BLOCK_CACHE_HPP
 
@@ -27,8 +30,13 @@ struct BlockCache {
   static constexpr size_t kBlockBytes = size_t(256) << 20;
   static constexpr size_t kIdleBytes  = size_t(512) << 20;
   std::mutex mtx;
-  std::unordered_map<void*, size_t> live;
-  std::multimap<size_t, void*> idle;
+  struct Block {
+    int device;
+    size_t bytes;
+    bool operator<(const Block& o) const { return device != o.device ? device < o.device : bytes < o.bytes; }
+  };
+  std::unordered_map<void*, Block> live;
+  std::multimap<Block, void*> idle;
   size_t idle_bytes = 0;
 
   // Sizes that would wrap stay as they are, for the allocation to refuse.
@@ -47,13 +55,16 @@ struct BlockCache {
     release_idle();
   }
   int take(void** ptr, size_t bytes) {
+    *ptr              = nullptr;
     const size_t want = rounded(bytes);
+    int device        = 0;
+    if (const int e = Api::device(&device)) return e;
     std::lock_guard<std::mutex> lk(mtx);
-    auto it = idle.lower_bound(want);
-    if (it != idle.end() && it->first <= want + want / 4) {
+    auto it = idle.lower_bound({device, want});
+    if (it != idle.end() && it->first.device == device && it->first.bytes <= want + want / 4) {
       *ptr       = it->second;
       live[*ptr] = it->first;
-      idle_bytes -= it->first;
+      idle_bytes -= it->first.bytes;
       idle.erase(it);
       return 0;
     }
@@ -63,29 +74,39 @@ struct BlockCache {
       release_idle();
       e = Api::alloc(ptr, want);
     }
-    if (e == 0) live[*ptr] = want;
+    if (e == 0) live[*ptr] = {device, want};
     else *ptr = nullptr;
     return e;
   }
+  // Waits for `device`, from a thread on any device.
+  static int wait_for(int device) {
+    int mine = 0;
+    if (const int e = Api::device(&mine)) return e;
+    if (mine == device) return Api::sync();
+    if (const int e = Api::set_device(device)) return e;
+    const int e = Api::sync();
+    (void)Api::set_device(mine);
+    return e;
+  }
   int give(void* ptr, bool recording) {
-    size_t bytes = 0;
+    Block b{0, 0};
     {
       std::lock_guard<std::mutex> lk(mtx);
       auto it = live.find(ptr);
       if (it != live.end()) {
-        bytes = it->second;
+        b = it->second;
         live.erase(it);
       }
     }
-    if (bytes == 0 || bytes > kBlockBytes || recording) return Api::free(ptr);
-    if (Api::sync() != 0) {
+    if (b.bytes == 0 || b.bytes > kBlockBytes || recording) return Api::free(ptr);
+    if (wait_for(b.device) != 0) {
       Api::clear_error();
       return Api::free(ptr);
     }
     std::lock_guard<std::mutex> lk(mtx);
-    if (idle_bytes + bytes > kIdleBytes) return Api::free(ptr);
-    idle.emplace(bytes, ptr);
-    idle_bytes += bytes;
+    if (idle_bytes + b.bytes > kIdleBytes) return Api::free(ptr);
+    idle.emplace(b, ptr);
+    idle_bytes += b.bytes;
     return 0;
   }
 };

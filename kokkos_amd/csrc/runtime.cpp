@@ -40,6 +40,8 @@ inline int rc(hipError_t e) { return static_cast<int>(e); }
 struct HipBlocks {
   static int alloc(void** ptr, size_t bytes) { return rc(hipMalloc(ptr, bytes)); }
   static int free(void* ptr) { return rc(hipFree(ptr)); }
+  static int device(int* id) { return rc(hipGetDevice(id)); }
+  static int set_device(int id) { return rc(hipSetDevice(id)); }
   static int sync() { return rc(hipDeviceSynchronize()); }
   static void clear_error() { (void)hipGetLastError(); }
 };

@@ -4,6 +4,7 @@
 #include <cstdio>
 #include <cstring>
 #include <map>
+#include <thread>
 
 #include "block_cache.hpp"
 
@@ -19,18 +20,25 @@ constexpr size_t MiB = size_t(1) << 20;
 constexpr int kInvalid = 1, kNoMemory = 2;
 
 // Addresses without memory behind them; like hipMalloc, nothing for 0 bytes.
+// pending[d]: whether device d has queued work that may use any block.
 struct Model {
-  static inline std::map<void*, size_t> allocated;
-  static inline uintptr_t next    = 1 << 20;
-  static inline size_t capacity   = size_t(64) << 30, used = 0;
+  struct Alloc {
+    size_t bytes;
+    int device;
+  };
+  static inline std::map<void*, Alloc> allocated;
+  static inline uintptr_t next  = 1 << 20;
+  static inline size_t capacity = size_t(64) << 30, used = 0;
   static inline int allocs = 0, frees = 0;
+  static inline bool pending[2] = {};
+  static inline thread_local int current = 0;
   static int alloc(void** ptr, size_t bytes) {
     *ptr = nullptr;
     if (bytes == 0) return 0;
     if (bytes > capacity - used) return kNoMemory;
     *ptr = reinterpret_cast<void*>(next);
     next += (bytes + MiB) / MiB * MiB;
-    allocated[*ptr] = bytes;
+    allocated[*ptr] = {bytes, current};
     used += bytes;
     ++allocs;
     return 0;
@@ -38,12 +46,24 @@ struct Model {
   static int free(void* ptr) {
     auto it = allocated.find(ptr);
     if (it == allocated.end()) return kInvalid;
-    used -= it->second;
+    pending[it->second.device] = false;
+    used -= it->second.bytes;
     allocated.erase(it);
     ++frees;
     return 0;
   }
-  static int sync() { return 0; }
+  static int device(int* id) {
+    *id = current;
+    return 0;
+  }
+  static int set_device(int id) {
+    current = id;
+    return 0;
+  }
+  static int sync() {
+    pending[current] = false;
+    return 0;
+  }
   static void clear_error() {}
 };
 using Cache = BlockCache<Model>;
@@ -64,11 +84,35 @@ int huge_requests() {
   return 0;
 }
 
+// A free waits for the block's device from a thread on another one, and the
+// block goes to threads on its device only.
+int devices() {
+  Cache c;
+  void *p = nullptr, *q = nullptr, *r = nullptr;
+  Model::current = 1;
+  CHECK(c.take(&p, MiB) == 0);
+  Model::pending[0] = Model::pending[1] = true;
+  int rc = -1, device = -1;
+  std::thread([&] {
+    rc     = c.give(p, false);
+    device = Model::current;
+  }).join();
+  CHECK(rc == 0 && device == 0);
+  CHECK(!Model::pending[1]);
+  Model::current = 0;
+  CHECK(c.take(&q, MiB) == 0);
+  CHECK(q != p);
+  Model::current = 1;
+  CHECK(c.take(&r, MiB) == 0);
+  CHECK(r == p);
+  return 0;
+}
+
 int main(int argc, char** argv) {
   const struct {
     const char* name;
     int (*run)();
-  } checks[] = {{"huge_requests", huge_requests}};
+  } checks[] = {{"huge_requests", huge_requests}, {"devices", devices}};
   for (const auto& c : checks)
     if (argc > 1 && !std::strcmp(argv[1], c.name)) return c.run();
   std::printf("no such check\n");
