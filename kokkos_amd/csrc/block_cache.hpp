@@ -8,15 +8,18 @@
 //    block's device has run everything queued before it, on any stream, so a
 //    kept block is idle whoever takes it next.  That device need not be the
 //    freeing thread's own: a thread starts on device 0, whichever mx_init chose.
+//    The wait is that of a hipFree, of a page on the block's device (1.3 us when
+//    it is idle): hipDeviceSynchronize would invalidate a stream capture that
+//    another thread is in, which freeing memory there does not.
 //  * A block is handed out only to threads on its device.
 //  * Kept blocks go back to the device when an allocation fails, by mx_trim
 //    (Kokkos::finalize calls it) and at mx_finalize.
-//  * A thread that is recording a stream goes to hipFree as before: waiting
-//    for the device is not allowed there.
+//  * A thread that is recording a stream gets what hipFree answers there.
 //
 // Api stands for the HIP calls, as static functions that return 0 or an error:
-//   alloc(ptr*, bytes), free(ptr), device(id*), set_device(id), sync(), clear_error()
-// alloc, sync and set_device are about the calling thread's device.
+//   alloc(ptr*, bytes), free(ptr), device(id*), set_device(id), clear_error()
+// alloc and set_device are about the calling thread's device; free waits for the
+// device of ptr.
 #ifndef KKMX_BLOCK_CACHE_HPP
 #define KKMX_BLOCK_CACHE_HPP
 
@@ -82,13 +85,14 @@ struct BlockCache {
   static int wait_for(int device) {
     int mine = 0;
     if (const int e = Api::device(&mine)) return e;
-    if (mine == device) return Api::sync();
-    if (const int e = Api::set_device(device)) return e;
-    const int e = Api::sync();
-    (void)Api::set_device(mine);
-    return e;
+    if (mine != device)
+      if (const int e = Api::set_device(device)) return e;
+    void* page  = nullptr;
+    const int e = Api::alloc(&page, 4096);
+    if (mine != device) (void)Api::set_device(mine);
+    return e ? e : Api::free(page);
   }
-  int give(void* ptr, bool recording) {
+  int give(void* ptr) {
     Block b{0, 0};
     {
       std::lock_guard<std::mutex> lk(mtx);
@@ -98,7 +102,7 @@ struct BlockCache {
         live.erase(it);
       }
     }
-    if (b.bytes == 0 || b.bytes > kBlockBytes || recording) return Api::free(ptr);
+    if (b.bytes == 0 || b.bytes > kBlockBytes) return Api::free(ptr);
     if (wait_for(b.device) != 0) {
       Api::clear_error();
       return Api::free(ptr);

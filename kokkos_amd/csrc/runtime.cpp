@@ -42,14 +42,12 @@ struct HipBlocks {
   static int free(void* ptr) { return rc(hipFree(ptr)); }
   static int device(int* id) { return rc(hipGetDevice(id)); }
   static int set_device(int id) { return rc(hipSetDevice(id)); }
-  static int sync() { return rc(hipDeviceSynchronize()); }
   static void clear_error() { (void)hipGetLastError(); }
 };
 BlockCache<HipBlocks>& blocks() {
   static BlockCache<HipBlocks>* c = new BlockCache<HipBlocks>;  // outlives every static that frees a block
   return *c;
 }
-thread_local int g_recording = 0;
 
 }  // namespace
 
@@ -146,7 +144,7 @@ int mx_malloc(void** ptr, size_t bytes, mx_stream_t stream) {
 int mx_free(void* ptr, mx_stream_t stream) {
   if (!ptr) return 0;
   if (stream) return rc(hipFreeAsync(ptr, static_cast<hipStream_t>(stream)));
-  return blocks().give(ptr, g_recording > 0);
+  return blocks().give(ptr);
 }
 
 int mx_trim(void) {
@@ -294,16 +292,13 @@ int mx_occupancy(const void* fn, int block_size, size_t dyn_lds_bytes,
 int mx_get_last_error(void) { return rc(hipGetLastError()); }
 
 int mx_graph_capture_begin(mx_stream_t stream) {
-  const hipError_t e = hipStreamBeginCapture(static_cast<hipStream_t>(stream),
-                                             hipStreamCaptureModeThreadLocal);
-  if (e == hipSuccess) ++g_recording;
-  return rc(e);
+  return rc(hipStreamBeginCapture(static_cast<hipStream_t>(stream),
+                                  hipStreamCaptureModeThreadLocal));
 }
 
 int mx_graph_capture_end(mx_stream_t stream, mx_graph_t* graph) {
   hipGraph_t g = nullptr;
   hipError_t e = hipStreamEndCapture(static_cast<hipStream_t>(stream), &g);
-  if (g_recording > 0) --g_recording;
   *graph       = g;
   return rc(e);
 }

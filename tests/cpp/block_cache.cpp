@@ -17,7 +17,7 @@
   } while (0)
 
 constexpr size_t MiB = size_t(1) << 20;
-constexpr int kInvalid = 1, kNoMemory = 2;
+constexpr int kInvalid = 1, kNoMemory = 2, kUnsupported = 900;
 
 // Addresses without memory behind them; like hipMalloc, nothing for 0 bytes.
 // pending[d]: whether device d has queued work that may use any block.
@@ -32,8 +32,10 @@ struct Model {
   static inline int allocs = 0, frees = 0;
   static inline bool pending[2] = {};
   static inline thread_local int current = 0;
+  static inline thread_local bool recording = false;  // this thread records a stream
   static int alloc(void** ptr, size_t bytes) {
     *ptr = nullptr;
+    if (recording) return kUnsupported;
     if (bytes == 0) return 0;
     if (bytes > capacity - used) return kNoMemory;
     *ptr = reinterpret_cast<void*>(next);
@@ -44,6 +46,7 @@ struct Model {
     return 0;
   }
   static int free(void* ptr) {
+    if (recording) return kUnsupported;
     auto it = allocated.find(ptr);
     if (it == allocated.end()) return kInvalid;
     pending[it->second.device] = false;
@@ -58,10 +61,6 @@ struct Model {
   }
   static int set_device(int id) {
     current = id;
-    return 0;
-  }
-  static int sync() {
-    pending[current] = false;
     return 0;
   }
   static void clear_error() {}
@@ -94,7 +93,7 @@ int devices() {
   Model::pending[0] = Model::pending[1] = true;
   int rc = -1, device = -1;
   std::thread([&] {
-    rc     = c.give(p, false);
+    rc     = c.give(p);
     device = Model::current;
   }).join();
   CHECK(rc == 0 && device == 0);
@@ -108,11 +107,31 @@ int devices() {
   return 0;
 }
 
+// A thread that records a stream gets the answer of the call it stands for,
+// and the block can be freed afterwards; a recording elsewhere changes nothing
+// (the model has no call that would wait for a device by itself).
+int recording() {
+  Cache c;
+  void* p = nullptr;
+  CHECK(c.take(&p, MiB) == 0);
+  Model::recording = true;
+  CHECK(c.give(p) == kUnsupported);
+  int rc = -1;
+  std::thread([&] {
+    void* q = nullptr;
+    rc      = c.take(&q, 2 * MiB) || c.give(q);
+  }).join();
+  CHECK(rc == 0 && c.idle.size() == 1);
+  Model::recording = false;
+  CHECK(c.give(p) == 0);
+  return 0;
+}
+
 int main(int argc, char** argv) {
   const struct {
     const char* name;
     int (*run)();
-  } checks[] = {{"huge_requests", huge_requests}, {"devices", devices}};
+  } checks[] = {{"huge_requests", huge_requests}, {"devices", devices}, {"recording", recording}};
   for (const auto& c : checks)
     if (argc > 1 && !std::strcmp(argv[1], c.name)) return c.run();
   std::printf("no such check\n");
