@@ -81,6 +81,12 @@ struct BlockCache {
     else *ptr = nullptr;
     return e;
   }
+  // The block leaves by another way (a stream-ordered free): its size must not
+  // stay for another block at its address.
+  void forget(void* ptr) {
+    std::lock_guard<std::mutex> lk(mtx);
+    live.erase(ptr);
+  }
   // Waits for `device`, from a thread on any device.
   static int wait_for(int device) {
     int mine = 0;

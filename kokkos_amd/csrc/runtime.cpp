@@ -143,7 +143,10 @@ int mx_malloc(void** ptr, size_t bytes, mx_stream_t stream) {
 
 int mx_free(void* ptr, mx_stream_t stream) {
   if (!ptr) return 0;
-  if (stream) return rc(hipFreeAsync(ptr, static_cast<hipStream_t>(stream)));
+  if (stream) {
+    blocks().forget(ptr);
+    return rc(hipFreeAsync(ptr, static_cast<hipStream_t>(stream)));
+  }
   return blocks().give(ptr);
 }
 

@@ -127,11 +127,27 @@ int recording() {
   return 0;
 }
 
+// A block freed in stream order leaves no size behind for the block that the
+// stream's allocator next makes at its address.
+int freed_in_stream_order() {
+  Cache c;
+  void* p = nullptr;
+  CHECK(c.take(&p, 64 * MiB) == 0);
+  c.forget(p);
+  CHECK(Model::free(p) == 0);
+  Model::allocated[p] = {MiB, 0};  // the smaller one
+  Model::used += MiB;
+  CHECK(c.give(p) == 0);
+  CHECK(c.idle.empty() && Model::allocated.count(p) == 0);
+  return 0;
+}
+
 int main(int argc, char** argv) {
   const struct {
     const char* name;
     int (*run)();
-  } checks[] = {{"huge_requests", huge_requests}, {"devices", devices}, {"recording", recording}};
+  } checks[] = {{"huge_requests", huge_requests}, {"devices", devices}, {"recording", recording},
+                {"freed_in_stream_order", freed_in_stream_order}};
   for (const auto& c : checks)
     if (argc > 1 && !std::strcmp(argv[1], c.name)) return c.run();
   std::printf("no such check\n");
