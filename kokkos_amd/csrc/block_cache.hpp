@@ -18,6 +18,7 @@
 //
 // Api stands for the HIP calls, as static functions that return 0 or an error:
 //   alloc(ptr*, bytes), free(ptr), device(id*), set_device(id), clear_error()
+// and the error kInvalid of an argument that cannot be.
 // alloc and set_device are about the calling thread's device; free waits for the
 // device of ptr.
 #ifndef KKMX_BLOCK_CACHE_HPP
@@ -38,7 +39,10 @@ struct BlockCache {
     size_t bytes;
     bool operator<(const Block& o) const { return device != o.device ? device < o.device : bytes < o.bytes; }
   };
-  std::unordered_map<void*, Block> live;
+  struct State : Block {
+    bool freed;  // by the caller: kept, or on the way there
+  };
+  std::unordered_map<void*, State> blocks;  // the callers' and the kept ones
   std::multimap<Block, void*> idle;
   size_t idle_bytes = 0;
 
@@ -49,7 +53,10 @@ struct BlockCache {
   }
   // with mtx held
   void release_idle() {
-    for (auto& b : idle) (void)Api::free(b.second);
+    for (auto& b : idle) {
+      blocks.erase(b.second);
+      (void)Api::free(b.second);
+    }
     idle.clear();
     idle_bytes = 0;
   }
@@ -65,8 +72,8 @@ struct BlockCache {
     std::lock_guard<std::mutex> lk(mtx);
     auto it = idle.lower_bound({device, want});
     if (it != idle.end() && it->first.device == device && it->first.bytes <= want + want / 4) {
-      *ptr       = it->second;
-      live[*ptr] = it->first;
+      *ptr         = it->second;
+      blocks[*ptr] = {it->first, false};
       idle_bytes -= it->first.bytes;
       idle.erase(it);
       return 0;
@@ -77,15 +84,19 @@ struct BlockCache {
       release_idle();
       e = Api::alloc(ptr, want);
     }
-    if (e == 0) live[*ptr] = {device, want};
+    if (e == 0) blocks[*ptr] = {{device, want}, false};
     else *ptr = nullptr;
     return e;
   }
   // The block leaves by another way (a stream-ordered free): its size must not
   // stay for another block at its address.
-  void forget(void* ptr) {
+  int forget(void* ptr) {
     std::lock_guard<std::mutex> lk(mtx);
-    live.erase(ptr);
+    auto it = blocks.find(ptr);
+    if (it == blocks.end()) return 0;
+    if (it->second.freed) return Api::kInvalid;
+    blocks.erase(it);
+    return 0;
   }
   // Waits for `device`, from a thread on any device.
   static int wait_for(int device) {
@@ -98,26 +109,32 @@ struct BlockCache {
     if (mine != device) (void)Api::set_device(mine);
     return e ? e : Api::free(page);
   }
+  // A block that is freed a second time is refused, as hipFree does.
   int give(void* ptr) {
-    Block b{0, 0};
+    State b{{0, 0}, false};
     {
       std::lock_guard<std::mutex> lk(mtx);
-      auto it = live.find(ptr);
-      if (it != live.end()) {
-        b = it->second;
-        live.erase(it);
+      auto it = blocks.find(ptr);
+      if (it != blocks.end()) {
+        if (it->second.freed) return Api::kInvalid;
+        it->second.freed = true;
+        b                = it->second;
       }
     }
-    if (b.bytes == 0 || b.bytes > kBlockBytes) return Api::free(ptr);
-    if (wait_for(b.device) != 0) {
-      Api::clear_error();
-      return Api::free(ptr);
+    if (b.bytes == 0) return Api::free(ptr);
+    const bool keep   = b.bytes <= kBlockBytes;
+    const bool waited = keep && wait_for(b.device) == 0;
+    if (keep && !waited) Api::clear_error();
+    {
+      std::lock_guard<std::mutex> lk(mtx);
+      if (waited && idle_bytes + b.bytes <= kIdleBytes) {
+        idle.emplace(b, ptr);
+        idle_bytes += b.bytes;
+        return 0;
+      }
+      blocks.erase(ptr);
     }
-    std::lock_guard<std::mutex> lk(mtx);
-    if (idle_bytes + b.bytes > kIdleBytes) return Api::free(ptr);
-    idle.emplace(b, ptr);
-    idle_bytes += b.bytes;
-    return 0;
+    return Api::free(ptr);
   }
 };
 

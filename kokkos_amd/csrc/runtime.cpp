@@ -38,6 +38,7 @@ RuntimeState& state() {
 inline int rc(hipError_t e) { return static_cast<int>(e); }
 
 struct HipBlocks {
+  static constexpr int kInvalid = static_cast<int>(hipErrorInvalidValue);
   static int alloc(void** ptr, size_t bytes) { return rc(hipMalloc(ptr, bytes)); }
   static int free(void* ptr) { return rc(hipFree(ptr)); }
   static int device(int* id) { return rc(hipGetDevice(id)); }
@@ -144,7 +145,7 @@ int mx_malloc(void** ptr, size_t bytes, mx_stream_t stream) {
 int mx_free(void* ptr, mx_stream_t stream) {
   if (!ptr) return 0;
   if (stream) {
-    blocks().forget(ptr);
+    if (const int e = blocks().forget(ptr)) return e;
     return rc(hipFreeAsync(ptr, static_cast<hipStream_t>(stream)));
   }
   return blocks().give(ptr);

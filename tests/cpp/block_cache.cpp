@@ -17,11 +17,12 @@
   } while (0)
 
 constexpr size_t MiB = size_t(1) << 20;
-constexpr int kInvalid = 1, kNoMemory = 2, kUnsupported = 900;
+constexpr int kNoMemory = 2, kUnsupported = 900;
 
 // Addresses without memory behind them; like hipMalloc, nothing for 0 bytes.
 // pending[d]: whether device d has queued work that may use any block.
 struct Model {
+  static constexpr int kInvalid = 1;
   struct Alloc {
     size_t bytes;
     int device;
@@ -142,12 +143,31 @@ int freed_in_stream_order() {
   return 0;
 }
 
+// A second free of a kept block is an error and leaves it kept, until it is
+// handed out again.
+int freed_twice() {
+  Cache c;
+  void *p = nullptr, *q = nullptr;
+  CHECK(c.take(&p, MiB) == 0);
+  CHECK(c.give(p) == 0);
+  CHECK(c.give(p) == Model::kInvalid);
+  CHECK(c.forget(p) == Model::kInvalid);
+  CHECK(Model::allocated.count(p) == 1);
+  CHECK(c.take(&q, MiB) == 0 && q == p);
+  CHECK(c.give(q) == 0);
+  c.trim();
+  CHECK(c.give(q) == Model::kInvalid);
+  CHECK(c.blocks.empty() && c.idle_bytes == 0 && Model::used == 0);
+  return 0;
+}
+
 int main(int argc, char** argv) {
   const struct {
     const char* name;
     int (*run)();
   } checks[] = {{"huge_requests", huge_requests}, {"devices", devices}, {"recording", recording},
-                {"freed_in_stream_order", freed_in_stream_order}};
+                {"freed_in_stream_order", freed_in_stream_order},
+                {"freed_twice", freed_twice}};
   for (const auto& c : checks)
     if (argc > 1 && !std::strcmp(argv[1], c.name)) return c.run();
   std::printf("no such check\n");
