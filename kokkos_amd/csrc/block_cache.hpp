@@ -12,13 +12,14 @@
 //    it is idle): hipDeviceSynchronize would invalidate a stream capture that
 //    another thread is in, which freeing memory there does not.
 //  * A block is handed out only to threads on its device.
-//  * Kept blocks go back to the device when an allocation fails, by mx_trim
-//    (Kokkos::finalize calls it) and at mx_finalize.
+//  * Kept blocks go back to the device when an allocation, also a stream-ordered
+//    one, finds no memory, by mx_trim (Kokkos::finalize calls it) and at
+//    mx_finalize.
 //  * A thread that is recording a stream gets what hipFree answers there.
 //
 // Api stands for the HIP calls, as static functions that return 0 or an error:
 //   alloc(ptr*, bytes), free(ptr), device(id*), set_device(id), clear_error()
-// and the error kInvalid of an argument that cannot be.
+// and the errors kInvalid of an argument that cannot be and kNoMemory.
 // alloc and set_device are about the calling thread's device; free waits for the
 // device of ptr.
 #ifndef KKMX_BLOCK_CACHE_HPP
@@ -51,18 +52,26 @@ struct BlockCache {
     const size_t unit = n <= (size_t(1) << 20) ? size_t(4) << 10 : size_t(64) << 10;
     return n > ~size_t(0) - unit ? n : (n + unit - 1) / unit * unit;
   }
-  // with mtx held
-  void release_idle() {
-    for (auto& b : idle) {
-      blocks.erase(b.second);
-      (void)Api::free(b.second);
+  // With mtx held.  Returns whether any block went back; one that cannot be
+  // freed now (this thread is recording) stays.
+  bool release_idle() {
+    bool any = false;
+    for (auto it = idle.begin(); it != idle.end();) {
+      if (Api::free(it->second) != 0) {
+        Api::clear_error();
+        ++it;
+        continue;
+      }
+      any = true;
+      idle_bytes -= it->first.bytes;
+      blocks.erase(it->second);
+      it = idle.erase(it);
     }
-    idle.clear();
-    idle_bytes = 0;
+    return any;
   }
-  void trim() {
+  bool trim() {
     std::lock_guard<std::mutex> lk(mtx);
-    release_idle();
+    return release_idle();
   }
   int take(void** ptr, size_t bytes) {
     *ptr              = nullptr;
@@ -79,14 +88,22 @@ struct BlockCache {
       return 0;
     }
     int e = Api::alloc(ptr, want);
-    if (e != 0 && !idle.empty()) {
+    if (e == Api::kNoMemory && !idle.empty()) {
       Api::clear_error();
-      release_idle();
-      e = Api::alloc(ptr, want);
+      if (release_idle()) e = Api::alloc(ptr, want);
     }
     if (e == 0) blocks[*ptr] = {{device, want}, false};
     else *ptr = nullptr;
     return e;
+  }
+  // An allocation that is not for the cache: `alloc` again after the kept blocks
+  // went back, where it found no memory.
+  template <class F>
+  int with_room(const F& alloc) {
+    const int e = alloc();
+    if (e != Api::kNoMemory || !trim()) return e;
+    Api::clear_error();
+    return alloc();
   }
   // The block leaves by another way (a stream-ordered free): its size must not
   // stay for another block at its address.

@@ -38,7 +38,8 @@ RuntimeState& state() {
 inline int rc(hipError_t e) { return static_cast<int>(e); }
 
 struct HipBlocks {
-  static constexpr int kInvalid = static_cast<int>(hipErrorInvalidValue);
+  static constexpr int kInvalid  = static_cast<int>(hipErrorInvalidValue);
+  static constexpr int kNoMemory = static_cast<int>(hipErrorOutOfMemory);
   static int alloc(void** ptr, size_t bytes) { return rc(hipMalloc(ptr, bytes)); }
   static int free(void* ptr) { return rc(hipFree(ptr)); }
   static int device(int* id) { return rc(hipGetDevice(id)); }
@@ -109,7 +110,7 @@ int mx_finalize(void) {
   std::lock_guard<std::mutex> lk(s.mtx);
   if (!s.initialized) return 0;
   hipError_t e = hipStreamSynchronize(s.stream);
-  blocks().trim();
+  (void)blocks().trim();
   hipError_t e2 = hipStreamDestroy(s.stream);
   s.stream      = nullptr;
   s.initialized = false;
@@ -138,7 +139,7 @@ int mx_malloc(void** ptr, size_t bytes, mx_stream_t stream) {
   *ptr = nullptr;
   if (bytes == 0) return 0;
   if (stream)
-    return rc(hipMallocAsync(ptr, bytes, static_cast<hipStream_t>(stream)));
+    return blocks().with_room([&] { return rc(hipMallocAsync(ptr, bytes, static_cast<hipStream_t>(stream))); });
   return blocks().take(ptr, bytes);
 }
 
@@ -152,7 +153,7 @@ int mx_free(void* ptr, mx_stream_t stream) {
 }
 
 int mx_trim(void) {
-  blocks().trim();
+  (void)blocks().trim();
   return 0;
 }
 

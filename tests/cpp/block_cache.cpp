@@ -17,12 +17,12 @@
   } while (0)
 
 constexpr size_t MiB = size_t(1) << 20;
-constexpr int kNoMemory = 2, kUnsupported = 900;
+constexpr int kUnsupported = 900;
 
 // Addresses without memory behind them; like hipMalloc, nothing for 0 bytes.
 // pending[d]: whether device d has queued work that may use any block.
 struct Model {
-  static constexpr int kInvalid = 1;
+  static constexpr int kInvalid = 1, kNoMemory = 2;
   struct Alloc {
     size_t bytes;
     int device;
@@ -78,7 +78,7 @@ int huge_requests() {
   Cache c;
   for (size_t n : {~size_t(0), ~size_t(0) - 42, ~size_t(0) - 65535, ~size_t(0) / 2}) {
     void* p = &c;
-    CHECK(c.take(&p, n) == kNoMemory);
+    CHECK(c.take(&p, n) == Model::kNoMemory);
     CHECK(p == nullptr);
   }
   return 0;
@@ -161,13 +161,42 @@ int freed_twice() {
   return 0;
 }
 
+// Kept blocks go back where an allocation finds no memory, one of the cache's
+// own or a stream-ordered one, and only there.
+int no_memory() {
+  Cache c;
+  void *p = nullptr, *q = nullptr;
+  Model::capacity = Model::used + 200 * MiB;
+  CHECK(c.take(&p, 150 * MiB) == 0 && c.give(p) == 0 && c.idle.size() == 1);
+  CHECK(c.take(&q, 100 * MiB) == 0);  // not of the kept block's size
+  CHECK(c.idle.empty() && c.give(q) == 0 && c.idle.size() == 1);
+  int calls       = 0;
+  const auto pool = [&] {
+    ++calls;
+    return Model::alloc(&p, 150 * MiB);
+  };
+  CHECK(c.with_room(pool) == 0 && calls == 2 && c.idle.empty());
+  q = p;
+  CHECK(c.with_room(pool) == Model::kNoMemory && calls == 3);  // nothing to give back
+  CHECK(Model::free(q) == 0);
+  // an error of another kind, and blocks that cannot be freed now: they stay
+  CHECK(c.take(&q, 100 * MiB) == 0 && c.give(q) == 0);
+  Model::recording = true;
+  CHECK(c.take(&p, 50 * MiB) == kUnsupported && c.with_room(pool) == kUnsupported);
+  CHECK(!c.trim() && c.idle.size() == 1 && c.idle_bytes == 100 * MiB);
+  Model::recording = false;
+  CHECK(c.trim() && c.idle.empty() && c.idle_bytes == 0 && Model::used == 0);
+  return 0;
+}
+
 int main(int argc, char** argv) {
   const struct {
     const char* name;
     int (*run)();
   } checks[] = {{"huge_requests", huge_requests}, {"devices", devices}, {"recording", recording},
                 {"freed_in_stream_order", freed_in_stream_order},
-                {"freed_twice", freed_twice}};
+                {"freed_twice", freed_twice},
+                {"no_memory", no_memory}};
   for (const auto& c : checks)
     if (argc > 1 && !std::strcmp(argv[1], c.name)) return c.run();
   std::printf("no such check\n");
