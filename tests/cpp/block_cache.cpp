@@ -189,6 +189,32 @@ int no_memory() {
   return 0;
 }
 
+// A kept block serves requests of 80-100 % of its size, at most 256 MiB are
+// kept of one block and 512 MiB of all, and trim gives everything back.
+int rules() {
+  Cache c;
+  void *p = nullptr, *q = nullptr;
+  CHECK(c.take(&p, 100 * MiB) == 0 && c.give(p) == 0);
+  CHECK(c.take(&q, 79 * MiB) == 0 && q != p && c.give(q) == 0);
+  CHECK(c.take(&q, 101 * MiB) == 0 && q != p && c.give(q) == 0);
+  c.trim();
+  CHECK(c.take(&p, 100 * MiB) == 0 && c.give(p) == 0);
+  CHECK(c.take(&q, 80 * MiB) == 0 && q == p && c.give(q) == 0);
+  CHECK(c.take(&q, 100 * MiB) == 0 && q == p && c.give(q) == 0);
+  CHECK(c.idle_bytes == 100 * MiB && c.idle.size() == 1);
+  CHECK(c.take(&p, 256 * MiB) == 0 && c.take(&q, 256 * MiB + 1) == 0);
+  Model::pending[0] = true;
+  CHECK(c.give(q) == 0 && !Model::pending[0] && Model::allocated.count(q) == 0);
+  CHECK(c.give(p) == 0 && c.idle_bytes == 356 * MiB);
+  void* many[5];
+  for (void*& m : many) CHECK(c.take(&m, 40 * MiB) == 0);
+  for (void* m : many) CHECK(c.give(m) == 0);
+  CHECK(c.idle_bytes == 476 * MiB && c.idle.size() == 5);
+  CHECK(c.trim() && c.idle_bytes == 0 && Model::used == 0 && c.blocks.empty());
+  CHECK(!c.trim());
+  return 0;
+}
+
 int main(int argc, char** argv) {
   const struct {
     const char* name;
@@ -196,7 +222,7 @@ int main(int argc, char** argv) {
   } checks[] = {{"huge_requests", huge_requests}, {"devices", devices}, {"recording", recording},
                 {"freed_in_stream_order", freed_in_stream_order},
                 {"freed_twice", freed_twice},
-                {"no_memory", no_memory}};
+                {"no_memory", no_memory}, {"rules", rules}};
   for (const auto& c : checks)
     if (argc > 1 && !std::strcmp(argv[1], c.name)) return c.run();
   std::printf("no such check\n");

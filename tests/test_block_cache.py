@@ -23,7 +23,7 @@ def checks(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("name", ["huge_requests", "devices", "recording", "freed_in_stream_order", "freed_twice", "no_memory"])
+@pytest.mark.parametrize("name", ["huge_requests", "devices", "recording", "freed_in_stream_order", "freed_twice", "no_memory", "rules"])
 def test_block_cache(checks, name):
     r = subprocess.run([str(checks), name], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout + r.stderr

@@ -3,6 +3,7 @@ rules themselves run on the CPU in test_block_cache.py."""
 import ctypes as C
 import threading
 
+import numpy as np
 import pytest
 
 import kokkos_amd as K
@@ -46,3 +47,50 @@ def test_free_leaves_a_capture_elsewhere_alone(paths):
     K.check(rt.mx_graph_exec_destroy(ex))
     K.check(rt.mx_graph_destroy(graph))
     K.check(rt.mx_stream_destroy(stream))
+
+
+def test_free_waits_for_queued_work(paths):
+    """A block is freed while kernels that write it are still queued on a
+    second stream, and taken again: its new content is the new owner's."""
+    P, rt = paths, K.load("kkmx_rt")
+    n = 16 * MiB  # doubles
+    K.check(rt.mx_trim())
+    a = alloc(rt, n * 8)
+    K.check(P.kkmx_deep_fill_f64(a, n, 1.0), P)
+    for _ in range(200):  # about 10 ms of kernels over the block, in place
+        K.check(P.kkmx_stream_scale(a, a, n, 1.0), P)
+    done = C.c_void_p()
+    K.check(rt.mx_event_create(C.byref(done)))
+    K.check(rt.mx_event_record(done, C.c_void_p(P.kkmx_stream())))
+    assert rt.mx_event_query(done) != 0  # still at work
+    K.check(rt.mx_free(a, None))
+    assert rt.mx_event_query(done) == 0
+    b = alloc(rt, n * 8)
+    assert b.value == a.value
+    other = C.c_void_p()
+    K.check(rt.mx_stream_create(C.byref(other)))
+    K.check(rt.mx_memset_async(b, 0, n * 8, other))
+    K.check(rt.mx_stream_sync(other))
+    K.fence()
+    got = np.empty(n)
+    K.check(rt.mx_memcpy(got.ctypes.data, b, n * 8))
+    assert not got.any()
+    K.check(rt.mx_free(b, None))
+    K.check(rt.mx_event_destroy(done))
+    K.check(rt.mx_stream_destroy(other))
+
+
+def test_impossible_request_and_second_free(paths):
+    rt = K.load("kkmx_rt")
+    for n in (2**64 - 1, 2**64 - 43, 2**64 - 65536, 1 << 60):
+        p = C.c_void_p(1)
+        assert rt.mx_malloc(C.byref(p), C.c_size_t(n), None) != 0
+        assert not p.value
+        rt.mx_get_last_error()
+    a = alloc(rt, 3 * MiB)
+    K.check(rt.mx_free(a, None))
+    assert rt.mx_free(a, None) != 0
+    b = alloc(rt, 3 * MiB)
+    assert b.value == a.value
+    K.check(rt.mx_free(b, None))
+    K.check(rt.mx_trim())
