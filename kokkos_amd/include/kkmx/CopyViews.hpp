@@ -119,7 +119,10 @@ struct TransposeShape {
   uint32_t mid[4];  // extents of the middle dimensions (1 when absent)
   int nmid;
   uint32_t tiles0, tileslast;  // their product with M is below 2^31
+  uint32_t first;              // tile of the launch's first workgroup
 };
+// Tiles of one launch: HIP takes fewer than 2^32 lanes along a grid dimension.
+constexpr int64_t kTransposeTiles = int64_t(1) << 22;
 // Tile extent along the destination's contiguous dimension.
 template <class W>
 constexpr int transpose_narrow = sizeof(W) == 8 ? 32 : 64;
@@ -128,7 +131,7 @@ __global__ __launch_bounds__(512) void k_layout_transpose(W* __restrict__ dst, c
                                                           const TransposeShape sh) {
   constexpr int N = transpose_narrow<W>;
   __shared__ W tile[N][65];
-  const uint32_t b  = blockIdx.x;
+  const uint32_t b  = sh.first + blockIdx.x;
   const uint32_t tk = b % sh.tileslast;
   const uint32_t t0 = (b / sh.tileslast) % sh.tiles0;
   uint32_t g        = b / (sh.tiles0 * sh.tileslast);  // middle multi-index, flattened left-first
@@ -215,7 +218,11 @@ bool layout_transpose(const MI355X& exec, const DV& dst, const SV& src) {
     const W* s_ = reinterpret_cast<const W*>(src.data());
     const void* k = lr ? reinterpret_cast<const void*>(&k_layout_transpose<W, true>)
                        : reinterpret_cast<const void*>(&k_layout_transpose<W, false>);
-    mx_launch_kernel(k, static_cast<unsigned>(blocks), 512, 0, exec.stream(), d, s_, sh);
+    for (int64_t done = 0; done < blocks; done += kTransposeTiles) {
+      sh.first            = uint32_t(done);
+      const int64_t tiles = blocks - done < kTransposeTiles ? blocks - done : kTransposeTiles;
+      mx_launch_kernel(k, static_cast<unsigned>(tiles), 512, 0, exec.stream(), d, s_, sh);
+    }
     return true;
   }
 }

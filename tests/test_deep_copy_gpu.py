@@ -56,6 +56,20 @@ def test_layout_copy_tile_edges(paths, oracle, shape, dst_layout, src_layout):
     test_layout_copy(paths, oracle, shape, dst_layout, src_layout)
 
 
+@pytest.mark.parametrize("to_right", [1, 0])
+def test_transpose_in_several_launches(paths, to_right):
+    """One tile more than a launch takes, 2^22, and some."""
+    import torch
+
+    m = (1 << 22) + 7
+    src = torch.randint(0, 1 << 62, (16, m, 16), device="cuda", generator=torch.Generator("cuda").manual_seed(to_right))
+    dst = torch.zeros_like(src)
+    torch.cuda.synchronize()
+    run(paths, paths.kkmx_deep_copy_f64(dst.data_ptr(), src.data_ptr(), 16, m, 16, to_right, 1 - to_right))
+    for a in range(0, m, 1 << 20):
+        assert torch.equal(dst[:, a : a + (1 << 20)], src[:, a : a + (1 << 20)].permute(2, 1, 0))
+
+
 def test_transpose_512_cubed(paths, oracle):
     """The measured case: 512^3 doubles, LayoutLeft -> LayoutRight."""
     P = paths

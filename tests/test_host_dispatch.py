@@ -1,0 +1,75 @@
+"""The host side of dispatches, without a GPU: libkkmx_paths.so on a stand-in
+for the runtime that records launches (tests/cpp/host_runtime.cpp).  Each test
+runs in a process of its own, as the stand-in takes the runtime's place."""
+import os
+import shutil
+import subprocess
+import sys
+import textwrap
+from pathlib import Path
+
+import pytest
+
+ROOT = Path(__file__).resolve().parents[1]
+PATHS = ROOT / "kokkos_amd" / "lib" / "libkkmx_paths.so"
+CXX = shutil.which("g++") or shutil.which("c++")
+
+PRELUDE = """
+import ctypes as C, sys
+H = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
+H.host_kernel.restype = H.host_label.restype = C.c_char_p
+H.host_grid.restype = H.host_block.restype = C.c_uint64
+H.host_held.restype = C.c_size_t
+P = C.CDLL(sys.argv[2], mode=C.RTLD_GLOBAL)
+P.kkmx_last_error.restype = P.kkmx_stream.restype = C.c_void_p
+at = lambda a: C.c_void_p(a)  # addresses that no launch reads here
+i64, f64, size = C.c_int64, C.c_double, C.c_size_t
+def launches():
+    return [(H.host_kernel(i).decode(), H.host_grid(i), H.host_block(i)) for i in range(H.host_launches())]
+def labels():
+    return [H.host_label(i).decode() for i in range(H.host_labels())]
+def start(cus=256):
+    H.host_set_cus(cus)
+    P.kkmx_init(0)
+    assert P.kkmx_stream()
+    H.host_clear()
+"""
+
+
+@pytest.fixture(scope="module")
+def runtime(tmp_path_factory):
+    if not CXX or not PATHS.exists():
+        pytest.skip("no host compiler, or the libraries are not built")
+    so = tmp_path_factory.mktemp("host_runtime") / "libkkmx_rt.so"
+    # the name by which libkkmx_paths.so asks for its runtime
+    cmd = [CXX, "-std=c++17", "-O1", "-Wall", "-shared", "-fPIC", "-Wl,-soname,libkkmx_rt.so", "-I", str(ROOT / "include"),
+           str(ROOT / "tests" / "cpp" / "host_runtime.cpp"), "-o", str(so), "-ldl"]
+    r = subprocess.run(cmd, capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stderr[-4000:]
+    return so
+
+
+def run(runtime, body, tool=False):
+    env = dict(os.environ)
+    env.pop("KOKKOS_TOOLS_LIBS", None)
+    if tool:
+        env["KOKKOS_TOOLS_LIBS"] = str(runtime)
+    r = subprocess.run([sys.executable, "-c", PRELUDE + textwrap.dedent(body), str(runtime), str(PATHS)],
+                       capture_output=True, text=True, timeout=120, env=env)
+    assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-4000:]
+
+
+@pytest.mark.parametrize("m", [(1 << 22) - 1, 1 << 22, (1 << 22) + 1, (1 << 23) + 5, 40_000_000])
+@pytest.mark.parametrize("to_right", [1, 0])
+def test_transpose_of_many_tiles(runtime, m, to_right):
+    """16 x m x 16 doubles are m tiles.  A launch has fewer than 2^32 lanes, and
+    the launches together have m workgroups."""
+    run(runtime, f"""
+        start()
+        rc = P.kkmx_deep_copy_f64(at(1 << 46), at(1 << 45), i64(16), i64({m}), i64(16), {to_right}, {1 - to_right})
+        got = launches()
+        assert rc == 0 and got
+        assert all('k_layout_transpose' in k for k, _, _ in got), got
+        assert all(grid * block < 1 << 32 for _, grid, block in got), got
+        assert sum(grid for _, grid, _ in got) == {m}, got
+    """)
