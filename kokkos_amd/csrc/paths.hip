@@ -801,7 +801,9 @@ struct HistRowSum {
     }
   }
 };
-// Grow-only table of team rows for mode 3, released by Kokkos::finalize.
+// Grow-only table of team rows for mode 3, released by Kokkos::finalize.  Calls
+// ask for a row per CU also where fewer teams run, so that a call with more keys
+// leaves the table in place that a captured call's graph writes to.
 int32_t* hist_rows_space(size_t elems) {
   static Kokkos::View<int32_t*, Kokkos::MI355XSpace>* rows = nullptr;
   if (!rows) {
@@ -1469,7 +1471,7 @@ int kkmx_histogram(const int32_t* keys, int64_t n, int32_t* bins, int32_t nbins,
       const size_t budget = Kokkos::TeamPolicy<Kokkos::MI355X>(cus_, 1024).scratch_size_max(0);
       if (HistPacked::scratch_words(nbins) * 4 <= budget && n / cus_ < HistPacked::kMaxKeysPerTeam - 4096) {
         const int teams = hist_teams(n, cus_);
-        int32_t* rows   = hist_rows_space(size_t(teams) * nbins);
+        int32_t* rows   = hist_rows_space(size_t(cus_) * nbins);
         using Rows = Kokkos::View<int32_t**, Kokkos::LayoutRight, Kokkos::MI355XSpace, Kokkos::MemoryTraits<Kokkos::Unmanaged>>;
         auto pol = Kokkos::TeamPolicy<Kokkos::MI355X>(teams, 1024)
                        .set_scratch_size(0, Kokkos::PerTeam(HistPacked::scratch_words(nbins) * 4));
@@ -1489,7 +1491,7 @@ int kkmx_histogram(const int32_t* keys, int64_t n, int32_t* bins, int32_t nbins,
       const int64_t fit   = int64_t(budget / 4) - int64_t(HistRows::kHotCopies) * (hot + 1);
       if (lb3 > fit) lb3 = int32_t(fit);
       const int teams = hist_teams(n, cus);
-      int32_t* rows   = hist_rows_space(size_t(teams) * nbins);
+      int32_t* rows   = hist_rows_space(size_t(cus) * nbins);
       using Rows = Kokkos::View<int32_t**, Kokkos::LayoutRight, Kokkos::MI355XSpace, Kokkos::MemoryTraits<Kokkos::Unmanaged>>;
       auto pol = Kokkos::TeamPolicy<Kokkos::MI355X>(teams, 1024)
                      .set_scratch_size(0, Kokkos::PerTeam(HistRows::scratch_bytes(lb3, hot)));

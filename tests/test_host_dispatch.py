@@ -73,3 +73,16 @@ def test_transpose_of_many_tiles(runtime, m, to_right):
         assert all(grid * block < 1 << 32 for _, grid, block in got), got
         assert sum(grid for _, grid, _ in got) == {m}, got
     """)
+
+
+@pytest.mark.parametrize("nbins", [65536, 100000])
+def test_histogram_rows_stay(runtime, nbins):
+    """A call with few keys makes the table that one with many keys uses: a
+    graph that captured the former keeps its address."""
+    run(runtime, f"""
+        start()
+        for n in (1000, 1 << 18, 1 << 22, 1 << 24):
+            assert P.kkmx_histogram(at(1 << 45), i64(n), at(1 << 46), {nbins}, 3, 0) == 0
+            assert H.host_allocs() == (1 if n == 1000 else 0), (n, H.host_allocs())
+            H.host_clear()
+    """)

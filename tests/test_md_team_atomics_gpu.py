@@ -354,3 +354,31 @@ def test_histogram_mode3_team_counts(paths, oracle, n, nb):
     Kb, Bb = dev(keys), dev(np.full(nb, 5, np.int32))
     run(P, P.kkmx_histogram(Kb.ptr, n, Bb.ptr, nb, 3, 0))
     assert np.array_equal(Bb.download(np.int32, nb), oracle.histogram(keys, nb) + 5)
+
+
+def test_histogram_captured_then_more_keys(paths, oracle):
+    """A captured call with few keys keeps its table of team rows when calls
+    with many keys follow: replays count right and write nowhere else."""
+    P, rt = paths, K.load("kkmx_rt")
+    n, many, nb = 20011, 1 << 23, 65536
+    keys = oracle.fill_uniform_i32(n, 96, 0, nb - 1)
+    Kb, Bb = dev(keys), dev(np.zeros(nb, np.int32))
+    Km, Bm = dev(oracle.fill_uniform_i32(many, 97, 0, nb - 1)), dev(np.zeros(nb, np.int32))
+    run(P, P.kkmx_histogram(Kb.ptr, n, Bb.ptr, nb, 3, 0))
+    s = P.kkmx_stream()
+    graph, ex = C.c_void_p(), C.c_void_p()
+    K.check(rt.mx_graph_capture_begin(C.c_void_p(s)))
+    K.check(P.kkmx_histogram(Kb.ptr, n, Bb.ptr, nb, 3, 0), P)
+    K.check(rt.mx_graph_capture_end(C.c_void_p(s), C.byref(graph)))
+    K.check(rt.mx_graph_instantiate(C.byref(ex), graph))
+    ref = oracle.histogram(keys, nb)
+    others = []
+    for k in range(3):
+        run(P, P.kkmx_histogram(Km.ptr, many, Bm.ptr, nb, 3, 0))
+        others += [dev(np.full(1 << 20, -7, np.int32)), dev(np.full(1 << 24, -7, np.int32))]
+        K.check(rt.mx_graph_launch(ex, C.c_void_p(s)))
+        K.fence()
+        assert np.array_equal(Bb.download(np.int32, nb), ref * (k + 2))
+        assert all(np.all(o.download(np.int32, o.nbytes // 4) == -7) for o in others)
+    K.check(rt.mx_graph_exec_destroy(ex))
+    K.check(rt.mx_graph_destroy(graph))
