@@ -475,6 +475,10 @@ class BinSort {
     sort_order  = offset_type(view_alloc(WithoutInitializing, std::string("Kokkos::BinSort::sort_order")), len);
     bin_count   = View<int*, MI355XSpace>(view_alloc(WithoutInitializing, std::string("Kokkos::BinSort::bin_count")), bins);
     bin_offsets = offset_type(view_alloc(WithoutInitializing, std::string("Kokkos::BinSort::bin_offsets")), bins);
+    // made here and not where it is used, so that create_permute_vector can be
+    // captured; a radix sort cannot, and its calls hardly ever need it
+    if (!(by_code && sort_within_bins && len > 0))
+      bin_fill = View<int*, MI355XSpace>(view_alloc(WithoutInitializing, std::string("Kokkos::BinSort::bin_fill")), bins);
     // one launch and one wait for all three
     using U = View<int*, MI355XSpace, MemoryTraits<Unmanaged>>;
     parallel_for("Kokkos::Sort::BinZero", RangePolicy<MI355X, IndexType<size_t>>(exec, 0, len > bins ? len : bins),
@@ -498,8 +502,7 @@ class BinSort {
     const int bins = bin_op.max_bins();
     U cnt(bin_count.data(), size_t(bins));
     U off(bin_offsets.data(), size_t(bins)), order(sort_order.data(), size_t(len));
-    if constexpr (Impl::is_bin_op_1d<BinSortOp>::value && KeyViewType::rank == 1 &&
-                  Impl::radix_sortable<KeyViewType>()) {
+    if constexpr (by_code) {
       if (sort_within_bins && len > 0 &&
           Impl::bin_order_by_code(exec, keys, bin_op, range_begin, len, bins, order.data(), cnt.data(), off.data())) {
         if (range_begin != 0)
@@ -514,8 +517,7 @@ class BinSort {
     parallel_for("Kokkos::Sort::BinCount", RangePolicy<MI355X>(exec, 0, len),
                  Impl::BinCountF<const_key_view_type, BinSortOp>{keys, bin_op, cnt, range_begin});
     parallel_scan("Kokkos::Sort::BinOffset", RangePolicy<MI355X>(exec, 0, bins), Impl::BinOffsetF{CU(cnt), off});
-    if constexpr (Impl::is_bin_op_1d<BinSortOp>::value && KeyViewType::rank == 1 &&
-                  Impl::radix_sortable<KeyViewType>()) {
+    if constexpr (by_code) {
       // BinOp1D's bin never decreases as the key grows, so "by bin, then by
       // key, equal keys in index order" is the stable order of the keys: the
       // permutation of a radix sort of (key, position) pairs
@@ -597,6 +599,9 @@ class BinSort {
   bin_count_type get_bin_count() const { return bin_count; }
 
  private:
+  // within bins, the ordering is a radix sort
+  static constexpr bool by_code =
+      Impl::is_bin_op_1d<BinSortOp>::value && KeyViewType::rank == 1 && Impl::radix_sortable<KeyViewType>();
   const_key_view_type keys;
   int range_begin = 0, range_end = 0;
   BinSortOp bin_op;

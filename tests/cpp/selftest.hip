@@ -2862,6 +2862,54 @@ KKMX_TEST(binsort_quantised_forms) {
   }
 }
 
+// A sorter made beforehand orders by bins (no order within them) in a captured
+// call, the first on this sorter; replays see the keys of their time.
+KKMX_TEST(binsort_captured) {
+  const int n = 5000, nbins = 37;
+  using DV = Kokkos::View<double*, Exec>;
+  DV keys("keys", n);
+  mx_stream_t stream = nullptr;
+  KKMX_SAFE_CALL(mx_stream_create(&stream));
+  mx_graph_t graph      = nullptr;
+  mx_graph_exec_t ready = nullptr;
+  {
+    Exec ex(stream);
+    Kokkos::BinOp1D<DV> op(nbins, 0.0, 1.0);
+    using Sorter = Kokkos::BinSort<DV, Kokkos::BinOp1D<DV>>;
+    Sorter(ex, keys, 0, n, op).create_permute_vector(ex);  // the instance's own scratch
+    Sorter sorter(ex, keys, 0, n, op);
+    ex.fence();
+    KKMX_SAFE_CALL(mx_graph_capture_begin(stream));
+    sorter.create_permute_vector(ex);
+    KKMX_SAFE_CALL(mx_graph_capture_end(stream, &graph));
+    KKMX_SAFE_CALL(mx_graph_instantiate(&ready, graph));
+    for (int replay = 0; replay < 3; ++replay) {
+      auto m = Kokkos::create_mirror_view(keys);
+      std::vector<int> want(nbins + 1, 0);
+      for (int i = 0; i < n; ++i) {
+        m(i) = double((int64_t(i + replay) * 2654435761ll) % 10007) / 10007.0;
+        ++want[op.bin(m, i)];
+      }
+      Kokkos::deep_copy(keys, m);
+      KKMX_SAFE_CALL(mx_graph_launch(ready, stream));
+      ex.fence();
+      auto perm = Kokkos::create_mirror_view_and_copy(Kokkos::HostSpace(), sorter.get_permute_vector());
+      auto cnt  = Kokkos::create_mirror_view_and_copy(Kokkos::HostSpace(), sorter.get_bin_count());
+      std::vector<int> seen(n, 0);
+      for (int i = 0; i < n; ++i) {
+        CHECK(perm(i) >= 0 && perm(i) < n);
+        ++seen[perm(i)];
+        if (i > 0) CHECK(op.bin(m, perm(i - 1)) <= op.bin(m, perm(i)));
+      }
+      for (int i = 0; i < n; ++i) CHECK_EQ(seen[i], 1);
+      for (int b = 0; b <= nbins; ++b) CHECK_EQ(cnt(b), want[b]);
+    }
+    KKMX_SAFE_CALL(mx_graph_exec_destroy(ready));
+    KKMX_SAFE_CALL(mx_graph_destroy(graph));
+  }
+  KKMX_SAFE_CALL(mx_stream_destroy(stream));
+}
+
 // =========================================================================
 // Kokkos::sort of strided keys (TestSort.hpp sorts subviews): every third
 // element of a buffer, whole and over [begin, end), on the device; the
