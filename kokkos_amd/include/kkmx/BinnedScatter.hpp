@@ -180,7 +180,7 @@ inline void binned_scatter_add(const double* vals, const int32_t* idx, int64_t n
   uint32_t* counts  = reinterpret_cast<uint32_t*>(base + key_bytes + val_bytes);
   RadixControl* ctl = reinterpret_cast<RadixControl*>(base + key_bytes + val_bytes + count_bytes);
   int pass = -1, turn = 0;
-  bool fold = false;
+  bool fold = false, summed = true;  // k_scatter_bins reads the totals, so k_radix_offsets always runs
   for (int64_t done = 0; done < n; done += piece) {
     int64_t m              = n - done < piece ? n - done : piece;
     const uint32_t* i0     = k0 + done;
@@ -195,7 +195,8 @@ inline void binned_scatter_add(const double* vals, const int32_t* idx, int64_t n
                      pass, ctl, turn, counts, segments);
     mx_launch_kernel(
         reinterpret_cast<const void*>(&k_radix_scatter<uint32_t, uint64_t, false, Shape::lanes, Shape::items>),
-        unsigned(segments), Shape::lanes, 0, stream, pass, bin_shift, m, segment, i0, k1, v0, v1, ctl, turn, counts);
+        unsigned(segments), Shape::lanes, 0, stream, pass, bin_shift, m, segment, i0, k1, v0, v1, ctl, turn, counts,
+        summed);
     // a part of an evenly filled run is the whole run
     int64_t part           = m / 256 + m / 2048 + 1;
     const uint32_t* totals = ctl->totals;

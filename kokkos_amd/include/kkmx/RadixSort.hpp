@@ -298,11 +298,13 @@ constexpr int kRadixDirect = 48;
 // One digit, one segment per block, tile after tile of Lanes x Items keys;
 // wavefront w holds a run of 64 * Items of them.  Thread d < 256 carries digit
 // d's next output position from tile to tile, and the next tile's keys are
-// loaded before this one is written out.
+// loaded before this one is written out.  `summed` says that k_radix_offsets has
+// been over the counts; else they are the segments' own, added up here.
 template <class T, class PT, bool Iota, int Lanes, int Items>
 __global__ __launch_bounds__(Lanes, 4) void k_radix_scatter(
     const int p, const int pass_shift, const int64_t n, const int64_t segment, const typename RadixKey<T>::U* k0,
-    typename RadixKey<T>::U* k1, const PT* p0, PT* p1, const RadixControl* ctl, const int turn, const uint32_t* counts) {
+    typename RadixKey<T>::U* k1, const PT* p0, PT* p1, const RadixControl* ctl, const int turn, const uint32_t* counts,
+    const bool summed) {
   using R              = RadixKey<T>;
   using U              = typename R::U;
   constexpr bool Pairs = !std::is_same<PT, NoPayload>::value;
@@ -356,7 +358,7 @@ __global__ __launch_bounds__(Lanes, 4) void k_radix_scatter(
   {
     uint32_t total = 0;
     if (t < 256) {
-      if (int(gridDim.x) <= kRadixDirect) {
+      if (!summed) {
 #pragma unroll 16
         for (int q = 0; q < int(gridDim.x); ++q) {
           const uint32_t x = counts[q * 256 + t];
@@ -910,12 +912,13 @@ struct RadixRun {
       if (p > 0 || sizeof(T) == 8)  // digit 0 of 4-byte keys is counted by the fold
         mx_launch_kernel(reinterpret_cast<const void*>(&k_radix_count<T, Iota>), unsigned(segments), kRadixCountLanes,
                          0, stream, p, shift, n, segment, k0, k1, ctl, turn, no, counts);
-      if (segments > kRadixDirect)
+      bool summed = segments > kRadixDirect;
+      if (summed)
         mx_launch_kernel(reinterpret_cast<const void*>(&k_radix_offsets<T, Iota>), 64, kRadixOffsetLanes, 0, stream, p,
                          ctl, turn, counts, segments);
       mx_launch_kernel(reinterpret_cast<const void*>(&k_radix_scatter<T, PT, Iota, Shape::lanes, Shape::items>),
                        unsigned(segments), Shape::lanes, 0, stream, p, shift, n, segment, k0, k1, p0, p1, ctl, turn,
-                       counts);
+                       counts, summed);
     }
   }
   void sample(bool allow) {

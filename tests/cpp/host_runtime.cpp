@@ -18,6 +18,7 @@ namespace {
 struct Launch {
   std::string kernel;
   uint64_t grid, block;
+  std::string args;  // the first byte of each
 };
 std::vector<Launch> launches;
 std::vector<std::string> labels;
@@ -58,6 +59,8 @@ int host_launches() { return int(launches.size()); }
 const char* host_kernel(int i) { return launches[i].kernel.c_str(); }
 uint64_t host_grid(int i) { return launches[i].grid; }
 uint64_t host_block(int i) { return launches[i].block; }
+int host_args(int i) { return int(launches[i].args.size()); }
+int host_arg(int i, int arg) { return static_cast<unsigned char>(launches[i].args[arg]); }
 int host_labels() { return int(labels.size()); }
 const char* host_label(int i) { return labels[i].c_str(); }
 int host_allocs() { return allocs; }
@@ -148,10 +151,12 @@ int mx_stream_capturing(mx_stream_t, int* yes) {
 }
 int mx_stream_wait_event(mx_stream_t, mx_event_t) { return 0; }
 int mx_launch(const void* fn, unsigned gx, unsigned gy, unsigned gz, unsigned bx, unsigned by, unsigned bz, size_t,
-              void**, mx_stream_t) {
+              void** args, mx_stream_t) {
+  std::string bytes;
+  while (args && *args) bytes += *static_cast<char*>(*args++);
   Dl_info info;
   const bool known = dladdr(fn, &info) != 0 && info.dli_sname;
-  launches.push_back({known ? info.dli_sname : "", uint64_t(gx) * gy * gz, uint64_t(bx) * by * bz});
+  launches.push_back({known ? info.dli_sname : "", uint64_t(gx) * gy * gz, uint64_t(bx) * by * bz, bytes});
   return 0;
 }
 int mx_func_attributes(const void*, int* threads, int* regs, size_t* lds, size_t* priv) {

@@ -86,3 +86,24 @@ def test_histogram_rows_stay(runtime, nbins):
             assert H.host_allocs() == (1 if n == 1000 else 0), (n, H.host_allocs())
             H.host_clear()
     """)
+
+
+@pytest.mark.parametrize("cus", [8, 24, 25, 32, 256])
+def test_scatter_moves_by_summed_counts(runtime, cus):
+    """However many segments the CUs give the move, its last kernel is told that
+    the counts were summed; a sort's, where the launch before it did that."""
+    run(runtime, f"""
+        start({cus})
+        def check():
+            got = [k for k, _, _ in launches()]
+            for i, k in enumerate(got):
+                if 'k_radix_scatter' in k:
+                    assert H.host_arg(i, H.host_args(i) - 1) == ('k_radix_offsets' in got[i - 1]), got
+            return sum('k_radix_scatter' in k for k in got), sum('k_radix_offsets' in k for k in got)
+        assert P.kkmx_scatter_add_f64(at(1 << 45), at(1 << 46), i64(1 << 20), at(1 << 47), 1 << 20) == 0
+        assert check() == (1, 1)
+        H.host_clear()
+        for n in (100000, 1 << 20, 1 << 24):
+            assert P.kkmx_sort(at(1 << 45), i64(n), 0) == 0
+        check()
+    """)
