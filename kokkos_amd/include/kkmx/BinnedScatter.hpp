@@ -127,8 +127,9 @@ inline bool binned_scatter_takes(int64_t n, int64_t nbins, mx_stream_t stream) {
   return mx_stream_capturing(stream, &capturing) == 0 && !capturing;
 }
 
-// bins[idx[i]] += vals[i], i < n, on the default instance.
-inline void binned_scatter_add(const double* vals, const int32_t* idx, int64_t n, double* bins, int64_t nbins) {
+// bins[idx[i]] += vals[i], i < n, on the default instance.  False, with nothing
+// done, where there is no memory for the workspace: atomics need none.
+inline bool binned_scatter_add(const double* vals, const int32_t* idx, int64_t n, double* bins, int64_t nbins) {
   MI355X exec;
   mx_stream_t stream = exec.stream();
   const int cus      = MI355X::impl_cu_count() > 0 ? MI355X::impl_cu_count() : 256;
@@ -149,7 +150,7 @@ inline void binned_scatter_add(const double* vals, const int32_t* idx, int64_t n
                        i0, v0, m, totals, part, bin_shift, bins, nbins);
       done += m;
     }
-    return;
+    return true;
   }
   int bin_shift = 10;  // at least 1024 bins a run: fewer would meet in LDS
   while ((nbins - 1) >> bin_shift > 255) ++bin_shift;
@@ -167,7 +168,10 @@ inline void binned_scatter_add(const double* vals, const int32_t* idx, int64_t n
     if (ws.buf) KKMX_SAFE_CALL(mx_free(ws.buf, nullptr));
     ws.buf   = nullptr;
     ws.bytes = 0;
-    KKMX_SAFE_CALL(mx_malloc(&ws.buf, need, nullptr));
+    if (mx_malloc(&ws.buf, need, nullptr) != 0) {
+      (void)mx_get_last_error();
+      return false;
+    }
     ws.bytes = need;
   }
   if (!ws.hooked) {
@@ -205,6 +209,7 @@ inline void binned_scatter_add(const double* vals, const int32_t* idx, int64_t n
     mx_launch_kernel(kernel, unsigned(256 + (m + part - 1) / part), kScatterLanes, sizeof(double) << bin_shift, stream,
                      ck1, cv1, m, totals, part, bin_shift, bins, nbins);
   }
+  return true;
 }
 
 }  // namespace Impl

@@ -107,3 +107,21 @@ def test_scatter_moves_by_summed_counts(runtime, cus):
             assert P.kkmx_sort(at(1 << 45), i64(n), 0) == 0
         check()
     """)
+
+
+def test_scatter_without_memory(runtime):
+    """Without memory for its workspace the scatter-add runs by atomics, which
+    need none, and takes the workspace up again once there is some."""
+    run(runtime, """
+        start()
+        call = lambda: P.kkmx_scatter_add_f64(at(1 << 45), at(1 << 46), i64(1 << 24), at(1 << 47), 1 << 20)
+        for limit, binned in ((1 << 20, False), (1 << 30, True)):
+            H.host_set_limit(size(limit))
+            H.host_clear()
+            assert call() == 0
+            got = launches()
+            assert len(got) == (4 if binned else 1) and any('k_scatter_bins' in k for k, _, _ in got) == binned, got
+        held = H.host_held()
+        H.host_set_limit(size(0))
+        assert call() == 0 and H.host_held() == held
+    """)
