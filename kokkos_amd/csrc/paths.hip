@@ -1541,7 +1541,7 @@ int kkmx_scatter_add_f64(const double* vals, const int32_t* idx, int64_t n, doub
   if (n < 0 || nbins < 1 || !bins || (n && (!vals || !idx))) return reject("kkmx_scatter_add_f64: bad arguments");
   return guarded([&] {
     if (Kokkos::Impl::binned_scatter_takes(n, nbins, Kokkos::MI355X().stream()) &&
-        Kokkos::Impl::binned_scatter_add(vals, idx, n, bins, nbins))
+        Kokkos::Impl::binned_scatter_add("kkmx::scatter_f64", vals, idx, n, bins, nbins))
       return;
     Kokkos::parallel_for("kkmx::scatter_f64", Range64(0, n),
                          ScatterAdd{DevView<const double>(vals, n), DevView<const int32_t>(idx, n), DevView<double>(bins, nbins)});

@@ -127,15 +127,18 @@ inline bool binned_scatter_takes(int64_t n, int64_t nbins, mx_stream_t stream) {
   return mx_stream_capturing(stream, &capturing) == 0 && !capturing;
 }
 
-// bins[idx[i]] += vals[i], i < n, on the default instance.  False, with nothing
+// bins[idx[i]] += vals[i], i < n, on the default instance; to a tool, one
+// parallel_for by the name of `label`, as the atomics are.  False, with nothing
 // done, where there is no memory for the workspace: atomics need none.
-inline bool binned_scatter_add(const double* vals, const int32_t* idx, int64_t n, double* bins, int64_t nbins) {
+inline bool binned_scatter_add(const char* label, const double* vals, const int32_t* idx, int64_t n, double* bins,
+                               int64_t nbins) {
   MI355X exec;
   mx_stream_t stream = exec.stream();
   const int cus      = MI355X::impl_cu_count() > 0 ? MI355X::impl_cu_count() : 256;
   const uint32_t* k0 = reinterpret_cast<const uint32_t*>(idx);
   const void* kernel = reinterpret_cast<const void*>(&k_scatter_bins<>);
   if (nbins <= kScatterDirect) {
+    const ToolsKernel<MI355X> tools(label, exec, 0);
     // two blocks per CU, and a round of the lanes each; pieces keep the
     // positions 32-bit
     for (int64_t done = 0; done < n;) {
@@ -178,6 +181,7 @@ inline bool binned_scatter_add(const double* vals, const int32_t* idx, int64_t n
     push_finalize_hook(&scatter_workspace_release);
     ws.hooked = true;
   }
+  const ToolsKernel<MI355X> tools(label, exec, 0);
   char* base        = static_cast<char*>(ws.buf);
   uint32_t* k1      = reinterpret_cast<uint32_t*>(base);
   uint64_t* v1      = reinterpret_cast<uint64_t*>(base + key_bytes);

@@ -125,3 +125,15 @@ def test_scatter_without_memory(runtime):
         H.host_set_limit(size(0))
         assert call() == 0 and H.host_held() == held
     """)
+
+
+@pytest.mark.parametrize("n,nbins", [(1000, 100), (1 << 18, 4096), (1 << 20, 4097), (1 << 25, 1 << 20)])
+def test_scatter_is_one_dispatch_to_a_tool(runtime, n, nbins):
+    run(runtime, f"""
+        start()
+        for limit in (1 << 40, 0):
+            H.host_set_limit(size(limit))
+            H.host_clear()
+            assert P.kkmx_scatter_add_f64(at(1 << 45), at(1 << 46), i64({n}), at(1 << 47), {nbins}) == 0
+            assert labels() == ['kkmx::scatter_f64'], labels()
+    """, tool=True)
