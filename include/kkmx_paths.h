@@ -147,7 +147,8 @@ int kkmx_scan_excl_f64(const double* in_dev, double* out_dev, int64_t n, double*
  * variant leaves both grids as sweeps u -> v -> u ... do, with the same bits;
  * with the default tile, at least 96 points a side and at least 5 sweeps it
  * takes them in pairs, each one pass over memory (a TeamPolicy dispatch in
- * place of two MDRange ones).  (reference: core/src/KokkosExp_MDRangePolicy.hpp:158-426) */
+ * place of two MDRange ones), unless a tuning tool is loaded, which chooses the
+ * MDRange tile.  (reference: core/src/KokkosExp_MDRangePolicy.hpp:158-426) */
 int kkmx_stencil7(const double* u_dev, double* v_dev, int64_t n, double c0, double c1, int t0, int t1, int t2);
 int kkmx_stencil7_sweeps(double* u_dev, double* v_dev, int64_t n, int sweeps, double c0, double c1, int t0, int t1,
                          int t2);

@@ -1335,7 +1335,9 @@ int kkmx_stencil7(const double* u, double* v, int64_t n, double c0, double c1, i
 }
 int kkmx_stencil7_sweeps(double* u, double* v, int64_t n, int sweeps, double c0, double c1, int t0, int t1, int t2) {
   int s = 0;
-  if (t0 <= 0 && n >= kPairMin && n < (int64_t(1) << 15) && u && v) {
+  // a tuning tool chooses the MDRange tile of sweeps with the default one
+  const bool tuned = Kokkos::Tools::Experimental::have_tuning_tool();
+  if (t0 <= 0 && !tuned && n >= kPairMin && n < (int64_t(1) << 15) && u && v) {
     // An even number of pairs, u -> v -> u, so that the sweeps after them,
     // one at least, leave both grids as single sweeps would.
     const int pairs = sweeps > 0 ? ((sweeps - 1) / 2) & ~1 : 0;

@@ -49,11 +49,11 @@ def runtime(tmp_path_factory):
     return so
 
 
-def run(runtime, body, tool=False):
+def run(runtime, body, tools=()):
     env = dict(os.environ)
     env.pop("KOKKOS_TOOLS_LIBS", None)
-    if tool:
-        env["KOKKOS_TOOLS_LIBS"] = str(runtime)
+    if tools:
+        env["KOKKOS_TOOLS_LIBS"] = ";".join(map(str, tools))
     r = subprocess.run([sys.executable, "-c", PRELUDE + textwrap.dedent(body), str(runtime), str(PATHS)],
                        capture_output=True, text=True, timeout=120, env=env)
     assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-4000:]
@@ -136,4 +136,21 @@ def test_scatter_is_one_dispatch_to_a_tool(runtime, n, nbins):
             H.host_clear()
             assert P.kkmx_scatter_add_f64(at(1 << 45), at(1 << 46), i64({n}), at(1 << 47), {nbins}) == 0
             assert labels() == ['kkmx::scatter_f64'], labels()
-    """, tool=True)
+    """, tools=[runtime])
+
+
+def test_stencil_sweeps_and_tuning_tools(runtime, tmp_path):
+    """Ten sweeps with the default tile: four pairs and two single sweeps, and
+    ten MDRange dispatches, whose tile it chooses, where a tuning tool is loaded."""
+    tuner = tmp_path / "libtuner.so"
+    src = tmp_path / "tuner.c"
+    src.write_text("void kokkosp_request_values(unsigned long a, unsigned long b, void* c, unsigned long d, void* e) {}")
+    r = subprocess.run([CXX, "-x", "c", "-shared", "-fPIC", str(src), "-o", str(tuner)], capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr
+    for tools, want in (([runtime], ["kkmx::stencil7_pair"] * 4 + ["kkmx::stencil7"] * 2),
+                        ([runtime, tuner], ["kkmx::stencil7"] * 10)):
+        run(runtime, f"""
+            start()
+            assert P.kkmx_stencil7_sweeps(at(1 << 45), at(1 << 46), i64(200), 10, f64(.4), f64(.1), 0, 0, 0) == 0
+            assert labels() == {want}, labels()
+        """, tools=tools)
