@@ -268,6 +268,9 @@ struct BinWorkspace {
   bool clear      = false;
   void* space(size_t need);
 };
+// Values of a sorter go through the kept scratch up to this size, larger ones
+// through a copy of their own: rows can be of any size, and the scratch stays.
+constexpr size_t kBinRowsKept = size_t(256) << 20;
 inline BinWorkspace& bin_workspace() {
   static BinWorkspace w;
   return w;
@@ -560,15 +563,18 @@ class BinSort {
     if constexpr (ValuesViewType::rank == 1 && std::is_trivially_copyable<W>::value) {
       // through the kept scratch, which is free again once the stream is done
       using Rows               = View<W*, MI355XSpace, MemoryTraits<Unmanaged>>;
+      const size_t need        = size_t(len) * sizeof(W);
       Impl::BinWorkspace& ws   = Impl::bin_workspace();
       std::lock_guard<std::mutex> lock(ws.mtx);
-      Rows rows(static_cast<W*>(ws.space(size_t(len) * sizeof(W))), size_t(len));
-      parallel_for("Kokkos::Sort::CopyPermute", RangePolicy<MI355X>(exec, 0, len),
-                   Impl::PermuteRowsF<Rows, ValuesViewType>{rows, values, order, values_range_begin - range_begin});
-      parallel_for("Kokkos::Sort::Copy", RangePolicy<MI355X>(exec, 0, len),
-                   Impl::CopyRowsF<ValuesViewType, Rows>{values, rows, range_begin});
-      exec.fence("Kokkos::BinSort::sort: values in place");
-      return;
+      if (need <= Impl::kBinRowsKept || need <= ws.bytes) {
+        Rows rows(static_cast<W*>(ws.space(need)), size_t(len));
+        parallel_for("Kokkos::Sort::CopyPermute", RangePolicy<MI355X>(exec, 0, len),
+                     Impl::PermuteRowsF<Rows, ValuesViewType>{rows, values, order, values_range_begin - range_begin});
+        parallel_for("Kokkos::Sort::Copy", RangePolicy<MI355X>(exec, 0, len),
+                     Impl::CopyRowsF<ValuesViewType, Rows>{values, rows, range_begin});
+        exec.fence("Kokkos::BinSort::sort: values in place");
+        return;
+      }
     }
     using Tmp = View<typename ValuesViewType::non_const_data_type, typename ValuesViewType::array_layout, MI355XSpace>;
     Tmp tmp(std::string("Kokkos::SortImpl::BinSortFunctor::sorted_values"), size_t(len),

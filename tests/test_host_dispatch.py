@@ -154,3 +154,15 @@ def test_stencil_sweeps_and_tuning_tools(runtime, tmp_path):
             assert P.kkmx_stencil7_sweeps(at(1 << 45), at(1 << 46), i64(200), 10, f64(.4), f64(.1), 0, 0, 0) == 0
             assert labels() == {want}, labels()
         """, tools=tools)
+
+
+@pytest.mark.parametrize("n,kept", [(1 << 25, 1 << 28), ((1 << 25) + 1024, 0)])
+def test_binsort_keeps_no_large_values(runtime, n, kept):
+    """Up to 256 MiB of values leave their scratch for the next call."""
+    run(runtime, f"""
+        start()
+        before = H.host_held()
+        assert P.kkmx_binsort_f64(at(1 << 45), at(1 << 46), i64({n}), 100, f64(0), f64(1), 0, None) == 0
+        assert {kept} <= H.host_held() - before < {kept} + (1 << 20), H.host_held() - before
+        assert sum('CopyRows' in k for k, _, _ in launches()) == 1, launches()
+    """)
