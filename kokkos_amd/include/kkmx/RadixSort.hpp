@@ -502,9 +502,10 @@ __global__ __launch_bounds__(1024) void k_radix_sample(const typename RadixKey<T
 // Most keys have no such neighbour, or a run already in order, which a
 // wavefront sees from its own and the neighbouring wavefronts' ballots.  A run
 // of 64 keys or more (every key of it sees that) is left as it is, and reported
-// where it is out of order (status 1): the caller's keys are then still a
-// stable order by the trimmed digits, and all digits are sorted over.  Status 2
-// reports digits left to sort where nothing was trimmed.
+// where it is out of order (status[0] 1, status[1] the lowest bit sorted by): the
+// caller's keys are then still a stable order by the trimmed digits, and the keys
+// of such runs are sorted by themselves (radix_sort_long_runs).  Status 2 reports
+// digits left to sort where nothing was trimmed.
 constexpr int kRadixRun         = 64;
 constexpr int kRadixFinishLanes = 1024;
 constexpr int kRadixFinishTile  = 4096;
@@ -611,7 +612,7 @@ __global__ __launch_bounds__(kRadixFinishLanes) void k_radix_finish(const int64_
     }
     __syncthreads();
   }
-  if (broken) *status = 1;
+  if (broken) status[0] = 1, status[1] = uint32_t(low);
 }
 
 // Runs of at most 1024 x Items keys, each sorted by one block in LDS: every
@@ -800,7 +801,7 @@ struct RadixWorkspace {
   void* buf             = nullptr;
   size_t bytes          = 0;
   RadixControl* control = nullptr;
-  uint32_t* status      = nullptr;  // pinned host word that k_radix_finish reports to
+  uint32_t* status      = nullptr;  // pinned host words that k_radix_finish reports to
   int turn              = 0;
   bool hooked           = false;
   // under the mutex
@@ -931,21 +932,74 @@ struct RadixRun {
   }
 };
 
+// Places of the keys in runs of kRadixRun keys or more that share the digits
+// from bit `low` on, in order; the keys are ordered by those.
+template <class T>
+struct RadixLongRunsF {
+  using R = RadixKey<T>;
+  using U = typename R::U;
+  const U* keys;
+  int64_t n;
+  int low;
+  uint32_t* places;
+  KOKKOS_INLINE_FUNCTION U high(int64_t i) const { return R::canon(R::encode(keys[i])) >> low; }
+  KOKKOS_INLINE_FUNCTION bool in_long_run(const int64_t i) const {
+    const U mine = high(i);
+    if ((i == 0 || high(i - 1) != mine) && (i + 1 >= n || high(i + 1) != mine)) return false;
+    int64_t below = i >= kRadixRun ? i - kRadixRun : -1, first = i;  // the run's first key is above `below`
+    while (first - below > 1) {
+      const int64_t mid = below + (first - below) / 2;
+      if (high(mid) == mine) first = mid;
+      else below = mid;
+    }
+    return first + kRadixRun - 1 < n && high(first + kRadixRun - 1) == mine;
+  }
+  KOKKOS_INLINE_FUNCTION void operator()(const int64_t i, uint32_t& upd, const bool final) const {
+    if (!in_long_run(i)) return;
+    if (final) places[upd] = uint32_t(i);
+    ++upd;
+  }
+};
+// to[j] = from[places[j]], or back.
+template <class U, class PT, bool Back>
+struct RadixPlacesF {
+  const uint32_t* places;
+  const U* from;
+  U* to;
+  const PT* from_p;
+  PT* to_p;
+  KOKKOS_INLINE_FUNCTION void operator()(const int64_t j) const {
+    const int64_t a = Back ? int64_t(places[j]) : j, b = Back ? j : int64_t(places[j]);
+    to[a]           = from[b];
+    if constexpr (!std::is_same<PT, NoPayload>::value) to_p[a] = from_p[b];
+  }
+};
+
+// Whole tiles per segment and segments of n keys, as many as stay resident.
+template <class Shape>
+int radix_segments(int64_t n, int cus, int64_t& segment) {
+  constexpr int tile   = Shape::lanes * Shape::items;
+  const int64_t ntiles = (n + tile - 1) / tile;
+  const int64_t tpb    = (ntiles + int64_t(cus) * Shape::blocks - 1) / (int64_t(cus) * Shape::blocks);
+  segment              = tpb * tile;
+  return int((ntiles + tpb - 1) / tpb);
+}
+
+template <class T, class PT, class Shape>
+bool radix_sort_long_runs(const MI355X& exec, RadixWorkspace& ws, const RadixRun<T, PT>& r, int low, int cus);
+
 // The passes of a sort that one block cannot hold.
 template <class T, class PT, bool Iota, class Shape>
 void radix_sort_passes(const MI355X& exec, typename RadixKey<T>::U* k0, int64_t n, PT* payload) {
   using U              = typename RadixKey<T>::U;
   constexpr bool pairs = !std::is_same<PT, NoPayload>::value;
-  constexpr int tile   = Shape::lanes * Shape::items;
-  // segments of whole tiles, as many as stay resident
   const int cus            = MI355X::impl_cu_count() > 0 ? MI355X::impl_cu_count() : 256;
-  const int64_t ntiles     = (n + tile - 1) / tile;
-  const int64_t tpb        = (ntiles + int64_t(cus) * Shape::blocks - 1) / (int64_t(cus) * Shape::blocks);
-  int64_t segment          = tpb * tile;
-  int segments             = int((ntiles + tpb - 1) / tpb);
+  int64_t segment          = 0;
+  const int segments       = radix_segments<Shape>(n, cus, segment);
   const size_t key_bytes   = radix_round(size_t(n) * sizeof(U));
   const size_t pay_bytes   = pairs ? radix_round(size_t(n) * sizeof(PT)) : 0;
-  const size_t need        = key_bytes + pay_bytes + radix_round(size_t(segments) * 256 * sizeof(uint32_t));
+  // counts for any number of keys: runs of some are sorted apart
+  const size_t need        = key_bytes + pay_bytes + size_t(cus) * Shape::blocks * 256 * sizeof(uint32_t);
   RadixWorkspace& ws       = radix_workspace();
   std::lock_guard<std::mutex> lock(ws.mtx);
   ws.hook();
@@ -992,6 +1046,7 @@ void radix_sort_passes(const MI355X& exec, typename RadixKey<T>::U* k0, int64_t 
     } else if (*static_cast<volatile uint32_t*>(status) == 1) {
       // the payload holds the permutation so far, also with Iota
       r.turn = ws.turn;
+      if (radix_sort_long_runs<T, PT, Shape>(exec, ws, r, int(status[1]), cus)) return;
       ws.turn ^= 1;
       r.template fold<false>();
       r.sample(false);
@@ -1041,6 +1096,49 @@ void radix_sort_few(const MI355X& exec, typename RadixKey<T>::U* k0, int n, PT* 
   else
     runs(reinterpret_cast<const void*>(&k_radix_small<T, PT, Iota, 4, false>),
          reinterpret_cast<const void*>(&k_radix_merge<T, PT, 4 * R>), 4 * R);
+}
+
+// The last step of a trimmed sort (`r`) with long runs out of order: their keys
+// are sorted by all digits apart from the others and go back to the places that
+// the runs had, which keeps the runs in order.  False, with nothing changed,
+// where they are more than a fifth of all keys.  The second buffers hold the
+// places, the runs' keys and payload and those sorts' second buffers.  3 M
+// (int64, 8-byte) pairs with one such run of 300 take 323 us, where sorting all
+// of them over by all digits made it 543, and 231 without the run; 2^25 int64
+// keys 1.52 ms, 2.93 and 1.22.
+template <class T, class PT, class Shape>
+bool radix_sort_long_runs(const MI355X& exec, RadixWorkspace& ws, const RadixRun<T, PT>& r, int low, int cus) {
+  using U              = typename RadixKey<T>::U;
+  constexpr bool pairs = !std::is_same<PT, NoPayload>::value;
+  using Range          = RangePolicy<MI355X, IndexType<int64_t>>;
+  uint32_t* places     = reinterpret_cast<uint32_t*>(r.k1);  // n of them at most: half of the keys' second buffer
+  uint32_t total       = 0;
+  parallel_scan("Kokkos::sort::long_runs", Range(exec, 0, r.n), RadixLongRunsF<T>{r.k0, r.n, low, places}, total);
+  const int64_t m = int64_t(total);
+  if (m > r.n / 5) return false;
+  RadixRun<T, PT> own = r;
+  own.n               = m;
+  own.segments        = radix_segments<Shape>(m, cus, own.segment);
+  own.k0              = reinterpret_cast<U*>(reinterpret_cast<char*>(r.k1) + radix_round(size_t(r.n) * sizeof(uint32_t)));
+  own.k1              = own.k0 + m;
+  if constexpr (pairs) {
+    own.p0 = r.p1;
+    own.p1 = r.p1 + m;
+  }
+  parallel_for("Kokkos::sort::take_long_runs", Range(exec, 0, m),
+               RadixPlacesF<U, PT, false>{places, r.k0, own.k0, r.p0, own.p0});
+  if (m <= kRadixSmallLanes * kRadixSmallItems<U>) {
+    radix_sort_few<T, PT, false>(exec, own.k0, int(m), own.p0, nullptr);
+  } else {
+    ws.turn ^= 1;  // r.turn is taken
+    own.template fold<false>();
+    own.sample(false);
+    own.template passes<false, Shape>(0, 8);
+  }
+  parallel_for("Kokkos::sort::place_long_runs", Range(exec, 0, m),
+               RadixPlacesF<U, PT, true>{places, own.k0, r.k0, own.p0, r.p0});
+  exec.fence("Kokkos::sort: long runs");
+  return true;
 }
 
 // A space for a merged sort, held until its owner is done with it.

@@ -239,6 +239,41 @@ def test_sort_of_8_byte_keys_by_their_highest_digits(paths, oracle, n, code, vby
     assert np.array_equal(Dk.download(TYPES[code], n).view(np.uint64), x[order].view(np.uint64))
 
 
+# Runs of keys that share their five highest digits and are too long to be put
+# right in place, where a sample of every (n // 4096)-th key does not show them:
+# fewer than a block sorts (2048), just more, as many as are sorted apart (a fifth
+# of all) and more.
+@pytest.mark.parametrize("n,m", [(100003, 64), (100003, 2048), (100003, 2049), (100003, 20000), (100003, 20001),
+                                 (100003, 90000), ((1 << 21) + 5, 400000), ((1 << 21) + 5, 1900000)])
+@pytest.mark.parametrize("code,vbytes,run_length", [(1, 0, 64), (5, 8, 100), (3, 4, 3000)])
+def test_sort_of_8_byte_keys_with_hidden_runs(paths, oracle, n, m, code, vbytes, run_length):
+    P = paths
+    r = oracle.fill_uniform_i64(n, 700 + code, -(1 << 62), 1 << 62)
+    low = oracle.fill_uniform_i64(m, 800 + code, 0, (1 << 20) - 1)
+    step = n // 4096
+    hidden = np.flatnonzero(np.arange(n) % step != 0)
+    at = hidden[np.argsort(oracle.fill_uniform_i64(len(hidden), 900 + code, 0, 1 << 62), kind="stable")[:m]]
+    runs = max(1, m // run_length)  # the last of them longer by the remainder
+    at.sort()
+    r[at] = (r[np.minimum(np.arange(m) % runs, n - 1)] & ~np.int64((1 << 20) - 1)) | low
+    x = r.view(np.float64) if code == 3 else r.astype(TYPES[code])
+    if code == 3:
+        x = np.where(np.isnan(x), 1.5, x)
+    order = np.argsort(x, kind="stable")
+    Dk = K.DeviceBuffer.from_array(x)
+    for again in range(2):  # the second call finds the sort's state as the first left it
+        if vbytes:
+            vdt = np.uint32 if vbytes == 4 else np.uint64
+            Dk.upload(x)
+            Dv = K.DeviceBuffer.from_array(np.arange(n, dtype=vdt))
+            run(P, P.kkmx_sort_by_key(Dk.ptr, Dv.ptr, n, code, vbytes, 0))
+            assert np.array_equal(Dv.download(vdt, n), order.astype(vdt))
+        else:
+            Dk.upload(x)
+            run(P, P.kkmx_sort(Dk.ptr, n, code))
+        assert np.array_equal(Dk.download(TYPES[code], n).view(np.uint64), x[order].view(np.uint64))
+
+
 @pytest.mark.parametrize("code", [0, 3])
 def test_sort_by_key_with_comparator(paths, oracle, code):
     """The comparator overload (Kokkos_SortByKeyPublicAPI.hpp:67-108) with a
