@@ -2862,6 +2862,54 @@ KKMX_TEST(binsort_quantised_forms) {
   }
 }
 
+// Within-bin order, counts and offsets for the other key types that are ordered
+// by codes, at a size of the few-keys sort and of the passes: keys over all of a
+// type's range or a part of it, integers wider than a double, repeated keys.
+template <class T>
+void check_binsort_of_type(T lo, T hi, T step) {
+  using DV = Kokkos::View<T*, Exec>;
+  for (int n : {5003, 100003}) {
+    DV keys("keys", n);
+    auto m = Kokkos::create_mirror_view(keys);
+    const double cells = (double(hi) - double(lo)) / double(step);
+    for (int i = 0; i < n; ++i) {
+      const double u = double((int64_t(i) * 2654435761ll + 12345) % 1000003) / 1000003.0;
+      m(i)           = i % 997 == 0 ? hi : i % 991 == 0 ? lo : T(lo + T(std::floor(u * cells)) * step + T(i % 3));
+      if (m(i) > hi) m(i) = hi;
+    }
+    Kokkos::deep_copy(keys, m);
+    for (int nbins : {1, 1000, 70000}) {
+      Kokkos::BinOp1D<DV> op(nbins, lo, hi);
+      Kokkos::BinSort<DV, Kokkos::BinOp1D<DV>> sorter(keys, 0, n, op, true);
+      sorter.create_permute_vector(Exec());
+      auto perm = Kokkos::create_mirror_view_and_copy(Kokkos::HostSpace(), sorter.get_permute_vector());
+      auto cnt  = Kokkos::create_mirror_view_and_copy(Kokkos::HostSpace(), sorter.get_bin_count());
+      auto off  = Kokkos::create_mirror_view_and_copy(Kokkos::HostSpace(), sorter.get_bin_offsets());
+      std::vector<int> order(n), want(op.max_bins(), 0);
+      for (int i = 0; i < n; ++i) {
+        order[i] = i;
+        ++want[op.bin(m, i)];
+      }
+      std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return m(x) < m(y); });
+      for (int i = 0; i < n; ++i) CHECK_EQ(perm(i), order[i]);
+      int total = 0;
+      for (int k = 0; k < op.max_bins(); ++k) {
+        CHECK_EQ(off(k), total);
+        CHECK_EQ(cnt(k), want[k]);
+        total += want[k];
+      }
+    }
+  }
+}
+KKMX_TEST(binsort_key_types) {
+  check_binsort_of_type<float>(-3.0f, 1000.0f, 0.125f);
+  check_binsort_of_type<int>(-500, 499, 1);
+  check_binsort_of_type<int>(-2000000000, 2000000000, 7);
+  check_binsort_of_type<unsigned>(0u, 4294967295u, 65536u);
+  check_binsort_of_type<int64_t>(-(int64_t(1) << 61), int64_t(1) << 61, int64_t(1) << 40);
+  check_binsort_of_type<uint64_t>(uint64_t(1) << 53, (uint64_t(1) << 53) + 5000, 1);  // some keys are one double
+}
+
 // A sorter made beforehand orders by bins (no order within them) in a captured
 // call, the first on this sorter; replays see the keys of their time.
 KKMX_TEST(binsort_captured) {
