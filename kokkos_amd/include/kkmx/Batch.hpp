@@ -661,10 +661,12 @@ class BatchDispatch {
   }
   // The default tile shape: 16384-element tiles, unless all tiles of half that
   // size run at once, two a CU.  Such a batch takes as long as its longest tile
-  // with its claim and look-back: 64 ops of 2^8..2^16 elements (118 tiles) 22.1
-  // us with the large tiles and 16.7 with the small ones, 32 of 2^4..2^20 (229)
-  // 24.8 and 18.5, 512 of 2^4..2^12 (512) 27.1 and 25.5.  With more tiles the
-  // large ones' fewer claims pay: 621 tiles 31.0 and 32.8, 730 32.6 and 36.9.
+  // with its claim and look-back: forty captured runs in a row, 64 ops of
+  // 2^8..2^16 elements (118 tiles) take 22.1 us each with the large tiles and 16.8
+  // with the small ones, 32 of 2^4..2^20 (229) 24.8 and 18.5, 512 of 2^4..2^12
+  // (512) 27.1 and 25.5; launched and not captured, the 64 ops 17.2 and 11.7.  With
+  // more tiles the large ones' fewer claims pay: 621 tiles 31.0 and 32.8, 730 32.6
+  // and 36.9.
   int default_shape() const {
     const int64_t tile = Impl::kBatchShape[Impl::kBatchSmallShape].tile();
     int64_t tiles      = 0;

@@ -107,9 +107,11 @@ struct ElementCopy {
 // coalesced; the tile sits in LDS with an odd row pitch so neither pass has
 // bank conflicts.  Consecutive workgroups take consecutive tiles of the last
 // index, and the destination is written with nontemporal stores (a copy's
-// output is not read back by the copy).  512^3 doubles: 0.421 ms with 64 x 32
-// tiles, 0.435 with 64 x 64 (0.449 with 64-bit index arithmetic), 0.51-0.64
-// with 128 in either direction, 0.65 with the middle index fastest.
+// output is not read back by the copy).  512^3 doubles: 0.436 ms a call
+// (kernel trace 0.437 on average, 0.429 at best), 0.447 with 64 x 64 tiles and
+// 64-bit index arithmetic.  Variants back to back in one loop: 0.421 with 64 x 32
+// tiles, 0.435 with 64 x 64 (0.449 with 64-bit arithmetic), 0.51-0.64 with 128 in
+// either direction, 0.65 with the middle index fastest.
 //   LayoutLeft  offset of (i, mid, k) = i + e0 * (midL + M * k)
 //   LayoutRight offset of (i, mid, k) = (i * M + midR) * e_last + k
 // midL / midR: the middle indices flattened left-first / right-first, M

@@ -12,7 +12,8 @@
 // itself.  8-byte keys are sorted by their five highest digits that vary where a
 // sample shows those to tell them apart (k_radix_sample), and neighbours that
 // share them are put right on the way back (k_radix_finish).  A sort is a fixed
-// sequence of launches and one wait, two for 8-byte keys that are not trimmed.
+// sequence of launches and one wait, two for 8-byte keys that are not trimmed,
+// and more where many keys share those digits after all (radix_sort_long_runs).
 // Few keys are sorted in LDS: those of one block by a single launch
 // (k_radix_small), those of several blocks' runs by one more that places every
 // key among the other runs (k_radix_merge).
