@@ -198,6 +198,17 @@ def test_sort_in_runs(paths, oracle, n, code, vbytes, form):
     assert np.array_equal(Dk.download(TYPES[code], n).view(bits), x[order].view(bits))
 
 
+def put_hidden_runs(oracle, r, m, runs, seed):
+    """m of the int64 keys r become members of `runs` runs of about the same
+    length that share all but their lowest 20 bits, at places that a sample of
+    every (n // 4096)-th key does not touch."""
+    n = len(r)
+    hidden = np.flatnonzero(np.arange(n) % max(1, n // 4096) != 0)
+    at = np.sort(hidden[np.argsort(oracle.fill_uniform_i64(len(hidden), seed, 0, 1 << 62), kind="stable")[:m]])
+    base = oracle.fill_uniform_i64(runs, seed + 1, -(1 << 62), 1 << 62) & ~np.int64((1 << 20) - 1)
+    r[at] = base[np.arange(m) % runs] | oracle.fill_uniform_i64(m, seed + 2, 0, (1 << 20) - 1)
+
+
 @pytest.mark.parametrize("form", ["spread", "runs", "crowd", "one_long_run", "equal", "six_digits"])
 @pytest.mark.parametrize("n", [8193, 100003, (1 << 21) + 5])
 @pytest.mark.parametrize("code,vbytes", [(1, 0), (3, 0), (5, 8), (3, 4)])
@@ -206,20 +217,19 @@ def test_sort_of_8_byte_keys_by_their_highest_digits(paths, oracle, n, code, vby
     those tell them apart: spread keys (no digits to spare), runs of up to 40
     keys that share them out of order, keys all crowded into few runs (seen in
     the sample: all digits), one run of 300 among spread keys (not seen, found
-    at the end: sorted over), many equal keys, and keys of six digits."""
+    at the end: sorted apart), many equal keys, and keys of six digits.  The
+    smallest size takes the sort of few keys."""
     P = paths
     r = oracle.fill_uniform_i64(n, 500 + code, -(1 << 62), 1 << 62)
     low = oracle.fill_uniform_i64(n, 600 + code, 0, (1 << 20) - 1)
     if form == "runs":
-        k = np.arange(n) // 40 % 997
-        r = np.where(k < 20, (r[k] & ~np.int64((1 << 20) - 1)) | low, r)[np.argsort(low, kind="stable")]
+        put_hidden_runs(oracle, r, n // 10, -(-(n // 10) // 40), 1000 + code)
     elif form == "crowd":
         r = (r[np.arange(n) % 7] & ~np.int64((1 << 20) - 1)) | low
         r[0] = -(1 << 62)
         r[1] = (1 << 62) - 1
     elif form == "one_long_run":
-        at = np.argsort(low, kind="stable")[:300]
-        r[at] = (r[0] & ~np.int64((1 << 20) - 1)) | low[at]
+        put_hidden_runs(oracle, r, 300, 1, 1000 + code)
     elif form == "equal":
         r = r[np.arange(n) % 1009]
     elif form == "six_digits":
@@ -239,23 +249,19 @@ def test_sort_of_8_byte_keys_by_their_highest_digits(paths, oracle, n, code, vby
     assert np.array_equal(Dk.download(TYPES[code], n).view(np.uint64), x[order].view(np.uint64))
 
 
-# Runs of keys that share their five highest digits and are too long to be put
-# right in place, where a sample of every (n // 4096)-th key does not show them:
-# fewer than a block sorts (2048), just more, as many as are sorted apart (a fifth
-# of all) and more.
+# Runs of keys that share their five highest digits, out of sight of the sample
+# that decides to sort by those: short ones, put in order in place, up to the
+# longest of 63, and longer ones; of the latter, fewer keys than a block sorts
+# (2048), just more, as many as are sorted apart (a fifth of all) and more.
 @pytest.mark.parametrize("n,m", [(100003, 64), (100003, 2048), (100003, 2049), (100003, 20000), (100003, 20001),
                                  (100003, 90000), ((1 << 21) + 5, 400000), ((1 << 21) + 5, 1900000)])
-@pytest.mark.parametrize("code,vbytes,run_length", [(1, 0, 64), (5, 8, 100), (3, 4, 3000)])
+@pytest.mark.parametrize("code,vbytes,run_length", [(1, 0, 64), (5, 8, 100), (3, 4, 3000), (1, 8, 63), (5, 0, 40),
+                                                    (3, 8, 3), (1, 4, 2)])
 def test_sort_of_8_byte_keys_with_hidden_runs(paths, oracle, n, m, code, vbytes, run_length):
     P = paths
     r = oracle.fill_uniform_i64(n, 700 + code, -(1 << 62), 1 << 62)
-    low = oracle.fill_uniform_i64(m, 800 + code, 0, (1 << 20) - 1)
-    step = n // 4096
-    hidden = np.flatnonzero(np.arange(n) % step != 0)
-    at = hidden[np.argsort(oracle.fill_uniform_i64(len(hidden), 900 + code, 0, 1 << 62), kind="stable")[:m]]
-    runs = max(1, m // run_length)  # the last of them longer by the remainder
-    at.sort()
-    r[at] = (r[np.minimum(np.arange(m) % runs, n - 1)] & ~np.int64((1 << 20) - 1)) | low
+    # at least run_length keys each, or, of the short ones, at most
+    put_hidden_runs(oracle, r, m, max(1, m // run_length) if run_length >= 64 else -(-m // run_length), 800 + code)
     x = r.view(np.float64) if code == 3 else r.astype(TYPES[code])
     if code == 3:
         x = np.where(np.isnan(x), 1.5, x)
