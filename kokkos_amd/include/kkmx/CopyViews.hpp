@@ -101,9 +101,9 @@ struct ElementCopy {
 // ViewCopy between LayoutLeft and LayoutRight (both contiguous, rank >= 2)
 // as an LDS-tiled transpose on gfx950: each 512-lane workgroup moves a tile of
 // (first index, last index) for one multi-index of the middle dimensions, 64
-// long in the source's contiguous dimension and in the destination's 64, for
-// 8-byte words 32, which leaves room for twice the workgroups.  It reads along
-// the source's contiguous dimension and writes along the destination's, both
+// long in the source's contiguous dimension and 64 or, for some shapes of 8-byte
+// words, 32 (transpose_narrow) in the destination's.  It reads along the
+// source's contiguous dimension and writes along the destination's, both
 // coalesced; the tile sits in LDS with an odd row pitch so neither pass has
 // bank conflicts.  Consecutive workgroups take consecutive tiles of the last
 // index, and the destination is written with nontemporal stores (a copy's
@@ -125,13 +125,10 @@ struct TransposeShape {
 };
 // Tiles of one launch: HIP takes fewer than 2^32 lanes along a grid dimension.
 constexpr int64_t kTransposeTiles = int64_t(1) << 22;
-// Tile extent along the destination's contiguous dimension.
-template <class W>
-constexpr int transpose_narrow = sizeof(W) == 8 ? 32 : 64;
-template <class W, bool SrcLeft>
+// N: tile extent along the destination's contiguous dimension.
+template <class W, bool SrcLeft, int N>
 __global__ __launch_bounds__(512) void k_layout_transpose(W* __restrict__ dst, const W* __restrict__ src,
                                                           const TransposeShape sh) {
-  constexpr int N = transpose_narrow<W>;
   __shared__ W tile[N][65];
   const uint32_t b  = sh.first + blockIdx.x;
   const uint32_t tk = b % sh.tileslast;
@@ -180,6 +177,25 @@ using transpose_word_t =
     std::conditional_t<sizeof(T) == 8, uint64_t,
                        std::conditional_t<sizeof(T) == 4, uint32_t, std::conditional_t<sizeof(T) == 2, uint16_t, uint8_t>>>;
 
+// Whether 8-byte words take 64 x 32 tiles, which leave room for twice the
+// workgroups on a CU but write rows of half the length.  `across` is the source's
+// contiguous extent, `along` the destination's.  Times against 64 x 64 tiles, 1 to
+// 32 M words in all:
+//  * Half as long tiles are not twice as many where the last of them is at most
+//    half full: 0.81-0.91 up to 32 along (17 to 31 of them 0.9-1.25 where across
+//    is 48 or more), 0.6-0.97 at 72 to 96, 0.74-1.03 at 200 to 224, 0.9-1.03 at 136
+//    to 160 and from 264 on; but 1.04-1.2 there for narrow sources, and 1.0-1.3 for
+//    rows that start within 64 bytes (65, 130).
+//  * Otherwise the rows of a tile count: 1.1-1.7 at 33 to 48, 1.0-1.2 at 100, 112
+//    and 300; even at 64, 128 and 256 (1.04-1.2 for narrow sources) and from 512 on
+//    0.97 at 512^3.
+inline bool transpose_narrow(int64_t across, int64_t along) {
+  if (along % 8 != 0) return along <= 32 && across < 48;
+  const int64_t last = along % 64;
+  if (last == 0) return along >= 512 && across >= 64;
+  return last <= 32 && (along < 128 || across >= 48);
+}
+
 // Launches the transpose when it applies (Left <-> Right, contiguous, rank
 // 2-6, trivially copyable elements of 1-8 bytes, first and last extents of
 // at least 16); returns false otherwise.
@@ -208,18 +224,19 @@ bool layout_transpose(const MI355X& exec, const DV& dst, const SV& src) {
       sh.mid[d] = uint32_t(dst.extent(d + 1));
     }
     if (sh.M == 0) return true;
-    using W                 = transpose_word_t<T>;
-    constexpr int64_t N     = transpose_narrow<W>;
-    const int64_t tiles0    = lr ? (sh.e0 + 63) / 64 : (sh.e0 + N - 1) / N;
+    using W              = transpose_word_t<T>;
+    const int N          = sizeof(W) == 8 && transpose_narrow(lr ? sh.e0 : sh.elast, lr ? sh.elast : sh.e0) ? 32 : 64;
+    const int64_t tiles0 = lr ? (sh.e0 + 63) / 64 : (sh.e0 + N - 1) / N;
     const int64_t tileslast = lr ? (sh.elast + N - 1) / N : (sh.elast + 63) / 64;
     if (tiles0 > 0x7fffffff || tileslast > 0x7fffffff / tiles0 || sh.M > 0x7fffffff / (tiles0 * tileslast)) return false;
     const int64_t blocks = tiles0 * tileslast * sh.M;
     sh.tiles0            = uint32_t(tiles0);
     sh.tileslast         = uint32_t(tileslast);
-    W* d     = reinterpret_cast<W*>(dst.data());
-    const W* s_ = reinterpret_cast<const W*>(src.data());
-    const void* k = lr ? reinterpret_cast<const void*>(&k_layout_transpose<W, true>)
-                       : reinterpret_cast<const void*>(&k_layout_transpose<W, false>);
+    W* d                 = reinterpret_cast<W*>(dst.data());
+    const W* s_          = reinterpret_cast<const W*>(src.data());
+    const void* k        = reinterpret_cast<const void*>(&k_layout_transpose<W, lr, 64>);
+    if constexpr (sizeof(W) == 8)
+      if (N == 32) k = reinterpret_cast<const void*>(&k_layout_transpose<W, lr, 32>);
     for (int64_t done = 0; done < blocks; done += kTransposeTiles) {
       sh.first            = uint32_t(done);
       const int64_t tiles = blocks - done < kTransposeTiles ? blocks - done : kTransposeTiles;

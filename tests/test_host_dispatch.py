@@ -75,6 +75,25 @@ def test_transpose_of_many_tiles(runtime, m, to_right):
     """)
 
 
+@pytest.mark.parametrize("across,along,narrow", [
+    (16, 16, 1), (512, 24, 1), (47, 31, 1), (48, 31, 0), (512, 32, 1), (16, 33, 0), (512, 64, 0), (100, 65, 0),
+    (16, 72, 1), (512, 96, 1), (512, 104, 0), (512, 128, 0), (47, 136, 0), (48, 136, 1), (512, 224, 1), (512, 256, 0),
+    (512, 300, 0), (63, 512, 0), (64, 512, 1), (512, 512, 1), (512, 1000, 0)])
+def test_transpose_tiles(runtime, across, along, narrow):
+    """Which shapes of doubles take tiles of 64 x 32, in either direction."""
+    run(runtime, f"""
+        start()
+        for right in (1, 0):
+            e0, e2 = ({across}, {along}) if right else ({along}, {across})
+            H.host_clear()
+            assert P.kkmx_deep_copy_f64(at(1 << 46), at(1 << 45), i64(e0), i64(3), i64(e2), right, 1 - right) == 0
+            (kernel, grid, block), = launches()
+            n = 32 if {narrow} else 64
+            assert f'k_layout_transposeImLb{{right}}ELi{{n}}E' in kernel, kernel
+            assert grid == 3 * -(-{across} // 64) * -(-{along} // n)
+    """)
+
+
 @pytest.mark.parametrize("nbins", [65536, 100000])
 def test_histogram_rows_stay(runtime, nbins):
     """A call with few keys makes the table that one with many keys uses: a
