@@ -190,7 +190,9 @@ int kkmx_spmv_csr(const int64_t* rowptr_dev, const int32_t* col_dev, const doubl
  *   2^20 values (2^18 into at most 4096 bins) and up to 2^21 bins, values of
  *   one bin are first added up in LDS.  That form keeps a workspace of up to
  *   194 MiB between calls, released by kkmx_finalize; under stream capture, or
- *   where there is no memory for it, the atomics run directly.  Every form only adds to bins. */
+ *   where there is no memory for it, the atomics run directly.  Indices that
+ *   run through the bins in order are faster by kkmx_scatter_view_f64's
+ *   atomics.  Every form only adds to bins. */
 int kkmx_xorshift64_stream(uint64_t* out_dev, int64_t n, uint64_t seed);
 int kkmx_gups(int64_t* table_dev, int64_t table_size, const uint64_t* stream_dev, int64_t nupdates);
 int kkmx_zipf_keys(int32_t* keys_dev, int64_t n, double s, int32_t nbins, uint64_t seed);

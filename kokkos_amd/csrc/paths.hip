@@ -819,10 +819,17 @@ int32_t* hist_rows_space(size_t elems) {
   return rows->data();
 }
 // Teams, and rows of the table, for n keys: one per CU, fewer where a team would
-// have less than 16384 keys.  A team pays for its bins whatever its keys, in
-// LDS and with a row written and read again: 65536 bins cost 256 rows 40 us.
-int hist_teams(int64_t n, int cus) {
-  const int64_t want = (n + 16383) / 16384;
+// have less than nbins / share keys, or 1024.  A team pays for its bins whatever
+// its keys, in LDS and with a row written and read again: 256 rows of 65536 bins
+// cost 40 us, 0.6 ps a bin and row.  Its keys may all meet in one counter, 0.7 ns
+// each in LDS (HistPacked) and 13 in the team's row (HistRows' bins above the LDS
+// range); the shares, 5 and 50, keep that below what the rows saved.  2^18 keys
+// into 65536 bins take 34 us, 43 with a team per CU, and 43 and 47 where they are
+// all one key.  2^14 keys a team for any number of bins took 262 us for 2^18 equal
+// keys into 100000 bins (72 with a team per CU), and 32 into 1000 (21).
+int hist_teams(int64_t n, int cus, int32_t nbins, int share) {
+  const int64_t keys = nbins / share < 1024 ? 1024 : nbins / share;
+  const int64_t want = (n + keys - 1) / keys;
   return int(want < 1 ? 1 : want < cus ? want : cus);
 }
 struct ScatterAdd {
@@ -1472,7 +1479,7 @@ int kkmx_histogram(const int32_t* keys, int64_t n, int32_t* bins, int32_t nbins,
       const int cus_ = Kokkos::MI355X::impl_cu_count();
       const size_t budget = Kokkos::TeamPolicy<Kokkos::MI355X>(cus_, 1024).scratch_size_max(0);
       if (HistPacked::scratch_words(nbins) * 4 <= budget && n / cus_ < HistPacked::kMaxKeysPerTeam - 4096) {
-        const int teams = hist_teams(n, cus_);
+        const int teams = hist_teams(n, cus_, nbins, 5);
         int32_t* rows   = hist_rows_space(size_t(cus_) * nbins);
         using Rows = Kokkos::View<int32_t**, Kokkos::LayoutRight, Kokkos::MI355XSpace, Kokkos::MemoryTraits<Kokkos::Unmanaged>>;
         auto pol = Kokkos::TeamPolicy<Kokkos::MI355X>(teams, 1024)
@@ -1492,7 +1499,7 @@ int kkmx_histogram(const int32_t* keys, int64_t n, int32_t* bins, int32_t nbins,
       const size_t budget = Kokkos::TeamPolicy<Kokkos::MI355X>(cus, 1024).scratch_size_max(0);
       const int64_t fit   = int64_t(budget / 4) - int64_t(HistRows::kHotCopies) * (hot + 1);
       if (lb3 > fit) lb3 = int32_t(fit);
-      const int teams = hist_teams(n, cus);
+      const int teams = hist_teams(n, cus, nbins, 50);
       int32_t* rows   = hist_rows_space(size_t(cus) * nbins);
       using Rows = Kokkos::View<int32_t**, Kokkos::LayoutRight, Kokkos::MI355XSpace, Kokkos::MemoryTraits<Kokkos::Unmanaged>>;
       auto pol = Kokkos::TeamPolicy<Kokkos::MI355X>(teams, 1024)

@@ -107,6 +107,20 @@ def test_histogram_rows_stay(runtime, nbins):
     """)
 
 
+@pytest.mark.parametrize("n,nbins,teams", [
+    (1, 65536, 1), (13107, 65536, 1), (13108, 65536, 2), (1 << 18, 65536, 21), (1 << 22, 65536, 256),
+    (1024, 1000, 1), (1025, 1000, 2), (100000, 1000, 98), (1 << 18, 300, 256), (2000, 100000, 1), (2001, 100000, 2),
+    (100000, 100000, 50), (1 << 20, 100000, 256)])
+def test_histogram_teams(runtime, n, nbins, teams):
+    """Teams by what a row of bins costs against keys that all meet in one
+    counter, in LDS (up to about 70000 bins) and in the team's row."""
+    run(runtime, f"""
+        start()
+        assert P.kkmx_histogram(at(1 << 45), i64({n}), at(1 << 46), {nbins}, 3, 0) == 0
+        assert launches()[0][1] == {teams} and len(launches()) == 2, launches()
+    """)
+
+
 @pytest.mark.parametrize("cus", [8, 24, 25, 32, 256])
 def test_scatter_moves_by_summed_counts(runtime, cus):
     """However many segments the CUs give the move, its last kernel is told that
