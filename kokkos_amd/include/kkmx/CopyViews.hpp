@@ -182,15 +182,16 @@ using transpose_word_t =
 // contiguous extent, `along` the destination's.  Times against 64 x 64 tiles, 1 to
 // 32 M words in all:
 //  * Half as long tiles are not twice as many where the last of them is at most
-//    half full: 0.81-0.91 up to 32 along (17 to 31 of them 0.9-1.25 where across
-//    is 48 or more), 0.6-0.97 at 72 to 96, 0.74-1.03 at 200 to 224, 0.9-1.03 at 136
-//    to 160 and from 264 on; but 1.04-1.2 there for narrow sources, and 1.0-1.3 for
-//    rows that start within 64 bytes (65, 130).
+//    half full: 0.81-1.0 up to 32 along (1.0-1.07, and 1.25 at 17 by 48, for large
+//    copies with rows that start within 64 bytes), 0.6-0.97 at 72 to 96, 0.74-1.03
+//    at 200 to 224, 0.9-1.03 at 136 to 160 and from 264 on; but 1.04-1.2 there for
+//    narrow sources, and 1.0-1.3 for rows that start within 64 bytes (65, 130).
 //  * Otherwise the rows of a tile count: 1.1-1.7 at 33 to 48, 1.0-1.2 at 100, 112
 //    and 300; even at 64, 128 and 256 (1.04-1.2 for narrow sources) and from 512 on
 //    0.97 at 512^3.
 inline bool transpose_narrow(int64_t across, int64_t along) {
-  if (along % 8 != 0) return along <= 32 && across < 48;
+  if (along <= 32) return true;
+  if (along % 8 != 0) return false;
   const int64_t last = along % 64;
   if (last == 0) return along >= 512 && across >= 64;
   return last <= 32 && (along < 128 || across >= 48);

@@ -76,7 +76,7 @@ def test_transpose_of_many_tiles(runtime, m, to_right):
 
 
 @pytest.mark.parametrize("across,along,narrow", [
-    (16, 16, 1), (512, 24, 1), (47, 31, 1), (48, 31, 0), (512, 32, 1), (16, 33, 0), (512, 64, 0), (100, 65, 0),
+    (16, 16, 1), (512, 24, 1), (128, 22, 1), (48, 31, 1), (512, 32, 1), (16, 33, 0), (512, 64, 0), (100, 65, 0),
     (16, 72, 1), (512, 96, 1), (512, 104, 0), (512, 128, 0), (47, 136, 0), (48, 136, 1), (512, 224, 1), (512, 256, 0),
     (512, 300, 0), (63, 512, 0), (64, 512, 1), (512, 512, 1), (512, 1000, 0)])
 def test_transpose_tiles(runtime, across, along, narrow):
