@@ -179,8 +179,9 @@ using transpose_word_t =
 
 // Whether 8-byte words take 64 x 32 tiles, which leave room for twice the
 // workgroups on a CU but write rows of half the length.  `across` is the source's
-// contiguous extent, `along` the destination's.  Times against 64 x 64 tiles, 1 to
-// 32 M words in all:
+// contiguous extent, `along` the destination's, `words` all of the copy.  Below 2^20
+// words the smaller tiles reach more CUs: 0.85-1.05 of the time of 64 x 64 ones, from
+// 2^20 to 2^21 0.9-1.1 with a middle above 1.  Of larger copies, to 32 M words:
 //  * Half as long tiles are not twice as many where the last of them is at most
 //    half full: 0.81-1.0 up to 32 along (1.0-1.07, and 1.25 at 17 by 48, for large
 //    copies with rows that start within 64 bytes), 0.6-0.97 at 72 to 96, 0.74-1.03
@@ -189,8 +190,8 @@ using transpose_word_t =
 //  * Otherwise the rows of a tile count: 1.1-1.7 at 33 to 48, 1.0-1.2 at 100, 112
 //    and 300; even at 64, 128 and 256 (1.04-1.2 for narrow sources) and from 512 on
 //    0.97 at 512^3.
-inline bool transpose_narrow(int64_t across, int64_t along) {
-  if (along <= 32) return true;
+inline bool transpose_narrow(int64_t across, int64_t along, int64_t words) {
+  if (words < (int64_t(1) << 20) || along <= 32) return true;
   if (along % 8 != 0) return false;
   const int64_t last = along % 64;
   if (last == 0) return along >= 512 && across >= 64;
@@ -226,7 +227,8 @@ bool layout_transpose(const MI355X& exec, const DV& dst, const SV& src) {
     }
     if (sh.M == 0) return true;
     using W              = transpose_word_t<T>;
-    const int N          = sizeof(W) == 8 && transpose_narrow(lr ? sh.e0 : sh.elast, lr ? sh.elast : sh.e0) ? 32 : 64;
+    const int64_t across = lr ? sh.e0 : sh.elast, along = lr ? sh.elast : sh.e0;
+    const int N          = sizeof(W) == 8 && transpose_narrow(across, along, int64_t(dst.span())) ? 32 : 64;
     const int64_t tiles0 = lr ? (sh.e0 + 63) / 64 : (sh.e0 + N - 1) / N;
     const int64_t tileslast = lr ? (sh.elast + N - 1) / N : (sh.elast + 63) / 64;
     if (tiles0 > 0x7fffffff || tileslast > 0x7fffffff / tiles0 || sh.M > 0x7fffffff / (tiles0 * tileslast)) return false;

@@ -50,7 +50,8 @@ def test_layout_copy(paths, oracle, shape, dst_layout, src_layout):
 
 
 @pytest.mark.parametrize("shape", [(33, 2, 65), (31, 5, 32), (32, 1, 33), (64, 3, 31), (129, 2, 96), (16, 1, 16),
-                                   (72, 3, 136), (200, 2, 47), (512, 1, 65), (63, 2, 512)])
+                                   (72, 3, 136), (200, 2, 47), (512, 1, 65), (63, 2, 512),
+                                   (65, 250, 65), (127, 100, 130), (33, 500, 65)])
 @pytest.mark.parametrize("dst_layout,src_layout", [(1, 0), (0, 1)])
 def test_layout_copy_tile_edges(paths, oracle, shape, dst_layout, src_layout):
     """Both sides of the transpose's 64 x 64 and 64 x 32 tiles, in either direction."""

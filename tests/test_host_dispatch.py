@@ -75,22 +75,23 @@ def test_transpose_of_many_tiles(runtime, m, to_right):
     """)
 
 
-@pytest.mark.parametrize("across,along,narrow", [
-    (16, 16, 1), (512, 24, 1), (128, 22, 1), (48, 31, 1), (512, 32, 1), (16, 33, 0), (512, 64, 0), (100, 65, 0),
-    (16, 72, 1), (512, 96, 1), (512, 104, 0), (512, 128, 0), (47, 136, 0), (48, 136, 1), (512, 224, 1), (512, 256, 0),
-    (512, 300, 0), (63, 512, 0), (64, 512, 1), (512, 512, 1), (512, 1000, 0)])
-def test_transpose_tiles(runtime, across, along, narrow):
+@pytest.mark.parametrize("across,along,middle,narrow", [
+    (16, 16, 9999, 1), (512, 24, 100, 1), (48, 31, 999, 1), (512, 32, 100, 1), (16, 33, 1985, 1), (16, 33, 1986, 0),
+    (512, 64, 31, 1), (512, 64, 32, 0), (100, 65, 999, 0), (16, 72, 999, 1), (512, 96, 99, 1), (512, 104, 99, 0),
+    (512, 128, 99, 0), (47, 136, 999, 0), (48, 136, 999, 1), (512, 224, 99, 1), (512, 256, 99, 0), (512, 300, 99, 0),
+    (63, 512, 99, 0), (64, 512, 99, 1), (512, 512, 3, 1), (512, 512, 9, 1), (512, 1000, 3, 0)])
+def test_transpose_tiles(runtime, across, along, middle, narrow):
     """Which shapes of doubles take tiles of 64 x 32, in either direction."""
     run(runtime, f"""
         start()
         for right in (1, 0):
             e0, e2 = ({across}, {along}) if right else ({along}, {across})
             H.host_clear()
-            assert P.kkmx_deep_copy_f64(at(1 << 46), at(1 << 45), i64(e0), i64(3), i64(e2), right, 1 - right) == 0
+            assert P.kkmx_deep_copy_f64(at(1 << 46), at(1 << 45), i64(e0), i64({middle}), i64(e2), right, 1 - right) == 0
             (kernel, grid, block), = launches()
             n = 32 if {narrow} else 64
             assert f'k_layout_transposeImLb{{right}}ELi{{n}}E' in kernel, kernel
-            assert grid == 3 * -(-{across} // 64) * -(-{along} // n)
+            assert grid == {middle} * -(-{across} // 64) * -(-{along} // n)
     """)
 
 
